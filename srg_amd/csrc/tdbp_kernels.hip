@@ -241,19 +241,9 @@ __device__ __forceinline__ void cpu_pair(const float2* __restrict__ row,
   }
 }
 
-template <bool CPU>
-__device__ __forceinline__ void fp64_pair(const float2* __restrict__ row,
-                                          const double* x, double sx, double sy,
-                                          double sz, const BurstDev& b, double& ar,
-                                          double& ai) {
-  if constexpr (CPU)
-    cpu_pair(row, x, sx, sy, sz, b, ar, ai);
-  else
-    plain_pair(row, x, sx, sy, sz, b, ar, ai);
-}
-
-template <int TR, bool STACK, bool CPU = false>
-__device__ __forceinline__ void plain_tile(const BurstDev& b, int tile) {
+// The CPU twin's tile: every pair by cpu_pair.
+template <int TR, bool STACK>
+__device__ __forceinline__ void cpu_tile(const BurstDev& b, int tile) {
   PixelCtx p = pixel_of<TR, STACK>(b, tile);
   double x[3] = {0., 0., 0.};
   const bool live = p.aze > p.azs;
@@ -267,7 +257,7 @@ __device__ __forceinline__ void plain_tile(const BurstDev& b, int tile) {
   for (int q = lo; q < hi; ++q) {
     const double sx = sat[3 * q], sy = sat[3 * q + 1], sz = sat[3 * q + 2];
     if ((unsigned)(q - p.azs) < n)
-      fp64_pair<CPU>(base + (size_t)q * b.S, x, sx, sy, sz, b, ar, ai);
+      cpu_pair(base + (size_t)q * b.S, x, sx, sy, sz, b, ar, ai);
   }
   store_out(b, p, (float)ar, (float)ai);
 }
@@ -942,6 +932,457 @@ __device__ __forceinline__ void staged_stage(const BurstDev& b, const PolyPixel&
     }
     __syncthreads();
   }
+}
+
+// ------------------------------------------- FP64 tile on the range excess
+//
+// The FP64 kernel is bound by FP64 VALU issue (and, at full issue, by the
+// clock the card holds under it): plain_pair takes 86 instructions, half of
+// them for the root, the reduction and the sin/cos of a phase that changes
+// smoothly from pulse to pulse.  Here a pixel's range is taken as
+//   R = R0 + e,   R0 = |x0 - s_p|,   e = (2 u.d + |d|^2) / (R + R0)
+// with x0 a reference pixel of the tile, u = x0 - s_p and d = x - x0.  R0, its
+// phase factor T = exp(j 4 pi R0/lambda) and its range index are formed once
+// per pulse and workgroup (PlainRec in LDS); the excess e of a pixel is a
+// quartic in the pulse index over the tile's window, interpolated at five
+// Chebyshev pulses.  Within a block of up to 2 kPlainHalf pulses the quartic
+// is a quadratic to 2e-11 m, so the index advances by differences and the
+// phase factor by a rotation (PlainBlock).  25 instructions per pair in a full
+// block, 33 over the launch with the blocks' and tiles' set-up, all in FP64
+// but the lerp, which is FP32 as in plain_pair.
+//
+// What the form rests on is checked: per pixel the quartic at the window's
+// two ends (1e-10 m, the rounding of R itself in FP64 at 8.5e5 m) and the
+// block length against its derivatives, per pulse the look vector u/R0
+// against its own quartic (1e-10 m at the tile's farthest pixel: a pulse
+// position that does not fit the others) and the range gate with the bound on
+// e.  Waves or stages that miss a check take plain_pair pair by pair.
+//
+// One IW burst (1500 x 21000 samples, 4000 x 1500 pixels, 3.05e9 pairs): 3.15
+// ms against 7.0 ms pair by pair, errors against 64 bits 7e-8 either way (the
+// FP32 lerp's).  With z *= w, w *= v pulse after pulse instead of pairs about
+// the block's centre: 3.6 ms (37 instructions per pair); blocks of 64 pulses:
+// 3.25 ms; 256 pulses per stage: 3.25 ms.
+constexpr int kPlainNodes = 5;    // interpolation pulses; two more check the ends
+constexpr int kPlainHalf = 16;    // half the pulses of a full block
+constexpr int kPlainStage = 768;  // pulses per stage of records (24 KB of LDS)
+constexpr double kPlainTol = 1e-10;
+
+struct PlainRec {
+  double rb;       // (R0 - rngstart)/dmrg
+  double tr, ti;   // T
+  double pad;
+};
+
+struct PlainShared {
+  double x0[3];
+  double u[kPlainNodes + 2][3], r2[kPlainNodes + 2], R0[kPlainNodes + 2], t[kPlainNodes + 2];
+  double rcp[10];                 // 1/(t_j - t_i) in the order newton4 takes them
+  double look[3][kPlainNodes];    // u/R0 per component, monomials in t
+  int key, wlo, whi;
+  unsigned dmax, emax;            // FP32 bits of max |x - x0|, of max sum |coefficient|
+};
+
+// Quartic through (t[j], y[j]), j < 5, as monomial coefficients: Newton's
+// divided differences (rcp: reciprocals of the node distances, level by
+// level), then multiplied out.
+__device__ __forceinline__ void newton4(const double* t, const double* rcp, const double* y,
+                                        double* c) {
+  double a[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) a[i] = y[i];
+  int k = 0;
+#pragma unroll
+  for (int l = 1; l < 5; ++l) {
+#pragma unroll
+    for (int i = 4; i >= l; --i) a[i] = (a[i] - a[i - 1]) * rcp[k + i - l];
+    k += 5 - l;
+  }
+#pragma unroll
+  for (int i = 0; i < 5; ++i) c[i] = 0.0;
+  c[0] = a[4];
+#pragma unroll
+  for (int l = 3; l >= 0; --l) {   // c(t) <- c(t) (t - t_l) + a_l
+#pragma unroll
+    for (int i = 4; i >= 1; --i) c[i] = fma(-t[l], c[i], c[i - 1]);
+    c[0] = fma(-t[l], c[0], a[l]);
+  }
+}
+
+__device__ __forceinline__ double quartic(const double* c, double t) {
+  return fma(fma(fma(fma(c[4], t, c[3]), t, c[2]), t, c[1]), t, c[0]);
+}
+
+// 1/x for normal x: the hardware estimate and two Newton steps.
+__device__ __forceinline__ double rcp64(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+
+// exp(2 pi j c) for any c of moderate size.
+__device__ __forceinline__ void cis_cycles(double c, double* re, double* im) {
+  sincos_2pi(c - rint(c), im, re);
+}
+
+// One block of pulses, summed from its centre outward in pairs at k = -(j +
+// 1/2) and j + 1/2 pulses from it.  With the excess e0 + a1 k + a2 k^2 the
+// phase factors of a pair are z0 g u* and z0 g u, u = exp(j 4 pi/lambda a1 k)
+// and g = exp(j 4 pi/lambda a2 k^2) common to both: one complex product by u
+// of the sum and difference of the two samples, one by g (|phase| <= 1e-3,
+// taken to second order), z0 once per block.  u advances by the three-term
+// recurrence u_{j+1} = 2 cos(theta) u_j - u_{j-1}.
+struct PlainBlock {
+  double pp, dp, pm, dm, d2;   // excess in samples at +-k, differences outward
+  double ur, ui, vr, vi, cc;   // u, the u before it, 2 cos(theta)
+  double eps;                  // phase of g is eps k^2
+  double ar, ai;               // the block's sum without z0
+};
+// What a pair holds between its loads and its use.
+struct PlainFront {
+  SbufF4 vp, vm;
+  float fp, fm;
+};
+
+// The loads of the pair whose records are rp (k > 0) and rm, rows at byte
+// offsets sp and sm; advances the index.
+__device__ __forceinline__ PlainFront plain_front(PlainBlock& s, const PlainRec& rp,
+                                                  const PlainRec& rm, const I32x4& rsrc,
+                                                  unsigned sp, unsigned sm) {
+  PlainFront f;
+  const double xp = rp.rb + s.pp, xm = rm.rb + s.pm;
+  f.vp = sbuf_load_v4f32(rsrc, (int)xp, 0, (int)sp, 0);   // xp >= 0: truncation is floor
+  f.vm = sbuf_load_v4f32(rsrc, (int)xm, 0, (int)sm, 0);
+  s.pp += s.dp;
+  s.pm += s.dm;
+  s.dp += s.d2;
+  s.dm += s.d2;
+  f.fp = (float)__builtin_amdgcn_fract(xp);
+  f.fm = (float)__builtin_amdgcn_fract(xm);
+  return f;
+}
+// The pair's sum.  inp, inm (MASK): lanes outside their window add nothing.
+template <bool MASK>
+__device__ __forceinline__ void plain_back(PlainBlock& s, const PlainRec& rp, const PlainRec& rm,
+                                           const PlainFront& f, double k2, bool inp, bool inm) {
+  float pr = fmaf(f.fp, f.vp.z - f.vp.x, f.vp.x), pi = fmaf(f.fp, f.vp.w - f.vp.y, f.vp.y);
+  float mr = fmaf(f.fm, f.vm.z - f.vm.x, f.vm.x), mi = fmaf(f.fm, f.vm.w - f.vm.y, f.vm.y);
+  if constexpr (MASK) {
+    pr = inp ? pr : 0.f;
+    pi = inp ? pi : 0.f;
+    mr = inm ? mr : 0.f;
+    mi = inm ? mi : 0.f;
+  }
+  const double dpr = pr, dpi = pi, dmr = mr, dmi = mi;
+  const double Pr = fma(-dpi, rp.ti, dpr * rp.tr), Pi = fma(dpi, rp.tr, dpr * rp.ti);
+  const double Mr = fma(-dmi, rm.ti, dmr * rm.tr), Mi = fma(dmi, rm.tr, dmr * rm.ti);
+  const double Sr = Pr + Mr, Si = Pi + Mi, Dr = Pr - Mr, Di = Pi - Mi;
+  // P u + M u*
+  const double qr = fma(-Di, s.ui, Sr * s.ur), qi = fma(Dr, s.ui, Si * s.ur);
+  const double x = s.eps * k2;
+  const double g = fma(-0.5 * x, x, 1.0);
+  s.ar = fma(qr, g, s.ar);
+  s.ar = fma(-qi, x, s.ar);
+  s.ai = fma(qi, g, s.ai);
+  s.ai = fma(qr, x, s.ai);
+  const double nr = fma(s.cc, s.ur, -s.vr), ni = fma(s.cc, s.ui, -s.vi);
+  s.vr = s.ur;
+  s.vi = s.ui;
+  s.ur = nr;
+  s.ui = ni;
+}
+
+// The 2 m pulses around the pair (rec[-1], rec[0]): rec points at the record
+// just after the centre, so at its row's byte offset.  One pair's loads are
+// in flight ahead of their use.  m = M when M > 0 (unrolled), else mm.  MASK:
+// pulse q0 + i belongs to rec[i]; the lane's window is [azs, azs + na).
+template <int M, bool MASK>
+__device__ __forceinline__ void plain_pulses(PlainBlock& s, const PlainRec* rec, int mm,
+                                             const I32x4& rsrc, unsigned so, unsigned rb32,
+                                             int q0, int azs, unsigned na) {
+  auto in = [&](int i) { return (unsigned)(q0 + i - azs) < na; };
+  auto front = [&](int j) {
+    return plain_front(s, rec[j], rec[-1 - j], rsrc, so + (unsigned)j * rb32,
+                       so - (unsigned)(j + 1) * rb32);
+  };
+  auto back = [&](int j, const PlainFront& f) {
+    plain_back<MASK>(s, rec[j], rec[-1 - j], f, (double)(j * (j + 1)) + 0.25, in(j), in(-1 - j));
+  };
+  PlainFront a = front(0), b;
+  if constexpr (M > 0) {
+#pragma unroll
+    for (int j = 0; j < M; j += 2) {
+      b = front(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      back(j, a);
+      if (j + 2 < M) a = front(j + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      back(j + 1, b);
+    }
+  } else {
+    int j = 0;
+    for (; j + 2 < mm; j += 2) {
+      b = front(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      back(j, a);
+      a = front(j + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      back(j + 1, b);
+    }
+    if (j + 1 < mm) {
+      b = front(j + 1);
+      back(j, a);
+      back(j + 1, b);
+    } else {
+      back(j, a);
+    }
+  }
+}
+
+// One block of n <= 2 * kPlainHalf pulses from pulse q, whose record is rec[0],
+// added to (ar, ai).  core: n is even and every live lane is inside its
+// window.  Else lanes are masked by theirs; an odd n takes one more pulse,
+// masked on every lane (its record exists: a stage has one more than its
+// pulses).
+__device__ __forceinline__ void plain_block(const double* c, double dt, int wlo, int q, int n,
+                                            const PlainRec* rec, const I32x4& rsrc, unsigned rb32,
+                                            bool core, int azs, unsigned na, double cyc_per_m,
+                                            double smp_per_m, double& ar, double& ai) {
+  const int m = (n + 1) >> 1;
+  const double h = m, hi = m == kPlainHalf ? 1.0 / kPlainHalf : 1.0 / m;
+  // the quadratic through the quartic at the centre and m pulses to each side
+  const double tc = fma((double)(q - wlo) + (m - 0.5), dt, -1.0);
+  const double e0 = quartic(c, tc), em = quartic(c, fma(-h, dt, tc)),
+               ep = quartic(c, fma(h, dt, tc));
+  const double a1 = (ep - em) * (0.5 * hi);
+  const double a2 = ((ep - e0) - (e0 - em)) * (0.5 * hi * hi);
+  PlainBlock s;
+  s.d2 = 2.0 * a2 * smp_per_m;
+  s.pp = fma(0.5, a1, fma(0.25, a2, e0)) * smp_per_m;
+  s.pm = fma(-0.5, a1, fma(0.25, a2, e0)) * smp_per_m;
+  s.dp = fma(2.0, a2, a1) * smp_per_m;
+  s.dm = fma(2.0, a2, -a1) * smp_per_m;
+  s.eps = a2 * (cyc_per_m * 6.283185307179586);
+  cis_cycles(0.5 * a1 * cyc_per_m, &s.ur, &s.ui);
+  s.vr = s.ur;
+  s.vi = -s.ui;
+  s.cc = fma(-4.0 * s.ui, s.ui, 2.0);
+  s.ar = 0.;
+  s.ai = 0.;
+  const unsigned so = (unsigned)(q + m) * rb32;
+  if (core && n == 2 * kPlainHalf)
+    plain_pulses<kPlainHalf, false>(s, rec + m, m, rsrc, so, rb32, q + m, azs, na);
+  else if (core)
+    plain_pulses<0, false>(s, rec + m, m, rsrc, so, rb32, q + m, azs, na);
+  else
+    plain_pulses<0, true>(s, rec + m, m, rsrc, so, rb32, q + m, azs,
+                          (unsigned)max(0, min((int)na, q + n - azs)));
+  double zr, zi;
+  cis_cycles(e0 * cyc_per_m, &zr, &zi);
+  ar = fma(s.ar, zr, ar);
+  ar = fma(-s.ai, zi, ar);
+  ai = fma(s.ar, zi, ai);
+  ai = fma(s.ai, zr, ai);
+}
+
+template <int TR, bool STACK>
+__device__ __forceinline__ void plain_excess_tile(const BurstDev& b, int tile, PlainRec* rec,
+                                                  PlainShared* sh) {
+  PixelCtx p = pixel_of<TR, STACK>(b, tile);
+  const int tid = threadIdx.x;
+  const bool live = p.aze > p.azs;
+  double x[3] = {0., 0., 0.};
+  if (live) pixel_ecef(b, p.row, p.col, x);
+
+  // Tile window and reference pixel (the live one nearest the centre).
+  constexpr int TC = kWave / TR;
+  constexpr int WR = STACK ? 4 * TR : TR, WC = STACK ? TC : 4 * TC;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wr = (STACK ? wave * TR : 0) + lane / TC;
+  const int wc = (STACK ? 0 : wave * TC) + lane % TC;
+  if (tid == 0) {
+    sh->key = 0x7fffffff;
+    sh->wlo = 0x7fffffff;
+    sh->whi = -1;
+    sh->dmax = 0u;
+    sh->emax = 0u;
+  }
+  __syncthreads();
+  if (live) {
+    atomicMin(&sh->key, (abs(2 * wr - WR) + abs(2 * wc - WC)) * 256 + tid);
+    atomicMin(&sh->wlo, p.azs);
+    atomicMax(&sh->whi, p.aze);
+  }
+  __syncthreads();
+  const int ref = sh->key;
+  if (ref == 0x7fffffff) {  // nothing to compute in this tile
+    store_out(b, p, 0.f, 0.f);
+    return;
+  }
+  const int wlo = __builtin_amdgcn_readfirstlane(sh->wlo);
+  const int whi = __builtin_amdgcn_readfirstlane(sh->whi);
+  if ((ref & 255) == tid) {
+    sh->x0[0] = x[0];
+    sh->x0[1] = x[1];
+    sh->x0[2] = x[2];
+  }
+  __syncthreads();
+  const double x0[3] = {uniform(sh->x0[0]), uniform(sh->x0[1]), uniform(sh->x0[2])};
+
+  // The quartics need 32 pulses to have distinct nodes, the gather 32-bit
+  // byte offsets into the burst.
+  const unsigned rb32 = (unsigned)b.S * 8u;
+  const bool quart = whi - wlo >= 32 && (size_t)b.L * b.S * 8u < (size_t)0x7fffffff;
+  // t = (q - wlo) dt - 1 maps the window's pulses to [-1, 1].
+  const double dt = quart ? 2.0 / (whi - 1 - wlo) : 0.0;
+  double c[kPlainNodes] = {0., 0., 0., 0., 0.};
+  bool fit = false;
+  int half = 1;   // longest half block the lane's quartic allows
+  if (quart) {
+    // Threads 0..6: the node pulses (Chebyshev points, then the two ends).
+    const int span = whi - 1 - wlo;
+    auto node_pulse = [&](int j) {
+      // (1 - cos((2 j + 1) pi / 10)) / 2
+      const double g[kPlainNodes] = {0.024471741852423214, 0.20610737385376343, 0.5,
+                                     0.79389262614623657, 0.97552825814757679};
+      double f = j == kPlainNodes ? 0.0 : 1.0;
+#pragma unroll
+      for (int i = 0; i < kPlainNodes; ++i) f = j == i ? g[i] : f;
+      return wlo + (int)rint(f * span);
+    };
+    if (tid < kPlainNodes + 2) {
+      const int q = node_pulse(tid);
+      const double* s = b.satloc + 3 * q;
+      const double u0 = x0[0] - s[0], u1 = x0[1] - s[1], u2 = x0[2] - s[2];
+      const double r2 = u0 * u0 + u1 * u1 + u2 * u2;
+      sh->u[tid][0] = u0;
+      sh->u[tid][1] = u1;
+      sh->u[tid][2] = u2;
+      sh->r2[tid] = r2;
+      sh->R0[tid] = range_sqrt(r2);
+      sh->t[tid] = fma((double)(q - wlo), dt, -1.0);
+    }
+    __syncthreads();
+    if (tid < 10) {   // level l, place i: nodes i and i + l
+      const int l = tid < 4 ? 1 : tid < 7 ? 2 : tid < 9 ? 3 : 4;
+      const int i = tid - (l == 1 ? 0 : l == 2 ? 4 : l == 3 ? 7 : 9);
+      sh->rcp[tid] = 1.0 / (sh->t[i + l] - sh->t[i]);
+    }
+    __syncthreads();
+    if (tid < 3) {    // component tid of the look vector
+      double y[kPlainNodes], l[kPlainNodes];
+      for (int j = 0; j < kPlainNodes; ++j) y[j] = sh->u[j][tid] / sh->R0[j];
+      newton4(sh->t, sh->rcp, y, l);
+      for (int j = 0; j < kPlainNodes; ++j) sh->look[tid][j] = l[j];
+    }
+    if (live) {
+      const double d0 = x[0] - x0[0], d1 = x[1] - x0[1], d2 = x[2] - x0[2];
+      const double bb = d0 * d0 + d1 * d1 + d2 * d2;
+      double y[kPlainNodes + 2];
+#pragma unroll
+      for (int j = 0; j < kPlainNodes + 2; ++j) {
+        const double num =
+            fma(2.0, fma(sh->u[j][0], d0, fma(sh->u[j][1], d1, sh->u[j][2] * d2)), bb);
+        y[j] = num * rcp64(range_sqrt(sh->r2[j] + num) + sh->R0[j]);
+        __builtin_amdgcn_sched_barrier(0);   // one node's operands at a time
+      }
+      newton4(sh->t, sh->rcp, y, c);
+      const double el = fabs(quartic(c, sh->t[kPlainNodes]) - y[kPlainNodes]);
+      const double eh = fabs(quartic(c, sh->t[kPlainNodes + 1]) - y[kPlainNodes + 1]);
+      fit = el <= kPlainTol && eh <= kPlainTol;   // false for NaN
+      // Second and third derivative over [-1, 1] per pulse: a block of half
+      // length h has |eps k^2| <= 2 pi cycles c2 h^2 and leaves c3 h^3 (0.385
+      // its largest value over the block) of the quartic.
+      const double c2 =
+          (fabs(c[2]) + 3.0 * fabs(c[3]) + 6.0 * fabs(c[4])) * dt * dt * b.two_over_wvl * 6.2832;
+      const double c3 = (fabs(c[3]) + 4.0 * fabs(c[4])) * dt * dt * dt * 0.385;
+      half = kPlainHalf;
+      while (half > 1 && !(c2 * half * half <= 1e-3 && c3 * half * half * half <= 2e-11))
+        half >>= 1;
+      fit = fit && half >= 4;
+      // |quartic| <= sum |c_j| on [-1, 1]; FP32 rounded up.
+      const double em = fabs(c[0]) + fabs(c[1]) + fabs(c[2]) + fabs(c[3]) + fabs(c[4]);
+      if (fit) atomicMax(&sh->emax, __float_as_uint((float)(em * (1.0 + 1e-6))));
+      atomicMax(&sh->dmax, __float_as_uint((float)(sqrt(bb) * (1.0 + 1e-6))));
+    }
+    __syncthreads();
+  }
+  const bool wave_fit = quart && wave_min(live && !fit ? 0 : 1) == 1;
+  const int blk = 2 * wave_min(live ? half : kPlainHalf);
+  // Bound on the excess the recurrences can form, in samples: a block's
+  // quadratic through three values of the quartic stays within 5/4 of their
+  // largest, and those lie at most 1 1/2 pulses outside the window, |t| <=
+  // 1.1; two samples of margin.
+  const double ext =
+      2.0 * (double)__uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)sh->emax)) *
+          b.inv_dmrg + 2.0;
+  const double dmax =
+      (double)__uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)sh->dmax));
+
+  const int qlo = wave_min(live ? p.azs : 0x7fffffff);
+  const int qhi = wave_max(live ? p.aze : -1);
+  const int qc0 = wave_max(live ? p.azs : -1);         // every live lane inside
+  const int qc1 = wave_min(live ? p.aze : 0x7fffffff); // its window in [qc0, qc1)
+  const bool wave_live = qhi > qlo;
+  const unsigned na = (unsigned)(p.aze - p.azs);
+  const float2* base = (const float2*)b.data;
+  const const_dptr sat = (const_dptr)b.satloc;
+  I32x4 rsrc;   // one record per sample; indices past S - 2 read zeros
+  {
+    const unsigned long long a = (unsigned long long)b.data;
+    rsrc.x = __builtin_amdgcn_readfirstlane((int)(unsigned)a);
+    rsrc.y = __builtin_amdgcn_readfirstlane((int)(((unsigned)(a >> 32) & 0xffffu) | (8u << 16)));
+    rsrc.z = b.S - 1;
+    rsrc.w = kSbufWord3Raw32;
+  }
+
+  double ar = 0., ai = 0.;
+  for (int p0 = wlo; p0 < whi; p0 += kPlainStage) {
+    const int p1 = min(p0 + kPlainStage, whi);
+    bool safe = quart;
+    for (int q = p0 + tid; quart && q < p1; q += kBlock) {
+      const double* s = b.satloc + 3 * q;
+      const double u0 = x0[0] - s[0], u1 = x0[1] - s[1], u2 = x0[2] - s[2];
+      const double r2 = u0 * u0 + u1 * u1 + u2 * u2;
+      const double R0 = range_sqrt(r2), inv = rcp64(R0);
+      const double t = fma((double)(q - wlo), dt, -1.0);
+      const double dev = fmax(fmax(fabs(quartic(sh->look[0], t) - u0 * inv),
+                                   fabs(quartic(sh->look[1], t) - u1 * inv)),
+                              fabs(quartic(sh->look[2], t) - u2 * inv));
+      PlainRec r;
+      r.rb = (R0 - b.rngstart) * b.inv_dmrg;
+      cis_cycles(R0 * b.two_over_wvl, &r.tr, &r.ti);
+      r.pad = 0.;
+      rec[q - p0] = r;
+      safe = safe && r.rb - ext >= 0.0 && r.rb + ext <= b.r_hi && dev * dmax <= kPlainTol;
+    }
+    // The masked pulse of an odd last block: an index past every row reads
+    // nothing.
+    if (tid == 0) rec[p1 - p0] = PlainRec{-1e9, 0., 0., 0.};
+    const int stage_safe = __syncthreads_and(safe ? 1 : 0);
+    if (wave_live) {
+      const int qa = max(p0, qlo), qb = min(p1, qhi);
+      if (wave_fit && stage_safe) {
+        for (int q = qa; q < qb;) {
+          const int ce = min(qb, qc1);
+          const bool core = q >= qc0 && q + 1 < ce;
+          const int n = core ? min(blk, ce - q) & ~1
+                             : min(blk, (q < qc0 ? min(qb, qc0) : qb) - q);
+          plain_block(c, dt, wlo, q, n, rec + (q - p0), rsrc, rb32, core, p.azs, na,
+                      b.two_over_wvl, b.inv_dmrg, ar, ai);
+          q += n;
+        }
+      } else {
+        for (int q = qa; q < qb; ++q) {
+          const double sx = sat[3 * q], sy = sat[3 * q + 1], sz = sat[3 * q + 2];
+          if ((unsigned)(q - p.azs) < na)
+            plain_pair(base + (size_t)q * b.S, x, sx, sy, sz, b, ar, ai);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  store_out(b, p, (float)ar, (float)ai);
 }
 
 template <int TR, bool STACK, int DT, bool LDS = false>
@@ -1694,10 +2135,23 @@ __device__ __forceinline__ void mfma_tile(const BurstDev& b, int tile, MShared& 
 
 // ----------------------------------------------------------- kernels
 
+// Occupancy target of the FP64 kernels: 3 waves per SIMD leave 168 VGPRs, which
+// hold a block's recurrences without spills; the loads run a pair ahead, and
+// the kernel keeps VALU busy 91 % of its cycles (one IW burst: 3.15 ms at 3,
+// 3.2 at 4 with spills outside the loops, 3.9 at 5).
+#define TDBP_PLAIN_OCC __attribute__((amdgpu_waves_per_eu(3)))
+
 template <int TR, bool STACK, bool CPU>
-__global__ __launch_bounds__(kBlock) void k_plain(BurstDev b) {
+__global__ __launch_bounds__(kBlock) TDBP_PLAIN_OCC void k_plain(BurstDev b) {
   __shared__ int item;
-  persistent_tiles(b, &item, [&](int tile) { plain_tile<TR, STACK, CPU>(b, tile); });
+  if constexpr (CPU) {
+    persistent_tiles(b, &item, [&](int tile) { cpu_tile<TR, STACK>(b, tile); });
+  } else {
+    __shared__ PlainRec rec[kPlainStage + 1];
+    __shared__ PlainShared sh;
+    persistent_tiles(b, &item,
+                     [&](int tile) { plain_excess_tile<TR, STACK>(b, tile, rec, &sh); });
+  }
 }
 
 // Occupancy target of the mixed kernels: 8 waves per SIMD, the hardware
@@ -1765,12 +2219,12 @@ __global__ __launch_bounds__(kMBlock) TDBP_MIXED_OCC void k_batch_mfma(
 
 // Persistent batch kernel: workgroup on XCD x = blockIdx % 8 drains queue x,
 // then steals from the others.  Queue k holds items [qbase[k], qbase[k+1]).
-template <int PREC, int TR, bool STACK, int DT, bool LDS = false>
+template <int PREC, int TR, bool STACK, int DT, bool LDS = false, class REC, class SHARED>
 __device__ __forceinline__ void batch_body(const BurstDev* __restrict__ bursts,
                                            const int2* __restrict__ items,
                                            const int* __restrict__ qbase,
-                                           int* counters, PulseRec* rec,
-                                           TileShared* sh, int* item_s,
+                                           int* counters, REC* rec,
+                                           SHARED* sh, int* item_s,
                                            F32x4* sbuf = nullptr) {
   const int home = blockIdx.x & 7;
   int qi = 0;
@@ -1792,9 +2246,9 @@ __device__ __forceinline__ void batch_body(const BurstDev* __restrict__ bursts,
     if constexpr (PREC == TDBP_MIXED) {
       mixed_tile<TR, STACK, DT, LDS>(bd, w.y, rec, sh, sbuf);
     } else if (bd.cpu) {
-      plain_tile<TR, STACK, true>(bd, w.y);
+      cpu_tile<TR, STACK>(bd, w.y);
     } else {
-      plain_tile<TR, STACK, false>(bd, w.y);
+      plain_excess_tile<TR, STACK>(bd, w.y, rec, sh);
     }
     __syncthreads();
   }
@@ -1823,12 +2277,14 @@ __global__ __launch_bounds__(kBlock) TDBP_LDS_OCC void k_batch_mixed_lds(
 }
 
 template <int TR, bool STACK>
-__global__ __launch_bounds__(kBlock) void k_batch_plain(
+__global__ __launch_bounds__(kBlock) TDBP_PLAIN_OCC void k_batch_plain(
     const BurstDev* __restrict__ bursts, const int2* __restrict__ items,
     const int* __restrict__ qbase, int* counters) {
+  __shared__ PlainRec rec[kPlainStage + 1];
+  __shared__ PlainShared sh;
   __shared__ int item_s;
-  batch_body<TDBP_PLAIN_FP64, TR, STACK, TDBP_CF32>(bursts, items, qbase, counters,
-                                                     nullptr, nullptr, &item_s);
+  batch_body<TDBP_PLAIN_FP64, TR, STACK, TDBP_CF32>(bursts, items, qbase, counters, rec, &sh,
+                                                     &item_s);
 }
 
 // One thread per window line: three zero-Doppler solves, the aperture

@@ -66,6 +66,61 @@ TDBP_HD void hermite4(const double* x4, const double* v4, const double* t4,
   }
 }
 
+// a / b, correctly rounded, from the correctly rounded reciprocal r of b
+// (Markstein's theorem; a, b and a / b normal or zero): three instructions
+// where a division takes a dozen.
+TDBP_HD double div_by(double a, double b, double r) {
+  const double q = a * r;
+  return fma(fma(-q, b, a), r, q);
+}
+
+// hermite4 split by sample, one per lane of a quad: sample i's time, the
+// other three in ascending order with the differences ti - tj and their
+// reciprocals.  hermite_term gives the sample's terms of the position and
+// velocity sums, bit for bit those of hermite4; added in sample order they are
+// its result.
+struct HermiteNode {
+  double ti, tj[3], d[3], r[3], x[3], v[3];
+};
+TDBP_HD void hermite_term(const HermiteNode& n, double time, double* pos, double* vel) {
+#pragma clang fp contract(off)
+  double sinv = 0.0, h = 1.0, hd = 0.0;
+  for (int j = 0; j < 3; ++j) sinv = sinv + n.r[j];
+  const double f1 = time - n.ti;
+  const double f0 = 1.0 - 2.0 * f1 * sinv;
+  for (int k = 0; k < 3; ++k) h = div_by(h * (time - n.tj[k]), n.d[k], n.r[k]);
+  for (int j = 0; j < 3; ++j) {
+    double q = 1.0;
+    for (int k = 0; k < 3; ++k)
+      if (k != j) q = div_by(q * (time - n.tj[k]), n.d[k], n.r[k]);
+    hd = hd + n.r[j] * q;
+  }
+  const double g1 = h + 2.0 * f1 * hd;
+  const double g0 = 2.0 * (f0 * hd - h * sinv);
+  for (int k = 0; k < 3; ++k) {
+    pos[k] = (n.x[k] * f0 + n.v[k] * f1) * h * h;
+    vel[k] = (n.x[k] * g0 + n.v[k] * g1) * h;
+  }
+}
+// Sample i of the four state vectors from t, x, v; false where a difference of
+// their times has no finite reciprocal (hermite4 then divides as it is).
+TDBP_HD bool hermite_node(const double* t, const double* x, const double* v, int i,
+                          HermiteNode* n) {
+  n->ti = t[i];
+  bool ok = true;
+  for (int j = 0; j < 3; ++j) {
+    n->tj[j] = t[j < i ? j : j + 1];
+    n->d[j] = n->ti - n->tj[j];
+    n->r[j] = 1.0 / n->d[j];
+    ok = ok && fabs(n->r[j]) < 1e100 && fabs(n->r[j]) > 1e-100;
+  }
+  for (int k = 0; k < 3; ++k) {
+    n->x[k] = x[3 * i + k];
+    n->v[k] = v[3 * i + k];
+  }
+  return ok;
+}
+
 // State-vector selection of sentinel/intp_orbit.f90:6-20: 1-based index
 // int((t - t1)/dt) clamped to [2, n-2], Hermite over the 4 vectors starting
 // one before it.  t/x/v are the orbit arrays (x, v as [n][3]).
@@ -84,30 +139,6 @@ TDBP_HD double dot3(const double* a, const double* b) {
   double s = 0.0;
   for (int i = 0; i < 3; ++i) s = s + a[i] * b[i];
   return s;
-}
-
-// Zero-Doppler range of a ground point: Newton on (x - s(t)).v(t) with the
-// derivative taken as -|v|^2, at most 51 steps, stop at |dt| < 5e-9 s
-// (sentinel/orbitrangetime.f90:23-69).  s0/v0 are the starting state and are
-// not modified.
-TDBP_HD double zero_doppler_range(const double* xyz, const double* t,
-                                  const double* x, const double* v, int n,
-                                  double t0, const double* s0,
-                                  const double* v0) {
-#pragma clang fp contract(off)
-  double tl = t0, sx[3] = {s0[0], s0[1], s0[2]}, sv[3] = {v0[0], v0[1], v0[2]};
-  double dr[3];
-  for (int k = 0; k < 51; ++k) {
-    const double tprev = tl;
-    for (int i = 0; i < 3; ++i) dr[i] = xyz[i] - sx[i];
-    const double fn = dot3(dr, sv);
-    const double fnprime = -dot3(sv, sv) + 0.0 * fn;
-    tl = tl - fn / fnprime;
-    orbit_at(t, x, v, n, tl, sx, sv);
-    if (fabs(tl - tprev) < 5.0e-9) break;
-  }
-  for (int i = 0; i < 3; ++i) dr[i] = xyz[i] - sx[i];
-  return sqrt(dot3(dr, dr));
 }
 
 // WGS-84 geodetic -> ECEF of DEM sample (window line `line`, column `pixel`)
@@ -185,14 +216,11 @@ struct FitParams {
 };
 
 // Pulse index of the aperture centre of ground point p
-// (sentinel/azimuth_compress.cu:451-465): zero-Doppler range from the Newton
-// solve started at mid-burst, Doppler of p seen from the mid-burst state,
-// TOPS time offset td, n = int(td*prf + L/2).
-TDBP_HD int aperture_centre(const double* p, const double* t, const double* x,
-                            const double* v, int n, const FitParams& f) {
+// (sentinel/azimuth_compress.cu:451-465) from its zero-Doppler range: Doppler
+// of p seen from the mid-burst state, TOPS time offset td, n = int(td*prf +
+// L/2).
+TDBP_HD int aperture_centre(const double* p, double rngpix, const FitParams& f) {
 #pragma clang fp contract(off)
-  const double rngpix = zero_doppler_range(p, t, x, v, n, f.tmid, f.xyz_mid,
-                                           f.vel_mid);
   double u[3];
   for (int i = 0; i < 3; ++i) u[i] = p[i] - f.xyz_mid[i];
   const double umag = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);

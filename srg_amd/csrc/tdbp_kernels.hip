@@ -2287,15 +2287,87 @@ __global__ __launch_bounds__(kBlock) TDBP_PLAIN_OCC void k_batch_plain(
                                                      &item_s);
 }
 
-// One thread per window line: three zero-Doppler solves, the aperture
-// centres, the parabola.  Lines at or beyond nfit get (0, 0, 0).
+// The aperture fit is a latency chain (Newton steps of a 4-point Hermite
+// interpolation full of divisions, bit for bit the oracle's), so a window line
+// takes 16 lanes: a quad per fit node, a lane per state vector of the
+// interpolation, the divisions by state-vector times through their
+// reciprocals.  256 lines: 8 us; one lane per line, 60 divisions a step, took
+// 80 us at any line count up to the card's width.
+constexpr int kFitLanes = 16;
+
+// Lane J's double, on every lane of its quad.
+template <int J>
+__device__ __forceinline__ double quad_lane(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffll), J * 0x55, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), J * 0x55, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double quad_sum(double v) {
+#pragma clang fp contract(off)
+  return ((0.0 + quad_lane<0>(v) + quad_lane<1>(v)) + quad_lane<2>(v)) + quad_lane<3>(v);
+}
+
+// Zero-Doppler range of ground point xyz by a quad: Newton on (x - s(t)).v(t)
+// with the derivative taken as -|v|^2, at most 51 steps, stop at |dt| < 5e-9 s
+// (sentinel/orbitrangetime.f90:23-69), from the state (t0, s0, v0).  The state
+// vectors as orbit_at selects them.
+__device__ __forceinline__ double zero_doppler_range(const double* xyz, const double* t,
+                                                     const double* x, const double* v, int n,
+                                                     double t0, const double* s0,
+                                                     const double* v0) {
+#pragma clang fp contract(off)
+  const double dt = t[1] - t[0], rdt = 1.0 / dt;
+  const bool plain_dt = !(fabs(rdt) < 1e100 && fabs(rdt) > 1e-100);
+  double tl = t0, sx[3] = {s0[0], s0[1], s0[2]}, sv[3] = {v0[0], v0[1], v0[2]};
+  double dr[3];
+  HermiteNode node;
+  int have = -1;
+  bool split = false;
+  for (int k = 0; k < 51; ++k) {
+    const double tprev = tl;
+    for (int i = 0; i < 3; ++i) dr[i] = xyz[i] - sx[i];
+    const double fn = dot3(dr, sv);
+    const double fnprime = -dot3(sv, sv) + 0.0 * fn;
+    tl = tl - fn / fnprime;
+    int iloc = (int)(plain_dt ? (tl - t[0]) / dt : div_by(tl - t[0], dt, rdt));
+    iloc = iloc < 2 ? 2 : iloc;
+    iloc = iloc > n - 2 ? n - 2 : iloc;
+    const int first = iloc - 2;
+    if (first != have) {   // the same on the quad's four lanes
+      const bool ok =
+          hermite_node(t + first, x + 3 * first, v + 3 * first, threadIdx.x & 3, &node);
+      const int bad = ok ? 0 : 1;
+      split = (__builtin_amdgcn_mov_dpp(bad, 0x00, 0xf, 0xf, true) |
+               __builtin_amdgcn_mov_dpp(bad, 0x55, 0xf, 0xf, true) |
+               __builtin_amdgcn_mov_dpp(bad, 0xaa, 0xf, 0xf, true) |
+               __builtin_amdgcn_mov_dpp(bad, 0xff, 0xf, 0xf, true)) == 0;
+      have = first;
+    }
+    if (split) {
+      double p[3], w[3];
+      hermite_term(node, tl, p, w);
+      for (int i = 0; i < 3; ++i) {
+        sx[i] = quad_sum(p[i]);
+        sv[i] = quad_sum(w[i]);
+      }
+    } else {
+      hermite4(x + 3 * first, v + 3 * first, t + first, tl, sx, sv);
+    }
+    if (fabs(tl - tprev) < 5.0e-9) break;
+  }
+  for (int i = 0; i < 3; ++i) dr[i] = xyz[i] - sx[i];
+  return sqrt(dot3(dr, dr));
+}
+
+// Three zero-Doppler solves of a window line, the aperture centres, the
+// parabola, by its kFitLanes lanes.  Lines at or beyond nfit get (0, 0, 0).
 __device__ __forceinline__ void fit_line(const BurstDev& b, int line,
                                          double* coef) {
   double* c = coef + 3 * line;
+  const int sub = threadIdx.x & (kFitLanes - 1);
   if (line >= b.nfit) {
-    c[0] = 0.;
-    c[1] = 0.;
-    c[2] = 0.;
+    if (sub < 3) c[sub] = 0.;
     return;
   }
   FitParams f;
@@ -2309,25 +2381,26 @@ __device__ __forceinline__ void fit_line(const BurstDev& b, int line,
     f.xyz_mid[i] = b.xyz_mid[i];
     f.vel_mid[i] = b.vel_mid[i];
   }
-  const int step = fit_node_step(b.firstpix, b.lastpix);
-  int y[3];
-  for (int node = 0; node < 3; ++node) {
-    const int pix = b.firstpix + node * step;
-    double xyz[3];
-    pixel_ecef(b, line, pix, xyz);
-    y[node] = aperture_centre(xyz, b.orb_t, b.orb_x, b.orb_v, b.nsv, f);
-  }
-  parabola(y[0], y[1], y[2], c);
+  const int node = min(sub >> 2, 2);   // the fourth quad repeats the third's
+  const int pix = b.firstpix + node * fit_node_step(b.firstpix, b.lastpix);
+  double xyz[3];
+  pixel_ecef(b, line, pix, xyz);
+  const double rng = zero_doppler_range(xyz, b.orb_t, b.orb_x, b.orb_v, b.nsv, f.tmid, f.xyz_mid,
+                                        f.vel_mid);
+  const int y = aperture_centre(xyz, rng, f);
+  const int y0 = __shfl(y, 0, kFitLanes), y1 = __shfl(y, 4, kFitLanes),
+            y2 = __shfl(y, 8, kFitLanes);
+  if (sub == 0) parabola(y0, y1, y2, c);
 }
 
-__global__ void k_fit(BurstDev b, double* coef) {
-  const int line = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kWave) void k_fit(BurstDev b, double* coef) {
+  const int line = (blockIdx.x * kWave + threadIdx.x) / kFitLanes;
   if (line < b.nlines) fit_line(b, line, coef);
 }
 
-__global__ void k_batch_fit(const BurstDev* __restrict__ bursts) {
+__global__ __launch_bounds__(kWave) void k_batch_fit(const BurstDev* __restrict__ bursts) {
   const BurstDev& b = bursts[blockIdx.y];
-  const int line = blockIdx.x * blockDim.x + threadIdx.x;
+  const int line = (blockIdx.x * kWave + threadIdx.x) / kFitLanes;
   if (line < b.nlines) fit_line(b, line, const_cast<double*>(b.coef));
 }
 
@@ -2884,14 +2957,14 @@ hipError_t launch_batch(const BurstDev* d_bursts, const int2* d_items,
 
 hipError_t launch_batch_fit(const BurstDev* d_bursts, int nbursts,
                             int max_lines, hipStream_t s) {
-  dim3 grid(blocks_for(max_lines, 64), nbursts);
-  hipLaunchKernelGGL(k_batch_fit, grid, dim3(64), 0, s, d_bursts);
+  dim3 grid(blocks_for((size_t)max_lines * kFitLanes, kWave), nbursts);
+  hipLaunchKernelGGL(k_batch_fit, grid, dim3(kWave), 0, s, d_bursts);
   return hipGetLastError();
 }
 
 hipError_t launch_fit_one(const BurstDev& b, double* coef, hipStream_t s) {
-  hipLaunchKernelGGL(k_fit, dim3(blocks_for(b.nlines, 64)), dim3(64), 0, s, b,
-                     coef);
+  hipLaunchKernelGGL(k_fit, dim3(blocks_for((size_t)b.nlines * kFitLanes, kWave)), dim3(kWave), 0,
+                     s, b, coef);
   return hipGetLastError();
 }
 

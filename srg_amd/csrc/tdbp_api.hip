@@ -341,6 +341,33 @@ int run_backproject(const tdbp_geom* g, const tdbp_samples* smp,
   return st;
 }
 
+// The 80-byte headers of `nlines` device lines to (or from) host memory
+// [nlines][80]: gathered (scattered) by a kernel on the device side of one
+// contiguous copy.  A pitched hipMemcpy2DAsync moves such rows one by one:
+// 8.1 ms for 1200 lines, against 0.05 ms here.
+static int copy_headers(void* d_lines, int nlines, int stride, uint8_t* host, bool to_device,
+                        void* stream) {
+  if (!d_lines || !host || nlines < 1 || stride < 10)
+    return set_error(TDBP_ERR_ARG, "headers: bad arguments");
+  int st = current_device_ready();
+  if (st) return st;
+  hipStream_t s = (hipStream_t)stream;
+  const size_t bytes = (size_t)nlines * 80;
+  void* d = nullptr;
+  if ((st = hip_check(hipMallocAsync(&d, bytes, s), "header scratch"))) return st;
+  if (to_device) {
+    st = hip_check(hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, s), "header upload");
+    if (!st) st = hip_check(launch_headers(d_lines, nlines, stride, d, true, s), "header scatter");
+  } else {
+    st = hip_check(launch_headers(d_lines, nlines, stride, d, false, s), "header gather");
+    if (!st)
+      st = hip_check(hipMemcpyAsync(host, d, bytes, hipMemcpyDeviceToHost, s), "header download");
+  }
+  (void)hipFreeAsync(d, s);
+  const int st2 = hip_check(hipStreamSynchronize(s), "header sync");
+  return st ? st : st2;
+}
+
 }  // namespace tdbp
 
 using namespace tdbp;
@@ -437,30 +464,12 @@ int tdbp_compare(const void* d_img, const void* d_ref, size_t n, double* sums,
 }
 
 int tdbp_headers_dtoh(const void* d_lines, int nlines, int stride, uint8_t* host, void* stream) {
-  if (!d_lines || !host || nlines < 1 || stride < 10)
-    return set_error(TDBP_ERR_ARG, "headers: bad arguments");
-  int st = current_device_ready();
-  if (st) return st;
-  hipStream_t s = (hipStream_t)stream;
-  if ((st = hip_check(hipMemcpy2DAsync(host, 80, d_lines, (size_t)stride * 8, 80, (size_t)nlines,
-                                       hipMemcpyDeviceToHost, s),
-                      "header download")))
-    return st;
-  return hip_check(hipStreamSynchronize(s), "header sync");
+  return copy_headers(const_cast<void*>(d_lines), nlines, stride, host, false, stream);
 }
 
 int tdbp_headers_htod(void* d_lines, int nlines, int stride, const uint8_t* host,
                       void* stream) {
-  if (!d_lines || !host || nlines < 1 || stride < 10)
-    return set_error(TDBP_ERR_ARG, "headers: bad arguments");
-  int st = current_device_ready();
-  if (st) return st;
-  hipStream_t s = (hipStream_t)stream;
-  if ((st = hip_check(hipMemcpy2DAsync(d_lines, (size_t)stride * 8, host, 80, 80, (size_t)nlines,
-                                       hipMemcpyHostToDevice, s),
-                      "header upload")))
-    return st;
-  return hip_check(hipStreamSynchronize(s), "header sync");
+  return copy_headers(d_lines, nlines, stride, const_cast<uint8_t*>(host), true, stream);
 }
 
 int tdbp_dev_copy(void* d, const void* src, size_t n, void* s) {

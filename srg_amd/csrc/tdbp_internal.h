@@ -90,6 +90,10 @@ hipError_t launch_batch_fit(const BurstDev* d_bursts, int nbursts,
                             int max_lines, hipStream_t s);
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t s);
 hipError_t launch_copy(void* d, const void* src, size_t bytes, hipStream_t s);
+// The 80 header bytes of cf32 lines (`stride` samples apart) to or from
+// contiguous rows on the device.
+hipError_t launch_headers(void* lines, int nlines, int stride, void* rows, bool to_lines,
+                          hipStream_t s);
 int compare_blocks(size_t n);
 hipError_t launch_compare(const float2* g, const float2* o, size_t n, double* part,
                           int blocks, hipStream_t s);

@@ -2571,6 +2571,19 @@ __global__ void k_copy1(uint8_t* __restrict__ d, const uint8_t* __restrict__ s, 
     d[i] = s[i];
 }
 
+// Headers of lines `line_words` 4-byte words apart to (to_lines: from) rows of
+// 20 words.
+__global__ void k_headers(uint32_t* lines, size_t line_words, uint32_t* rows, size_t words,
+                          bool to_lines) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= words) return;
+  uint32_t* w = lines + (i / 20) * line_words + i % 20;
+  if (to_lines)
+    *w = rows[i];
+  else
+    rows[i] = *w;
+}
+
 __global__ void k_zero1(uint8_t* p, size_t n) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -3020,6 +3033,14 @@ hipError_t launch_merge(float2* grid, const float2* out, size_t n, size_t grid_o
   g = g < 16384 ? g : 16384;
   hipLaunchKernelGGL(k_merge, dim3((unsigned)g), dim3(kBlock), 0, s, grid, out, n, grid_off,
                      semantics == TDBP_SEM_CPU ? 1 : 0);
+  return hipGetLastError();
+}
+
+hipError_t launch_headers(void* lines, int nlines, int stride, void* rows, bool to_lines,
+                          hipStream_t s) {
+  const size_t words = (size_t)nlines * 20;
+  hipLaunchKernelGGL(k_headers, dim3(blocks_for(words, kBlock)), dim3(kBlock), 0, s,
+                     (uint32_t*)lines, 2 * (size_t)stride, (uint32_t*)rows, words, to_lines);
   return hipGetLastError();
 }
 

@@ -343,8 +343,14 @@ int run_backproject(const tdbp_geom* g, const tdbp_samples* smp,
 
 // The 80-byte headers of `nlines` device lines to (or from) host memory
 // [nlines][80]: gathered (scattered) by a kernel on the device side of one
-// contiguous copy.  A pitched hipMemcpy2DAsync moves such rows one by one:
-// 8.1 ms for 1200 lines, against 0.05 ms here.
+// contiguous copy, through a pinned chunk on the host side.  A pitched
+// hipMemcpy2DAsync moves such rows one by one: 7.9 ms for 1200 lines; the
+// gather with a copy into pageable memory took 0.10 ms, through the pinned
+// chunk 0.05 ms.  The chunk (320 KB, one per process, taken in turns) is kept.
+constexpr int kHeaderChunk = 4096;   // lines
+static std::mutex g_header_mu;
+static uint8_t* g_header_pin = nullptr;
+
 static int copy_headers(void* d_lines, int nlines, int stride, uint8_t* host, bool to_device,
                         void* stream) {
   if (!d_lines || !host || nlines < 1 || stride < 10)
@@ -352,20 +358,39 @@ static int copy_headers(void* d_lines, int nlines, int stride, uint8_t* host, bo
   int st = current_device_ready();
   if (st) return st;
   hipStream_t s = (hipStream_t)stream;
-  const size_t bytes = (size_t)nlines * 80;
+  std::lock_guard<std::mutex> lk(g_header_mu);
+  if (!g_header_pin &&
+      (st = hip_check(hipHostMalloc((void**)&g_header_pin, (size_t)kHeaderChunk * 80,
+                                    hipHostMallocPortable),
+                      "header staging"))) {
+    g_header_pin = nullptr;
+    return st;
+  }
   void* d = nullptr;
-  if ((st = hip_check(hipMallocAsync(&d, bytes, s), "header scratch"))) return st;
-  if (to_device) {
-    st = hip_check(hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, s), "header upload");
-    if (!st) st = hip_check(launch_headers(d_lines, nlines, stride, d, true, s), "header scatter");
-  } else {
-    st = hip_check(launch_headers(d_lines, nlines, stride, d, false, s), "header gather");
-    if (!st)
-      st = hip_check(hipMemcpyAsync(host, d, bytes, hipMemcpyDeviceToHost, s), "header download");
+  if ((st = hip_check(hipMallocAsync(&d, (size_t)std::min(nlines, kHeaderChunk) * 80, s),
+                      "header scratch")))
+    return st;
+  for (int l0 = 0; l0 < nlines && !st; l0 += kHeaderChunk) {
+    const int n = std::min(kHeaderChunk, nlines - l0);
+    const size_t bytes = (size_t)n * 80;
+    char* lines = (char*)d_lines + (size_t)l0 * (size_t)stride * 8;
+    if (to_device) {
+      std::memcpy(g_header_pin, host + (size_t)l0 * 80, bytes);
+      st = hip_check(hipMemcpyAsync(d, g_header_pin, bytes, hipMemcpyHostToDevice, s),
+                     "header upload");
+      if (!st) st = hip_check(launch_headers(lines, n, stride, d, true, s), "header scatter");
+    } else {
+      st = hip_check(launch_headers(lines, n, stride, d, false, s), "header gather");
+      if (!st)
+        st = hip_check(hipMemcpyAsync(g_header_pin, d, bytes, hipMemcpyDeviceToHost, s),
+                       "header download");
+    }
+    const int st2 = hip_check(hipStreamSynchronize(s), "header sync");
+    if (!st) st = st2;
+    if (!st && !to_device) std::memcpy(host + (size_t)l0 * 80, g_header_pin, bytes);
   }
   (void)hipFreeAsync(d, s);
-  const int st2 = hip_check(hipStreamSynchronize(s), "header sync");
-  return st ? st : st2;
+  return st;
 }
 
 }  // namespace tdbp

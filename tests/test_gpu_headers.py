@@ -1,5 +1,5 @@
 """Line headers to and from the device: every byte of every line's 80-byte
-header, the samples after it untouched; one line, many, the shortest stride."""
+header, the samples after it untouched; one line, many, more than one staging chunk (4096), the shortest stride."""
 import numpy as np
 import pytest
 
@@ -8,7 +8,7 @@ from srg_amd import tdbp as T
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nlines,stride", [(1, 10), (3, 11), (257, 40), (1201, 300)])
+@pytest.mark.parametrize("nlines,stride", [(1, 10), (3, 11), (257, 40), (1201, 300), (4097, 12)])
 def test_headers_round_trip(gpu, nlines, stride):
     rng = np.random.default_rng(nlines)
     raw = rng.integers(0, 256, (nlines, 8 * stride), dtype=np.uint8)

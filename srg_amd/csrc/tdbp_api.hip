@@ -202,10 +202,37 @@ void fill_burst(const tdbp_geom* g, BurstDev* b) {
   b->dtype = TDBP_CF32;
 }
 
-void set_tiles(BurstDev* b, int variant) {
+// Tile grid of a burst for a variant; returns the variant to launch.  own: the
+// caller asked for this variant by index; else it is the default, and where
+// variant 1 or 5 would leave most of the chip idle that is kSplitVariant.
+//
+// A wave that has a SIMD to itself issues an instruction about every 8 cycles,
+// whatever it waits for, so a burst of few tiles takes the time of one tile's
+// pulses one after another.  Split over the workgroup's four waves they take a
+// quarter, for four times the tiles and of the per-pixel set-up; that pays
+// while the 256-pixel tiles with work are at most about one per CU.  Kernel
+// times, whole and split: 51 tiles x 256 pulses 85 and 65 us (FP64 62 and 50);
+// 54 tiles x 710 pulses 130 and 88 (136 and 56); 196: 176 and 128 (169 and
+// 123); 288 x 200 pulses 62 and 75; 393: 186 and 180 (216 and 201); 785: 212
+// and 343 (298 and 340).  The rule sees the burst alone, so a batch computes
+// each of its bursts as a single launch does.
+constexpr double kSplitTiles = 256;
+int set_tiles(BurstDev* b, int variant, bool own) {
+  // Lines with a valid aperture centre span L - A pulses of the track on the
+  // ground.
+  const auto norm = [](const double* x) {
+    return std::sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
+  };
+  const double step = norm(b->vel_mid) / b->prf * kWgs84A / std::max(norm(b->xyz_mid), kWgs84A);
+  const double lines = std::min<double>(
+      b->nlines, (b->L - b->A) * step / std::max(std::fabs(b->deltalat) * 111320.0, 1e-3));
+  const double tiles = std::max(lines, 0.0) * b->W / 256.0;
+  b->split = !own && (variant == 1 || variant == 5) && !b->cpu && tiles <= kSplitTiles;
+  if (b->split) variant = kSplitVariant;
   const Variant& v = kVariants[variant];
   b->tiles_r = (b->nlines + wg_rows(v) - 1) / wg_rows(v);
   b->tiles_c = (b->W + wg_cols(v) - 1) / wg_cols(v);
+  return variant;
 }
 
 // Orbit arrays packed [t(n) | x(3n) | v(3n)] for the device.
@@ -319,8 +346,8 @@ int run_backproject(const tdbp_geom* g, const tdbp_samples* smp,
   b.satloc = d_satloc;
   b.dem = d_dem;
   b.out = (float2*)d_out;
-  if (variant < 0 || variant >= kNumVariants) variant = default_variant(precision);
-  set_tiles(&b, variant);
+  const bool asked = variant >= 0 && variant < kNumVariants;
+  variant = set_tiles(&b, asked ? variant : default_variant(precision), asked);
   if ((st = counters_for(s, &b.counters))) return st;
   double* own = nullptr;
   if (!d_coef) {
@@ -693,8 +720,7 @@ int tdbp_backproject_noalloc(const tdbp_geom* g, const tdbp_samples* smp,
   b.satloc = d_satloc;
   b.dem = d_dem;
   b.out = (float2*)d_out;
-  const int variant = default_variant(precision);
-  set_tiles(&b, variant);
+  const int variant = set_tiles(&b, default_variant(precision), false);
   const int n = g->numstatevec;
   if ((st = hip_check(hipMemcpyAsync(sc, g->timeorbit, n * sizeof(double),
                                      hipMemcpyHostToDevice, s), "orbit times")) ||

@@ -17,7 +17,7 @@ int current_device_ready();
 int cu_count();
 int validate_geom(const tdbp_geom* g);
 void fill_burst(const tdbp_geom* g, BurstDev* b);
-void set_tiles(BurstDev* b, int variant);
+int set_tiles(BurstDev* b, int variant, bool own);
 std::vector<double> pack_orbit(const tdbp_geom* g);
 void point_orbit(BurstDev* b, const double* d_orbit, int n);
 int check_samples(const tdbp_samples* s, int precision);

@@ -25,19 +25,27 @@ struct MergeTarget {
   int grid_lines = 0, firstline = 0;
 };
 
+// Work queues of one launch: the bursts of one tile kind.
+struct BatchQueue {
+  int variant = -1;
+  int2* items = nullptr;
+  int* qbase = nullptr;
+  int* counters = nullptr;
+  int grid = 0;
+};
+
 struct tdbp_batch {
   int precision = TDBP_MIXED;
   int variant = -1;
+  bool own_variant = false;   // the variant was asked for (or tuned), not the default
   int dtype = -1;
   std::vector<BurstDev> bursts;
   std::vector<MergeTarget> merges;  // per burst, applied in burst order
   std::vector<void*> owned;  // device allocations of the bursts (orbits, coefs)
   std::vector<void*> tables; // device allocations of build() (burst table, queues)
   BurstDev* d_bursts = nullptr;
-  int2* d_items = nullptr;
-  int* d_qbase = nullptr;
-  int* d_counters = nullptr;
-  int nitems = 0, grid = 0, max_lines = 0;
+  std::vector<BatchQueue> queues;   // bursts on the variant's tiles, then split ones
+  int max_lines = 0;
   int64_t pairs = 0;
   size_t dev_bytes = 0, table_bytes = 0;
   hipStream_t cap = nullptr;
@@ -77,27 +85,25 @@ void unbuild(tdbp_batch* b) {
   for (void* p : b->tables) (void)hipFree(p);
   b->tables.clear();
   b->d_bursts = nullptr;
-  b->d_items = nullptr;
-  b->d_qbase = nullptr;
-  b->d_counters = nullptr;
-  b->nitems = 0;
-  b->grid = 0;
+  b->queues.clear();
   b->dev_bytes -= b->table_bytes;
   b->table_bytes = 0;
   b->built = false;
 }
 
 int enqueue(tdbp_batch* b, hipStream_t s) {
-  int st = hip_check(launch_zero(b->d_counters, 8 * sizeof(int), s), "queue reset");
-  if (st) return st;
+  int st;
+  for (const BatchQueue& q : b->queues)
+    if ((st = hip_check(launch_zero(q.counters, 8 * sizeof(int), s), "queue reset"))) return st;
   st = hip_check(launch_batch_fit(b->d_bursts, (int)b->bursts.size(),
                                   b->max_lines, s),
                  "batch fit launch");
   if (st) return st;
-  st = hip_check(launch_batch(b->d_bursts, b->d_items, b->d_qbase, b->d_counters,
-                              b->precision, b->variant, b->dtype, b->grid, s),
-                 "batch launch");
-  if (st) return st;
+  for (const BatchQueue& q : b->queues)
+    if ((st = hip_check(launch_batch(b->d_bursts, q.items, q.qbase, q.counters, b->precision,
+                                     q.variant, b->dtype, q.grid, s),
+                        "batch launch")))
+      return st;
   // .geo merges in burst order: overlapping rows take the later burst, as the
   // reference's sequential read-modify-write does.
   for (size_t i = 0; i < b->bursts.size(); ++i) {
@@ -136,7 +142,7 @@ int build_tables(tdbp_batch* b) {
       if (!mfma_fits(bd)) b->variant = 5;
   b->max_lines = 0;
   for (auto& bd : b->bursts) {
-    set_tiles(&bd, b->variant);
+    set_tiles(&bd, b->variant, b->own_variant);
     b->max_lines = std::max(b->max_lines, bd.nlines);
   }
   const size_t nb = b->bursts.size();
@@ -170,37 +176,42 @@ int build_tables(tdbp_batch* b) {
   b->pairs = 0;
   for (int64_t v : hp) b->pairs += v;
 
-  // Work queues.
-  std::vector<std::vector<int2>> q(8);
-  int g = 0;
-  for (int bi = 0; bi < (int)nb; ++bi) {
-    const BurstDev& bd = b->bursts[bi];
-    for (int band = 0; band < bd.tiles_c; ++band, ++g) {
-      auto& dst = q[g & 7];
-      for (int rt = 0; rt < bd.tiles_r; ++rt)
-        dst.push_back(make_int2(bi, band * bd.tiles_r + rt));
+  // Work queues, one set per tile kind.
+  for (int split = 0; split < 2; ++split) {
+    std::vector<std::vector<int2>> q(8);
+    int g = 0;
+    for (int bi = 0; bi < (int)nb; ++bi) {
+      const BurstDev& bd = b->bursts[bi];
+      if (bd.split != split) continue;
+      for (int band = 0; band < bd.tiles_c; ++band, ++g) {
+        auto& dst = q[g & 7];
+        for (int rt = 0; rt < bd.tiles_r; ++rt)
+          dst.push_back(make_int2(bi, band * bd.tiles_r + rt));
+      }
     }
+    std::vector<int2> items;
+    std::vector<int> qbase(9, 0);
+    for (int k = 0; k < 8; ++k) {
+      qbase[k] = (int)items.size();
+      items.insert(items.end(), q[k].begin(), q[k].end());
+    }
+    qbase[8] = (int)items.size();
+    if (items.empty()) continue;
+    BatchQueue d;
+    d.variant = split ? kSplitVariant : b->variant;
+    if ((st = talloc(b, (void**)&d.items, items.size() * sizeof(int2))) ||
+        (st = talloc(b, (void**)&d.qbase, 9 * sizeof(int))) ||
+        (st = talloc(b, (void**)&d.counters, 8 * sizeof(int))))
+      return st;
+    if ((st = hip_check(hipMemcpy(d.items, items.data(), items.size() * sizeof(int2),
+                                  hipMemcpyHostToDevice),
+                        "item upload")) ||
+        (st = hip_check(hipMemcpy(d.qbase, qbase.data(), 9 * sizeof(int), hipMemcpyHostToDevice),
+                        "queue upload")))
+      return st;
+    d.grid = cu_count() * batch_blocks_per_cu(b->precision, d.variant, b->dtype);
+    b->queues.push_back(d);
   }
-  std::vector<int2> items;
-  std::vector<int> qbase(9, 0);
-  for (int k = 0; k < 8; ++k) {
-    qbase[k] = (int)items.size();
-    items.insert(items.end(), q[k].begin(), q[k].end());
-  }
-  qbase[8] = (int)items.size();
-  b->nitems = (int)items.size();
-  if ((st = talloc(b, (void**)&b->d_items, items.size() * sizeof(int2))) ||
-      (st = talloc(b, (void**)&b->d_qbase, 9 * sizeof(int))) ||
-      (st = talloc(b, (void**)&b->d_counters, 8 * sizeof(int))))
-    return st;
-  if ((st = hip_check(hipMemcpy(b->d_items, items.data(),
-                                items.size() * sizeof(int2), hipMemcpyHostToDevice),
-                      "item upload")) ||
-      (st = hip_check(hipMemcpy(b->d_qbase, qbase.data(), 9 * sizeof(int),
-                                hipMemcpyHostToDevice),
-                      "queue upload")))
-    return st;
-  b->grid = cu_count() * batch_blocks_per_cu(b->precision, b->variant, b->dtype);
 
   const char* eg = std::getenv("TDBP_GRAPH");
   b->use_graph = !(eg && eg[0] == '0');
@@ -239,6 +250,7 @@ tdbp_batch* tdbp_batch_create(int precision, int variant) {
   tdbp_batch* b = new tdbp_batch;
   b->precision = precision;
   b->variant = variant;
+  b->own_variant = variant >= 0;
   return b;
 }
 
@@ -347,6 +359,7 @@ int tdbp_batch_autotune(tdbp_batch* b, int reps, float* ms, int* best) {
     }
     unbuild(b);
     b->variant = v;
+    b->own_variant = true;
     if ((st = build(b))) break;
     if ((st = tdbp_batch_run(b, b->cap))) break;   // warm-up
     (void)hipEventRecord(e0, b->cap);

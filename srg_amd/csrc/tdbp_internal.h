@@ -31,6 +31,7 @@ struct BurstDev {
   int firstline, nlines, nfit, firstpix, lastpix;
   int dtype, nsv;
   int tiles_r, tiles_c;    // tile grid of this burst for the chosen variant
+  int split;               // 1: the tiles are those of kSplitVariant (set_tiles)
   int* counters;           // single-burst launches: 8 tile-queue counters on the
                            //    device, zeroed by the launcher before each launch
   int cpu;                 // 1: CPU-twin arithmetic (TDBP_SEM_CPU)
@@ -45,15 +46,22 @@ struct BurstDev {
 
 // Mixed-kernel variants: per-wave pixel tile rows (cols = 64 / rows) and
 // how the 4 waves of a workgroup are stacked.
+constexpr int kWavesSideBySide = 0, kWavesStacked = 1, kWavesSplit = 2;
 struct Variant {
   int tile_rows;     // rows of a wave tile
-  int stack_rows;    // 1: waves stacked along rows, 0: along columns
+  int stack;         // the workgroup's waves: side by side, stacked along rows,
+                     //    or all on one wave tile, each with a quarter of the
+                     //    pulses
   int mfma;          // 1: the MFMA kernel (16 waves on a 16 x 16 tile; the
                      //    tile shape is that of tile_rows 4, stacked)
   int lds;           // 1: the pulse windows of the samples staged in LDS
                      //    (kLdsPulses pulses of kLdsWindow samples at a time)
 };
 constexpr int kNumVariants = 11;
+// The tile that launches by default take instead of variants 1 and 5 (4-row
+// wave tiles) for a burst with too few pixels to fill the chip (set_tiles);
+// not a variant a caller can ask for.
+constexpr int kSplitVariant = kNumVariants;
 // LDS staging of the sample windows: pulses per sub-stage and samples per
 // pulse window (FP32 complex in LDS: 16 x 112 x 8 B = 14 KB per workgroup,
 // which with the 16 KB of pulse records leaves room for 5 workgroups in a
@@ -64,13 +72,13 @@ constexpr int kLdsWindow = 112;
 inline bool mfma_fits(const BurstDev& b) {
   return (size_t)b.L * (size_t)b.S * (b.dtype == TDBP_CF32 ? 8u : 4u) < (size_t)0xffffffffu;
 }
-extern const Variant kVariants[kNumVariants];
+extern const Variant kVariants[kNumVariants + 1];
 
 inline int wg_rows(const Variant& v) {
-  return v.stack_rows ? 4 * v.tile_rows : v.tile_rows;
+  return v.stack == kWavesStacked ? 4 * v.tile_rows : v.tile_rows;
 }
 inline int wg_cols(const Variant& v) {
-  return v.stack_rows ? kWave / v.tile_rows : 4 * (kWave / v.tile_rows);
+  return (v.stack == kWavesSideBySide ? 4 : 1) * (kWave / v.tile_rows);
 }
 
 // Launchers (tdbp_kernels.hip).  All return hipError_t of the launch.
@@ -81,6 +89,7 @@ hipError_t launch_setazoff(const BurstDev& b, double* azoff, hipStream_t s);
 hipError_t launch_pair_count(const BurstDev& b, int64_t* pairs, hipStream_t s);
 hipError_t launch_pixelint(const BurstDev& b, const double* xyz,
                            const double* azoff, hipStream_t s);
+// variant: the one set_tiles returned for the burst.
 hipError_t launch_plain(const BurstDev& b, int variant, hipStream_t s);
 hipError_t launch_mixed(const BurstDev& b, int variant, hipStream_t s);
 hipError_t launch_batch(const BurstDev* d_bursts, const int2* d_items,

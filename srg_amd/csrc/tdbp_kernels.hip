@@ -18,8 +18,8 @@
 //              once) + K (u - u_ref).d (small, FP32), hardware sin/cos on
 //              revolutions, stage-blocked FP32 sums joined by Kahan addition.
 //
-// Tile order is XCD-aware.  Single-burst launches are persistent: one
-// workgroup per resident slot; the workgroups on XCD x (blockIdx % 8 = x,
+// Tile order is XCD-aware.  Single-burst launches of more than two rounds of
+// resident workgroups are persistent: one workgroup per resident slot; the workgroups on XCD x (blockIdx % 8 = x,
 // the hardware's round-robin) take the tiles of the column bands x, x + 8,
 // ... (each band's row tiles in order) through counter x, then take what is
 // left of the other XCDs' bands -- tiles in one column band share range
@@ -40,10 +40,10 @@
 
 namespace tdbp {
 
-const Variant kVariants[kNumVariants] = {
+const Variant kVariants[kNumVariants + 1] = {
     {8, 0, 0, 0}, {4, 0, 0, 0}, {2, 0, 0, 0}, {1, 0, 0, 0}, {8, 1, 0, 0},
     {4, 1, 0, 0}, {2, 1, 0, 0}, {1, 1, 0, 0}, {4, 1, 1, 0},
-    {4, 1, 0, 1}, {8, 1, 0, 1}};
+    {4, 1, 0, 1}, {8, 1, 0, 1}, {4, kWavesSplit, 0, 0}};
 
 typedef const double __attribute__((address_space(4)))* const_dptr;
 
@@ -54,6 +54,31 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
   return x * q + (x < r ? x : r) + j;
 }
 
+// kWavesSplit: the wave's quarter of a stage's pulses [p0, p1), cut out of [*qa,
+// *qb).
+__device__ __forceinline__ void split_stage(int p0, int p1, int* qa, int* qb) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int seg = (p1 - p0 + 3) >> 2;
+  *qa = max(*qa, p0 + wave * seg);
+  *qb = min(*qb, p0 + (wave + 1) * seg);
+}
+// The four waves' sums of a pixel, added in wave order (part: 512 values of LDS
+// that the waves are done with); true on the wave that stores it.
+template <class T>
+__device__ __forceinline__ bool split_join(T* part, T* re, T* im) {
+  const int tid = threadIdx.x;
+  part[tid] = *re;
+  part[kBlock + tid] = *im;
+  __syncthreads();
+  if (tid >= kWave) return false;
+#pragma unroll
+  for (int w = 1; w < kBlock / kWave; ++w) {
+    *re += part[w * kWave + tid];
+    *im += part[kBlock + w * kWave + tid];
+  }
+  return true;
+}
+
 // The persistent tile loop of a single-burst launch: queue x holds the row
 // tiles of the column bands c = x, x + 8, ... in order (tile = c tiles_r +
 // row); a workgroup drains the queue of its XCD, then the other seven in
@@ -62,23 +87,30 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
 template <class F>
 __device__ __forceinline__ void persistent_tiles(const BurstDev& b, int* item, F&& f) {
   const int home = blockIdx.x & 7;
+  const bool queue = b.counters != nullptr;   // else a workgroup per tile
   int qi = 0;
   while (qi < 8) {
-    const int qk = (home + qi) & 7;
-    if (threadIdx.x == 0) {
-      const int bands = qk < b.tiles_c ? ((b.tiles_c - 1 - qk) >> 3) + 1 : 0;
-      const int k = atomicAdd(&b.counters[qk], 1);
-      *item = k < bands * b.tiles_r ? (qk + 8 * (k / b.tiles_r)) * b.tiles_r + k % b.tiles_r
-                                    : -1;
+    int it;
+    if (queue) {
+      const int qk = (home + qi) & 7;
+      if (threadIdx.x == 0) {
+        const int bands = qk < b.tiles_c ? ((b.tiles_c - 1 - qk) >> 3) + 1 : 0;
+        const int k = atomicAdd(&b.counters[qk], 1);
+        *item = k < bands * b.tiles_r ? (qk + 8 * (k / b.tiles_r)) * b.tiles_r + k % b.tiles_r
+                                      : -1;
+      }
+      __syncthreads();
+      it = *item;
+      __syncthreads();
+      if (it < 0) {
+        ++qi;
+        continue;
+      }
+    } else {
+      it = xcd_tile(blockIdx.x, b.tiles_r * b.tiles_c);
+      qi = 8;   // the only one
     }
-    __syncthreads();
-    const int it = *item;
-    __syncthreads();
-    if (it < 0) {
-      ++qi;
-      continue;
-    }
-    f(it);
+    f(it);   // the one call: inlined twice the kernels ran 8-17 % slower
     __syncthreads();
   }
 }
@@ -110,17 +142,30 @@ struct PixelCtx {
   int azs, aze;      // pulse window, empty if not computed
 };
 
-template <int TR, bool STACK>
+// Pixels of a workgroup: wave tiles of TR x 64/TR, the four waves side by side,
+// stacked along rows, or all on one wave tile with a quarter of the pulses
+// each (STACK = kWavesSideBySide, kWavesStacked, kWavesSplit).
+template <int TR, int STACK>
+struct TileShape {
+  static constexpr int TC = kWave / TR;
+  static constexpr int WR = STACK == kWavesStacked ? 4 * TR : TR;
+  static constexpr int WC = STACK == kWavesSideBySide ? 4 * TC : TC;
+  static __device__ __forceinline__ int row(int tid) {
+    return (STACK == kWavesStacked ? (tid >> 6) * TR : 0) + (tid & 63) / TC;
+  }
+  static __device__ __forceinline__ int col(int tid) {
+    return (STACK == kWavesSideBySide ? (tid >> 6) * TC : 0) + (tid & 63) % TC;
+  }
+};
+
+template <int TR, int STACK>
 __device__ __forceinline__ PixelCtx pixel_of(const BurstDev& b, int tile) {
-  constexpr int TC = kWave / TR;
-  constexpr int WR = STACK ? 4 * TR : TR;
-  constexpr int WC = STACK ? TC : 4 * TC;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  using G = TileShape<TR, STACK>;
   const int band = tile / b.tiles_r;
   const int rt = tile - band * b.tiles_r;
   PixelCtx p;
-  p.row = rt * WR + (STACK ? wave * TR : 0) + lane / TC;
-  p.col = band * WC + (STACK ? 0 : wave * TC) + lane % TC;
+  p.row = rt * G::WR + G::row(threadIdx.x);
+  p.col = band * G::WC + G::col(threadIdx.x);
   p.inwin = p.row < b.nlines && p.col < b.W;
   p.azs = 0;
   p.aze = 0;
@@ -242,7 +287,7 @@ __device__ __forceinline__ void cpu_pair(const float2* __restrict__ row,
 }
 
 // The CPU twin's tile: every pair by cpu_pair.
-template <int TR, bool STACK>
+template <int TR, int STACK>
 __device__ __forceinline__ void cpu_tile(const BurstDev& b, int tile) {
   PixelCtx p = pixel_of<TR, STACK>(b, tile);
   double x[3] = {0., 0., 0.};
@@ -465,22 +510,33 @@ struct MixedPixel {
 // floor(rho).  The row pointer of a pulse carries (i0s + ia_min) * elem,
 // the lane (ia - ia_min) * elem; the phase fa dmrg 2/lambda that P adds is
 // taken out once per pixel at the end.
+//
+// SD: the quadratic is sd alone and the offset fa is added to the index, one
+// instruction more; the phase then takes no cycles of fa dmrg (up to 21, whose
+// FP32 rounding is most of the quadratic form's error).  The split tiles, which
+// are not short of issue slots, take this form.
 struct PolyPixel {
   float c0, c1, c2;
   unsigned iaoff;    // (ia - ia_min) * elem
+  float fa;          // SD: aref/dmrg - ia
 };
+template <bool SD>
+__device__ __forceinline__ float poly_rho(const PolyPixel& pp, float P, float invd, float f0s) {
+  const float rho = fmaf(P, invd, f0s);
+  return SD ? rho + pp.fa : rho;
+}
 
 // One pair on the quadratic.  rows: row start shifted by (i0s + ia_min) *
 // elem (unchecked pairs); rowq: the row start (checked pairs, which address
 // by the sample index i0s + ia + floor(rho) = ibase + floor(rho)).  lim:
 // rho <= lim <=> r <= r_hi.
-template <int DT, bool CHECK>
+template <int DT, bool CHECK, bool SD>
 __device__ __forceinline__ void poly_pair(const PolyPixel& pp, const float4& r3, float sc,
                                           grow_t rowq, grow_t rows, float Kf, float invd,
                                           bool inwin, int ibase, unsigned smax, float lim,
                                           float& sr, float& si) {
   const float P = fmaf(fmaf(pp.c2, r3.x, pp.c1), r3.x, pp.c0);
-  const float rho = fmaf(P, invd, r3.y);
+  const float rho = poly_rho<SD>(pp, P, invd, r3.y);
   int il;
   asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(il) : "v"(rho));
   float2 c;
@@ -551,7 +607,7 @@ struct PairFront {
 };
 // POLY: the sample pair comes through the structured buffer `rsrc` at
 // scalar offset `soff` (row start + (i0s + ia_min) * elem + kSbufBias).
-template <int DT, bool POLY>
+template <int DT, bool POLY, bool SD>
 __device__ __forceinline__ PairFront<DT, POLY> mixed_front(const MixedPixel& m,
                                                            const PolyPixel& pp,
                                                            const PulseRec& r, grow_t rowb,
@@ -560,7 +616,7 @@ __device__ __forceinline__ PairFront<DT, POLY> mixed_front(const MixedPixel& m,
   PairFront<DT, POLY> f;
   if constexpr (POLY) {
     const float P = fmaf(fmaf(pp.c2, r.r3.x, pp.c1), r.r3.x, pp.c0);
-    const float rho = fmaf(P, invd, r.r3.y);
+    const float rho = poly_rho<SD>(pp, P, invd, r.r3.y);
     int il;
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(il) : "v"(rho));
     // Measured on the 27-burst IW scene: 1.5% above the same loop with a
@@ -615,7 +671,7 @@ __device__ __forceinline__ void mixed_back(const PairFront<DT, POLY>& f, float& 
 
 // The test-free core [qq, cb) of a stage on the quadratic form.  U: the
 // stage's pulses share one scale, which the caller applies to the stage sum.
-template <int DT, bool U>
+template <int DT, bool U, bool SD>
 __device__ __forceinline__ void poly_core(const MixedPixel& m, const PolyPixel& pp,
                                           const PulseRec* rec, int p0,
                                           int qq, int cb, grow_t base, const I32x4& rsrc,
@@ -629,7 +685,7 @@ __device__ __forceinline__ void poly_core(const MixedPixel& m, const PolyPixel& 
     if (qq < cb && ((cb - qq) & 1)) {
       const grow_t rowq = base + (size_t)qq * rowbytes;
       const float4 r3 = rec[qq - p0].r3;
-      poly_pair<DT, false>(pp, r3, U ? 1.f : r3.w, rowq, rowq + shift, Kf, invd, true, ibase,
+      poly_pair<DT, false, SD>(pp, r3, U ? 1.f : r3.w, rowq, rowq + shift, Kf, invd, true, ibase,
                            smax, lim, sr, si);
       ++qq;
     }
@@ -638,19 +694,19 @@ __device__ __forceinline__ void poly_core(const MixedPixel& m, const PolyPixel& 
       unsigned so = (unsigned)((long)qq * (long)rowbytes + shift + kSbufBias);
       const unsigned rb32 = (unsigned)rowbytes;
       const PulseRec* rr = rec + (qq - p0);
-      PairFront<DT, true> fa = mixed_front<DT, true>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
+      PairFront<DT, true> fa = mixed_front<DT, true, SD>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
       PairFront<DT, true> fb;
       for (; qq + 2 < cb; qq += 2) {
-        fb = mixed_front<DT, true>(m, pp, rr[1], rp, rsrc, so + rb32, Kf, invd);
+        fb = mixed_front<DT, true, SD>(m, pp, rr[1], rp, rsrc, so + rb32, Kf, invd);
         __builtin_amdgcn_sched_barrier(0);
         mixed_back<DT, U, true>(fa, sr, si);
         so += 2 * rb32;
         rr += 2;
-        fa = mixed_front<DT, true>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
+        fa = mixed_front<DT, true, SD>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
         __builtin_amdgcn_sched_barrier(0);
         mixed_back<DT, U, true>(fb, sr, si);
       }
-      fb = mixed_front<DT, true>(m, pp, rr[1], rp, rsrc, so + rb32, Kf, invd);
+      fb = mixed_front<DT, true, SD>(m, pp, rr[1], rp, rsrc, so + rb32, Kf, invd);
       mixed_back<DT, U, true>(fa, sr, si);
       mixed_back<DT, U, true>(fb, sr, si);
     }
@@ -666,7 +722,7 @@ __device__ __forceinline__ void poly_core(const MixedPixel& m, const PolyPixel& 
   for (int r = 0; r < rem; ++r, ++qq) {
     const grow_t rowq = base + (size_t)qq * rowbytes;
     const float4 r3 = rec[qq - p0].r3;
-    poly_pair<DT, false>(pp, r3, U ? 1.f : r3.w, rowq, rowq + shift, Kf, invd, true, ibase,
+    poly_pair<DT, false, SD>(pp, r3, U ? 1.f : r3.w, rowq, rowq + shift, Kf, invd, true, ibase,
                          smax, lim, sr, si);
   }
   if (qq < cb) {
@@ -674,23 +730,23 @@ __device__ __forceinline__ void poly_core(const MixedPixel& m, const PolyPixel& 
     unsigned so = (unsigned)((long)qq * (long)rowbytes + shift + kSbufBias);
     const unsigned rb32 = (unsigned)rowbytes;
     const PulseRec* rr = rec + (qq - p0);
-    PairFront<DT, true> fa = mixed_front<DT, true>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
-    PairFront<DT, true> fb = mixed_front<DT, true>(m, pp, rr[1], rp, rsrc, so + rb32, Kf, invd);
+    PairFront<DT, true> fa = mixed_front<DT, true, SD>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
+    PairFront<DT, true> fb = mixed_front<DT, true, SD>(m, pp, rr[1], rp, rsrc, so + rb32, Kf, invd);
     PairFront<DT, true> fc;
     for (; qq + 3 < cb; qq += 3) {
-      fc = mixed_front<DT, true>(m, pp, rr[2], rp, rsrc, so + 2 * rb32, Kf, invd);
+      fc = mixed_front<DT, true, SD>(m, pp, rr[2], rp, rsrc, so + 2 * rb32, Kf, invd);
       __builtin_amdgcn_sched_barrier(0);
       mixed_back<DT, U, true>(fa, sr, si);
-      fa = mixed_front<DT, true>(m, pp, rr[3], rp, rsrc, so + 3 * rb32, Kf, invd);
+      fa = mixed_front<DT, true, SD>(m, pp, rr[3], rp, rsrc, so + 3 * rb32, Kf, invd);
       __builtin_amdgcn_sched_barrier(0);
       mixed_back<DT, U, true>(fb, sr, si);
-      fb = mixed_front<DT, true>(m, pp, rr[4], rp, rsrc, so + 4 * rb32, Kf, invd);
+      fb = mixed_front<DT, true, SD>(m, pp, rr[4], rp, rsrc, so + 4 * rb32, Kf, invd);
       __builtin_amdgcn_sched_barrier(0);
       mixed_back<DT, U, true>(fc, sr, si);
       so += 3 * rb32;
       rr += 3;
     }
-    fc = mixed_front<DT, true>(m, pp, rr[2], rp, rsrc, so + 2 * rb32, Kf, invd);
+    fc = mixed_front<DT, true, SD>(m, pp, rr[2], rp, rsrc, so + 2 * rb32, Kf, invd);
     mixed_back<DT, U, true>(fa, sr, si);
     mixed_back<DT, U, true>(fb, sr, si);
     mixed_back<DT, U, true>(fc, sr, si);
@@ -702,7 +758,7 @@ __device__ __forceinline__ void poly_core(const MixedPixel& m, const PolyPixel& 
 // stage_safe: every pulse of the stage keeps the whole tile inside the gate.
 // POLY: the quadratic (shift = (i0s + ia_min) * elem, ibase = i0s + ia, lim
 // = r_hi - i0s - ia); else the FP32 chain.
-template <int DT, bool POLY>
+template <int DT, bool POLY, bool SD>
 __device__ __forceinline__ void stage_pulses(const MixedPixel& m, const PolyPixel& pp,
                                              const PulseRec* rec, int p0, int qa, int qb,
                                              int qc0, int qc1, bool stage_safe, bool uni,
@@ -716,7 +772,7 @@ __device__ __forceinline__ void stage_pulses(const MixedPixel& m, const PolyPixe
   auto checked = [&](int qq) {
     const grow_t rowq = base + (size_t)qq * rowbytes;
     if constexpr (POLY)
-      poly_pair<DT, true>(pp, rec[qq - p0].r3, uni ? 1.f : rec[qq - p0].r3.w, rowq, rowq, Kf,
+      poly_pair<DT, true, SD>(pp, rec[qq - p0].r3, uni ? 1.f : rec[qq - p0].r3.w, rowq, rowq, Kf,
                           invd, (unsigned)(qq - azs) < n,
                           ibase, smax, lim, sr, si);
     else
@@ -726,7 +782,7 @@ __device__ __forceinline__ void stage_pulses(const MixedPixel& m, const PolyPixe
   auto unchecked = [&](int qq) {
     const grow_t rowq = base + (size_t)qq * rowbytes;
     if constexpr (POLY)
-      poly_pair<DT, false>(pp, rec[qq - p0].r3, uni ? 1.f : rec[qq - p0].r3.w, rowq,
+      poly_pair<DT, false, SD>(pp, rec[qq - p0].r3, uni ? 1.f : rec[qq - p0].r3.w, rowq,
                            rowq + shift, Kf, invd, true, ibase,
                            smax, lim, sr, si);
     else
@@ -740,10 +796,10 @@ __device__ __forceinline__ void stage_pulses(const MixedPixel& m, const PolyPixe
     int qq = ca;
     if constexpr (POLY) {
       if (uni)
-        poly_core<DT, true>(m, pp, rec, p0, qq, cb, base, rsrc, rowbytes, shift, ibase, Kf, invd,
+        poly_core<DT, true, SD>(m, pp, rec, p0, qq, cb, base, rsrc, rowbytes, shift, ibase, Kf, invd,
                             smax, lim, sr, si);
       else
-        poly_core<DT, false>(m, pp, rec, p0, qq, cb, base, rsrc, rowbytes, shift, ibase, Kf, invd,
+        poly_core<DT, false, SD>(m, pp, rec, p0, qq, cb, base, rsrc, rowbytes, shift, ibase, Kf, invd,
                              smax, lim, sr, si);
     } else {
       // FP32 chain: two pairs in flight; an odd count starts with one plain
@@ -758,20 +814,20 @@ __device__ __forceinline__ void stage_pulses(const MixedPixel& m, const PolyPixe
         unsigned so = (unsigned)((long)qq * (long)rowbytes + shift + kSbufBias);
         const unsigned rb32 = (unsigned)rowbytes;
         const PulseRec* rr = rec + (qq - p0);
-        PairFront<DT, POLY> fa = mixed_front<DT, POLY>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
+        PairFront<DT, POLY> fa = mixed_front<DT, POLY, SD>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
         PairFront<DT, POLY> fb;
         for (; qq + 2 < cb; qq += 2) {
-          fb = mixed_front<DT, POLY>(m, pp, rr[1], rp + rowbytes, rsrc, so + rb32, Kf, invd);
+          fb = mixed_front<DT, POLY, SD>(m, pp, rr[1], rp + rowbytes, rsrc, so + rb32, Kf, invd);
           __builtin_amdgcn_sched_barrier(0);
           mixed_back<DT, false, POLY>(fa, sr, si);
           rp += 2 * rowbytes;
           so += 2 * rb32;
           rr += 2;
-          fa = mixed_front<DT, POLY>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
+          fa = mixed_front<DT, POLY, SD>(m, pp, rr[0], rp, rsrc, so, Kf, invd);
           __builtin_amdgcn_sched_barrier(0);
           mixed_back<DT, false, POLY>(fb, sr, si);
         }
-        fb = mixed_front<DT, POLY>(m, pp, rr[1], rp + rowbytes, rsrc, so + rb32, Kf, invd);
+        fb = mixed_front<DT, POLY, SD>(m, pp, rr[1], rp + rowbytes, rsrc, so + rb32, Kf, invd);
         mixed_back<DT, false, POLY>(fa, sr, si);
         mixed_back<DT, false, POLY>(fb, sr, si);
       }
@@ -1185,7 +1241,7 @@ __device__ __forceinline__ void plain_block(const double* c, double dt, int wlo,
   ai = fma(s.ai, zr, ai);
 }
 
-template <int TR, bool STACK>
+template <int TR, int STACK>
 __device__ __forceinline__ void plain_excess_tile(const BurstDev& b, int tile, PlainRec* rec,
                                                   PlainShared* sh) {
   PixelCtx p = pixel_of<TR, STACK>(b, tile);
@@ -1195,11 +1251,8 @@ __device__ __forceinline__ void plain_excess_tile(const BurstDev& b, int tile, P
   if (live) pixel_ecef(b, p.row, p.col, x);
 
   // Tile window and reference pixel (the live one nearest the centre).
-  constexpr int TC = kWave / TR;
-  constexpr int WR = STACK ? 4 * TR : TR, WC = STACK ? TC : 4 * TC;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wr = (STACK ? wave * TR : 0) + lane / TC;
-  const int wc = (STACK ? 0 : wave * TC) + lane % TC;
+  constexpr int WR = TileShape<TR, STACK>::WR, WC = TileShape<TR, STACK>::WC;
+  const int wr = TileShape<TR, STACK>::row(tid), wc = TileShape<TR, STACK>::col(tid);
   if (tid == 0) {
     sh->key = 0x7fffffff;
     sh->wlo = 0x7fffffff;
@@ -1361,7 +1414,8 @@ __device__ __forceinline__ void plain_excess_tile(const BurstDev& b, int tile, P
     if (tid == 0) rec[p1 - p0] = PlainRec{-1e9, 0., 0., 0.};
     const int stage_safe = __syncthreads_and(safe ? 1 : 0);
     if (wave_live) {
-      const int qa = max(p0, qlo), qb = min(p1, qhi);
+      int qa = max(p0, qlo), qb = min(p1, qhi);
+      if constexpr (STACK == kWavesSplit) split_stage(p0, p1, &qa, &qb);
       if (wave_fit && stage_safe) {
         for (int q = qa; q < qb;) {
           const int ce = min(qb, qc1);
@@ -1382,13 +1436,17 @@ __device__ __forceinline__ void plain_excess_tile(const BurstDev& b, int tile, P
     }
     __syncthreads();
   }
+  if constexpr (STACK == kWavesSplit) {
+    if (!split_join((double*)rec, &ar, &ai)) return;
+  }
   store_out(b, p, (float)ar, (float)ai);
 }
 
-template <int TR, bool STACK, int DT, bool LDS = false>
+template <int TR, int STACK, int DT, bool LDS = false>
 __device__ __forceinline__ void mixed_tile(const BurstDev& b, int tile,
                                            PulseRec* rec, TileShared* sh,
                                            F32x4* sbuf = nullptr) {
+  constexpr bool SD = STACK == kWavesSplit;   // PolyPixel
   PixelCtx p = pixel_of<TR, STACK>(b, tile);
   const int tid = threadIdx.x;
   const bool live = p.aze > p.azs;
@@ -1397,11 +1455,8 @@ __device__ __forceinline__ void mixed_tile(const BurstDev& b, int tile,
 
   // Workgroup window and reference pixel (the live pixel nearest the tile
   // centre, ties to the lowest thread).
-  constexpr int TC = kWave / TR;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wr = (STACK ? wave * TR : 0) + lane / TC;
-  const int wc = (STACK ? 0 : wave * TC) + lane % TC;
-  constexpr int WR = STACK ? 4 * TR : TR, WC = STACK ? TC : 4 * TC;
+  constexpr int WR = TileShape<TR, STACK>::WR, WC = TileShape<TR, STACK>::WC;
+  const int wr = TileShape<TR, STACK>::row(tid), wc = TileShape<TR, STACK>::col(tid);
   const int key = (abs(2 * wr - WR) + abs(2 * wc - WC)) * 256 + tid;
   if (tid == 0) {
     sh->key = 0x7fffffff;
@@ -1479,7 +1534,7 @@ __device__ __forceinline__ void mixed_tile(const BurstDev& b, int tile,
   const int ia = (int)rint(arefd64);
   const double fad = aref64 - ia * b.dmrg;          // fa dmrg, |fa| <= 1/2
   const int ia_min = wave_min(ia);
-  PolyPixel pp = {0.f, 0.f, 0.f, (unsigned)(ia - ia_min) * (unsigned)elem_bytes<DT>()};
+  PolyPixel pp = {0.f, 0.f, 0.f, (unsigned)(ia - ia_min) * (unsigned)elem_bytes<DT>(), 0.f};
   bool wave_poly = false;
   if (wave_live && qhi - qlo >= 16 && !b.chain) {
     const double mid = 0.5 * (qlo + qhi - 1), hh = 0.5 * (qhi - 1 - qlo);
@@ -1524,7 +1579,8 @@ __device__ __forceinline__ void mixed_tile(const BurstDev& b, int tile,
                     (size_t)b.L * rowbytes + (size_t)kSbufBias < (size_t)0x7fffffff;
     wave_poly = wave_min(ok ? 1 : 0) == 1;
     if (wave_poly && live) atomicMax(&sh->pmax, __float_as_uint((float)(pm * (1.0 + 1e-6))));
-    pp.c0 = (float)(c0 + fad);
+    pp.c0 = (float)(SD ? c0 : c0 + fad);
+    pp.fa = (float)(arefd64 - ia);
     pp.c1 = (float)c1;
     pp.c2 = (float)c2;
   }
@@ -1543,7 +1599,7 @@ __device__ __forceinline__ void mixed_tile(const BurstDev& b, int tile,
   }
   // Phase taken out at the end: frac(2/lambda aref), less Kf fa dmrg on the
   // quadratic, whose cycles Kf P carry it.
-  const double cp64 = aref64 * b.two_over_wvl - (wave_poly ? (double)Kf * fad : 0.0);
+  const double cp64 = aref64 * b.two_over_wvl - (wave_poly && !SD ? (double)Kf * fad : 0.0);
   const float cpix = (float)(cp64 - rint(cp64));
   if constexpr (LDS) {
     atomicMin(&sh->iamin, ia);
@@ -1650,14 +1706,15 @@ __device__ __forceinline__ void mixed_tile(const BurstDev& b, int tile,
     } else if (wave_live) {
       // A wave without a live pixel skips the pulse loops (its window bounds
       // are sentinels and must not enter index arithmetic).
-      const int qa = max(p0, qlo), qb = min(p0 + kStage, qhi);
+      int qa = max(p0, qlo), qb = min(p0 + kStage, qhi);
+      if constexpr (STACK == kWavesSplit) split_stage(p0, min(p0 + kStage, whi), &qa, &qb);
       if (wave_poly)
-        stage_pulses<DT, true>(m, pp, rec, p0, qa, qb, qc0, qc1, stage_safe != 0, stage_uni,
+        stage_pulses<DT, true, SD>(m, pp, rec, p0, qa, qb, qc0, qc1, stage_safe != 0, stage_uni,
                                base, rsrc,
                                rowbytes, (long)(i0s + ia_min) * elem_bytes<DT>(), i0s + ia,
                                (float)(b.r_hi - i0s - ia), Kf, invd, p.azs, n, smax, sr, si);
       else
-        stage_pulses<DT, false>(m, pp, rec, p0, qa, qb, qc0, qc1, stage_safe != 0, false,
+        stage_pulses<DT, false, SD>(m, pp, rec, p0, qa, qb, qc0, qc1, stage_safe != 0, false,
                                 base, rsrc,
                                 rowbytes, 0, 0, 0.f, Kf, invd, p.azs, n, smax, sr, si);
     }
@@ -1681,7 +1738,10 @@ __device__ __forceinline__ void mixed_tile(const BurstDev& b, int tile,
   // pulses: apply it once.
   float ps, pcs;
   sincospif(2.0f * cpix, &ps, &pcs);
-  const float fr_ = acc_r - cmp_r, fi_ = acc_i - cmp_i;
+  float fr_ = acc_r - cmp_r, fi_ = acc_i - cmp_i;
+  if constexpr (STACK == kWavesSplit) {
+    if (!split_join((float*)rec, &fr_, &fi_)) return;
+  }
   store_out(b, p, fr_ * pcs - fi_ * ps, fr_ * ps + fi_ * pcs);
 }
 
@@ -1845,7 +1905,7 @@ __device__ __forceinline__ void mfma_tile(const BurstDev& b, int tile, MShared& 
   double x[3] = {0., 0., 0.};
   bool live = false;
   if (owner) {
-    p = pixel_of<4, true>(b, tile);   // 16 x 16 tile: row tid/16, column tid%16
+    p = pixel_of<4, kWavesStacked>(b, tile);   // 16 x 16 tile: row tid/16, column tid%16
     live = p.aze > p.azs;
     if (live) pixel_ecef(b, p.row, p.col, x);
   }
@@ -2141,7 +2201,7 @@ __device__ __forceinline__ void mfma_tile(const BurstDev& b, int tile, MShared& 
 // 3.2 at 4 with spills outside the loops, 3.9 at 5).
 #define TDBP_PLAIN_OCC __attribute__((amdgpu_waves_per_eu(3)))
 
-template <int TR, bool STACK, bool CPU>
+template <int TR, int STACK, bool CPU>
 __global__ __launch_bounds__(kBlock) TDBP_PLAIN_OCC void k_plain(BurstDev b) {
   __shared__ int item;
   if constexpr (CPU) {
@@ -2163,7 +2223,7 @@ __global__ __launch_bounds__(kBlock) TDBP_PLAIN_OCC void k_plain(BurstDev b) {
 // 160 KB, and 5 waves give each 96 VGPRs.
 #define TDBP_LDS_OCC __attribute__((amdgpu_waves_per_eu(5)))
 
-template <int TR, bool STACK, int DT>
+template <int TR, int STACK, int DT>
 __global__ __launch_bounds__(kBlock) TDBP_MIXED_OCC void k_mixed(BurstDev b) {
   __shared__ PulseRec rec[kStage];
   __shared__ TileShared sh;
@@ -2171,7 +2231,7 @@ __global__ __launch_bounds__(kBlock) TDBP_MIXED_OCC void k_mixed(BurstDev b) {
   persistent_tiles(b, &item, [&](int tile) { mixed_tile<TR, STACK, DT>(b, tile, rec, &sh); });
 }
 
-template <int TR, bool STACK, int DT>
+template <int TR, int STACK, int DT>
 __global__ __launch_bounds__(kBlock) TDBP_LDS_OCC void k_mixed_lds(BurstDev b) {
   __shared__ PulseRec rec[kStage];
   __shared__ TileShared sh;
@@ -2219,7 +2279,7 @@ __global__ __launch_bounds__(kMBlock) TDBP_MIXED_OCC void k_batch_mfma(
 
 // Persistent batch kernel: workgroup on XCD x = blockIdx % 8 drains queue x,
 // then steals from the others.  Queue k holds items [qbase[k], qbase[k+1]).
-template <int PREC, int TR, bool STACK, int DT, bool LDS = false, class REC, class SHARED>
+template <int PREC, int TR, int STACK, int DT, bool LDS = false, class REC, class SHARED>
 __device__ __forceinline__ void batch_body(const BurstDev* __restrict__ bursts,
                                            const int2* __restrict__ items,
                                            const int* __restrict__ qbase,
@@ -2254,7 +2314,7 @@ __device__ __forceinline__ void batch_body(const BurstDev* __restrict__ bursts,
   }
 }
 
-template <int TR, bool STACK, int DT>
+template <int TR, int STACK, int DT>
 __global__ __launch_bounds__(kBlock) TDBP_MIXED_OCC void k_batch_mixed(
     const BurstDev* __restrict__ bursts, const int2* __restrict__ items,
     const int* __restrict__ qbase, int* counters) {
@@ -2264,7 +2324,7 @@ __global__ __launch_bounds__(kBlock) TDBP_MIXED_OCC void k_batch_mixed(
   batch_body<TDBP_MIXED, TR, STACK, DT>(bursts, items, qbase, counters, rec, &sh, &item_s);
 }
 
-template <int TR, bool STACK, int DT>
+template <int TR, int STACK, int DT>
 __global__ __launch_bounds__(kBlock) TDBP_LDS_OCC void k_batch_mixed_lds(
     const BurstDev* __restrict__ bursts, const int2* __restrict__ items,
     const int* __restrict__ qbase, int* counters) {
@@ -2276,7 +2336,7 @@ __global__ __launch_bounds__(kBlock) TDBP_LDS_OCC void k_batch_mixed_lds(
                                               &item_s, sbuf);
 }
 
-template <int TR, bool STACK>
+template <int TR, int STACK>
 __global__ __launch_bounds__(kBlock) TDBP_PLAIN_OCC void k_batch_plain(
     const BurstDev* __restrict__ bursts, const int2* __restrict__ items,
     const int* __restrict__ qbase, int* counters) {
@@ -2773,9 +2833,14 @@ inline unsigned blocks_for(size_t n, int bs) {
   return (unsigned)((n + bs - 1) / bs);
 }
 
-// Grid of a persistent single-burst launch: the resident workgroups of
-// `kernel` on every CU, at most one per tile.  The launch zeroes the burst's
-// tile-queue counters first (a fill kernel on the same stream).
+// Launch of a burst's tiles.  Up to two rounds of resident workgroups: one
+// workgroup per tile, no queue (b.counters null).  Beyond: persistent, the
+// resident workgroups of `kernel` on every CU, the tile-queue counters zeroed
+// first (a fill kernel on the same stream).  The queue keeps a band's tiles on
+// their XCD and evens out the end, but its counters cost a burst of few tiles
+// more than they give: 1400 x 12000 samples onto 400 x 800 pixels 0.31 -> 0.25
+// ms, 800 x 800 (1.2 rounds) 0.66 -> 0.52 ms, 600 x 1600 (1.9) 0.69 -> 0.67
+// ms without it; FP64 on 800 x 800 (3.4 rounds) 0.56 with, 0.64 without.
 template <void (*K)(BurstDev)>
 hipError_t persistent_launch(const BurstDev& b, hipStream_t s) {
   if (!b.counters) return hipErrorInvalidValue;
@@ -2785,27 +2850,33 @@ hipError_t persistent_launch(const BurstDev& b, hipStream_t s) {
        occ <= 0))
     occ = 1;
   const long nb = (long)b.tiles_r * b.tiles_c;
-  const long grid = std::min(nb, (long)cu_count() * occ);
-  if (grid <= 0) return hipSuccess;
+  const long room = (long)cu_count() * occ;
+  if (nb <= 0) return hipSuccess;
+  if (nb <= 2 * room) {
+    BurstDev d = b;
+    d.counters = nullptr;
+    hipLaunchKernelGGL(K, dim3((unsigned)nb), dim3(kBlock), 0, s, d);
+    return hipGetLastError();
+  }
   const hipError_t e = launch_zero(b.counters, 8 * sizeof(int), s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(K, dim3((unsigned)grid), dim3(kBlock), 0, s, b);
+  hipLaunchKernelGGL(K, dim3((unsigned)std::min(nb, room)), dim3(kBlock), 0, s, b);
   return hipGetLastError();
 }
 
-template <int TR, bool STACK>
+template <int TR, int STACK>
 hipError_t plain_launch(const BurstDev& b, hipStream_t s) {
   if (b.cpu) return persistent_launch<k_plain<TR, STACK, true>>(b, s);
   return persistent_launch<k_plain<TR, STACK, false>>(b, s);
 }
 
-template <int TR, bool STACK, int DT, bool LDS>
+template <int TR, int STACK, int DT, bool LDS>
 hipError_t mixed_launch(const BurstDev& b, hipStream_t s) {
   if constexpr (LDS) return persistent_launch<k_mixed_lds<TR, STACK, DT>>(b, s);
   else return persistent_launch<k_mixed<TR, STACK, DT>>(b, s);
 }
 
-template <int TR, bool STACK, bool LDS = false>
+template <int TR, int STACK, bool LDS = false>
 hipError_t mixed_dt(const BurstDev& b, hipStream_t s) {
   switch (b.dtype) {
     case TDBP_CF32: return mixed_launch<TR, STACK, TDBP_CF32, LDS>(b, s);
@@ -2815,7 +2886,7 @@ hipError_t mixed_dt(const BurstDev& b, hipStream_t s) {
   }
 }
 
-template <int PREC, int TR, bool STACK, int DT, bool LDS>
+template <int PREC, int TR, int STACK, int DT, bool LDS>
 hipError_t batch_launch(const BurstDev* d, const int2* it, const int* qb,
                         int* ctr, int grid, hipStream_t s) {
   if constexpr (PREC == TDBP_MIXED && LDS)
@@ -2830,7 +2901,7 @@ hipError_t batch_launch(const BurstDev* d, const int2* it, const int* qb,
   return hipGetLastError();
 }
 
-template <int PREC, int TR, bool STACK, int DT, bool LDS>
+template <int PREC, int TR, int STACK, int DT, bool LDS>
 int occupancy() {
   int n = 0;
   hipError_t e;
@@ -2850,7 +2921,7 @@ int occupancy() {
 // Dispatch (precision, variant, dtype) to a template instance.  Variants
 // 9 and 10 are the LDS-staged kernels on the tiles of variants 5 and 4 (the
 // FP64 kernel has no staged form and runs those tiles unstaged).
-template <template <int, int, bool, int, bool> class F, typename... Args>
+template <template <int, int, int, int, bool> class F, typename... Args>
 auto dispatch(int prec, int variant, int dt, Args... args) {
 #define TDBP_V(TR, ST, LDS)                                                     \
   if (prec == TDBP_PLAIN_FP64) return F<TDBP_PLAIN_FP64, TR, ST, TDBP_CF32, false>::run(args...); \
@@ -2859,28 +2930,29 @@ auto dispatch(int prec, int variant, int dt, Args... args) {
   if (dt == TDBP_CI16) return F<TDBP_MIXED, TR, ST, TDBP_CI16, LDS>::run(args...); \
   return F<TDBP_MIXED, TR, ST, TDBP_CBF16, LDS>::run(args...);
   switch (variant) {
-    case 0: { TDBP_V(8, false, false) }
-    case 1: { TDBP_V(4, false, false) }
-    case 2: { TDBP_V(2, false, false) }
-    case 3: { TDBP_V(1, false, false) }
-    case 4: { TDBP_V(8, true, false) }
-    case 5: { TDBP_V(4, true, false) }
-    case 6: { TDBP_V(2, true, false) }
-    case 9: { TDBP_V(4, true, true) }
-    case 10: { TDBP_V(8, true, true) }
-    default: { TDBP_V(1, true, false) }
+    case 0: { TDBP_V(8, kWavesSideBySide, false) }
+    case 1: { TDBP_V(4, kWavesSideBySide, false) }
+    case 2: { TDBP_V(2, kWavesSideBySide, false) }
+    case 3: { TDBP_V(1, kWavesSideBySide, false) }
+    case 4: { TDBP_V(8, kWavesStacked, false) }
+    case 5: { TDBP_V(4, kWavesStacked, false) }
+    case 6: { TDBP_V(2, kWavesStacked, false) }
+    case kSplitVariant: { TDBP_V(4, kWavesSplit, false) }
+    case 9: { TDBP_V(4, kWavesStacked, true) }
+    case 10: { TDBP_V(8, kWavesStacked, true) }
+    default: { TDBP_V(1, kWavesStacked, false) }
   }
 #undef TDBP_V
 }
 
-template <int PREC, int TR, bool STACK, int DT, bool LDS>
+template <int PREC, int TR, int STACK, int DT, bool LDS>
 struct BatchRun {
   static hipError_t run(const BurstDev* d, const int2* it, const int* qb,
                         int* ctr, int grid, hipStream_t s) {
     return batch_launch<PREC, TR, STACK, DT, LDS>(d, it, qb, ctr, grid, s);
   }
 };
-template <int PREC, int TR, bool STACK, int DT, bool LDS>
+template <int PREC, int TR, int STACK, int DT, bool LDS>
 struct OccRun {
   static int run() { return occupancy<PREC, TR, STACK, DT, LDS>(); }
 };
@@ -2888,17 +2960,18 @@ struct OccRun {
 
 hipError_t launch_plain(const BurstDev& b, int variant, hipStream_t s) {
   switch (variant) {
-    case 8: return plain_launch<4, true>(b, s);   // same tile as the MFMA variant
-    case 9: return plain_launch<4, true>(b, s);   // tiles of the LDS-staged variants
-    case 10: return plain_launch<8, true>(b, s);
-    case 0: return plain_launch<8, false>(b, s);
-    case 1: return plain_launch<4, false>(b, s);
-    case 2: return plain_launch<2, false>(b, s);
-    case 3: return plain_launch<1, false>(b, s);
-    case 4: return plain_launch<8, true>(b, s);
-    case 5: return plain_launch<4, true>(b, s);
-    case 6: return plain_launch<2, true>(b, s);
-    default: return plain_launch<1, true>(b, s);
+    case 8: return plain_launch<4, kWavesStacked>(b, s);   // same tile as the MFMA variant
+    case 9: return plain_launch<4, kWavesStacked>(b, s);   // tiles of the LDS-staged variants
+    case 10: return plain_launch<8, kWavesStacked>(b, s);
+    case 0: return plain_launch<8, kWavesSideBySide>(b, s);
+    case 1: return plain_launch<4, kWavesSideBySide>(b, s);
+    case 2: return plain_launch<2, kWavesSideBySide>(b, s);
+    case 3: return plain_launch<1, kWavesSideBySide>(b, s);
+    case 4: return plain_launch<8, kWavesStacked>(b, s);
+    case 5: return plain_launch<4, kWavesStacked>(b, s);
+    case 6: return plain_launch<2, kWavesStacked>(b, s);
+    case kSplitVariant: return persistent_launch<k_plain<4, kWavesSplit, false>>(b, s);
+    default: return plain_launch<1, kWavesStacked>(b, s);
   }
 }
 
@@ -2911,23 +2984,24 @@ hipError_t mfma_launch(const BurstDev& b, hipStream_t s) {
 
 hipError_t launch_mixed(const BurstDev& b, int variant, hipStream_t s) {
   if (variant == 8) {
-    if (!mfma_fits(b)) return mixed_dt<4, true>(b, s);   // same tile shape
+    if (!mfma_fits(b)) return mixed_dt<4, kWavesStacked>(b, s);   // same tile shape
     if (b.dtype == TDBP_CF32) return mfma_launch<TDBP_CF32>(b, s);
     if (b.dtype == TDBP_CF16) return mfma_launch<TDBP_CF16>(b, s);
     if (b.dtype == TDBP_CI16) return mfma_launch<TDBP_CI16>(b, s);
     return mfma_launch<TDBP_CBF16>(b, s);
   }
   switch (variant) {
-    case 0: return mixed_dt<8, false>(b, s);
-    case 1: return mixed_dt<4, false>(b, s);
-    case 2: return mixed_dt<2, false>(b, s);
-    case 3: return mixed_dt<1, false>(b, s);
-    case 4: return mixed_dt<8, true>(b, s);
-    case 5: return mixed_dt<4, true>(b, s);
-    case 6: return mixed_dt<2, true>(b, s);
-    case 9: return mixed_dt<4, true, true>(b, s);
-    case 10: return mixed_dt<8, true, true>(b, s);
-    default: return mixed_dt<1, true>(b, s);
+    case 0: return mixed_dt<8, kWavesSideBySide>(b, s);
+    case 1: return mixed_dt<4, kWavesSideBySide>(b, s);
+    case 2: return mixed_dt<2, kWavesSideBySide>(b, s);
+    case 3: return mixed_dt<1, kWavesSideBySide>(b, s);
+    case 4: return mixed_dt<8, kWavesStacked>(b, s);
+    case 5: return mixed_dt<4, kWavesStacked>(b, s);
+    case 6: return mixed_dt<2, kWavesStacked>(b, s);
+    case kSplitVariant: return mixed_dt<4, kWavesSplit>(b, s);
+    case 9: return mixed_dt<4, kWavesStacked, true>(b, s);
+    case 10: return mixed_dt<8, kWavesStacked, true>(b, s);
+    default: return mixed_dt<1, kWavesStacked>(b, s);
   }
 }
 

@@ -278,10 +278,24 @@ int default_variant(int precision) {
   return (v >= 0 && v < kNumVariants) ? v : 5;
 }
 
-// Orbit upload + fit on a stream with stream-ordered temporary memory.
+// Whether the fit may carry the orbit in its arguments (launch_fit_arg).  Not
+// while the stream is captured: the fit of a captured call stays refused, by
+// the wait below, as replays would keep the orbit of the capture.
+static bool orbit_in_args(const tdbp_geom* g, hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (s && (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone))
+    return false;
+  return g->numstatevec <= kFitArgVec;
+}
+
+// The fit on a stream.  Orbits of up to kFitArgVec vectors go with the launch
+// and the call returns at once; larger ones are uploaded to stream-ordered
+// temporary memory, which the call waits for (31 us of a small burst's 81).
 int fit_on_stream(BurstDev& b, const tdbp_geom* g, double* d_coef,
                   hipStream_t s) {
   std::vector<double> orb = pack_orbit(g);
+  if (orbit_in_args(g, s))
+    return hip_check(launch_fit_arg(b, orb.data(), d_coef, s), "fit launch");
   double* d_orb = nullptr;
   int st = hip_check(hipMallocAsync((void**)&d_orb, orb.size() * 8, s),
                      "hipMallocAsync(orbit)");
@@ -620,7 +634,9 @@ int tdbp_fit_aperture(const tdbp_geom* g, const int16_t* d_dem, double* d_coef,
   BurstDev b;
   fill_burst(g, &b);
   b.dem = d_dem;
-  return fit_on_stream(b, g, d_coef, (hipStream_t)stream);
+  if ((st = fit_on_stream(b, g, d_coef, (hipStream_t)stream))) return st;
+  // Callers may use the parabolas on another stream.
+  return hip_check(hipStreamSynchronize((hipStream_t)stream), "fit sync");
 }
 
 int tdbp_setazoff(const tdbp_geom* g, const double* d_coef, double* d_azoff,
@@ -722,16 +738,24 @@ int tdbp_backproject_noalloc(const tdbp_geom* g, const tdbp_samples* smp,
   b.out = (float2*)d_out;
   const int variant = set_tiles(&b, default_variant(precision), false);
   const int n = g->numstatevec;
-  if ((st = hip_check(hipMemcpyAsync(sc, g->timeorbit, n * sizeof(double),
-                                     hipMemcpyHostToDevice, s), "orbit times")) ||
-      (st = hip_check(hipMemcpyAsync(sc + n, g->xx, 3 * n * sizeof(double),
-                                     hipMemcpyHostToDevice, s), "orbit positions")) ||
-      (st = hip_check(hipMemcpyAsync(sc + 4 * n, g->vv, 3 * n * sizeof(double),
-                                     hipMemcpyHostToDevice, s), "orbit velocities")))
-    return st;
-  point_orbit(&b, sc, n);
   double* coef = sc + kScratchOrbit;
-  if ((st = hip_check(launch_fit_one(b, coef, s), "fit launch"))) return st;
+  if (orbit_in_args(g, s)) {
+    double orb[7 * kFitArgVec];
+    std::copy(g->timeorbit, g->timeorbit + n, orb);
+    std::copy(g->xx, g->xx + 3 * n, orb + n);
+    std::copy(g->vv, g->vv + 3 * n, orb + 4 * n);
+    if ((st = hip_check(launch_fit_arg(b, orb, coef, s), "fit launch"))) return st;
+  } else {
+    if ((st = hip_check(hipMemcpyAsync(sc, g->timeorbit, n * sizeof(double),
+                                       hipMemcpyHostToDevice, s), "orbit times")) ||
+        (st = hip_check(hipMemcpyAsync(sc + n, g->xx, 3 * n * sizeof(double),
+                                       hipMemcpyHostToDevice, s), "orbit positions")) ||
+        (st = hip_check(hipMemcpyAsync(sc + 4 * n, g->vv, 3 * n * sizeof(double),
+                                       hipMemcpyHostToDevice, s), "orbit velocities")))
+      return st;
+    point_orbit(&b, sc, n);
+    if ((st = hip_check(launch_fit_one(b, coef, s), "fit launch"))) return st;
+  }
   b.orb_t = b.orb_x = b.orb_v = nullptr;
   b.coef = coef;
   b.counters = (int*)(sc + kScratchCounters);

@@ -83,6 +83,10 @@ inline int wg_cols(const Variant& v) {
 
 // Launchers (tdbp_kernels.hip).  All return hipError_t of the launch.
 hipError_t launch_fit_one(const BurstDev& b, double* coef, hipStream_t s);
+// The same with the orbit table [t(n) | x(3n) | v(3n)] (host memory, read before
+// the call returns) in the kernel's arguments: b.nsv <= kFitArgVec.
+constexpr int kFitArgVec = 32;   // 1.8 KB; orbit files hold 11 to 17 vectors
+hipError_t launch_fit_arg(const BurstDev& b, const double* orbit, double* coef, hipStream_t s);
 hipError_t launch_setxyz(const BurstDev& b, double* xyz, double* xyzfit,
                          hipStream_t s);
 hipError_t launch_setazoff(const BurstDev& b, double* azoff, hipStream_t s);

@@ -2422,7 +2422,8 @@ __device__ __forceinline__ double zero_doppler_range(const double* xyz, const do
 
 // Three zero-Doppler solves of a window line, the aperture centres, the
 // parabola, by its kFitLanes lanes.  Lines at or beyond nfit get (0, 0, 0).
-__device__ __forceinline__ void fit_line(const BurstDev& b, int line,
+__device__ __forceinline__ void fit_line(const BurstDev& b, const double* orb_t,
+                                         const double* orb_x, const double* orb_v, int line,
                                          double* coef) {
   double* c = coef + 3 * line;
   const int sub = threadIdx.x & (kFitLanes - 1);
@@ -2445,7 +2446,7 @@ __device__ __forceinline__ void fit_line(const BurstDev& b, int line,
   const int pix = b.firstpix + node * fit_node_step(b.firstpix, b.lastpix);
   double xyz[3];
   pixel_ecef(b, line, pix, xyz);
-  const double rng = zero_doppler_range(xyz, b.orb_t, b.orb_x, b.orb_v, b.nsv, f.tmid, f.xyz_mid,
+  const double rng = zero_doppler_range(xyz, orb_t, orb_x, orb_v, b.nsv, f.tmid, f.xyz_mid,
                                         f.vel_mid);
   const int y = aperture_centre(xyz, rng, f);
   const int y0 = __shfl(y, 0, kFitLanes), y1 = __shfl(y, 4, kFitLanes),
@@ -2455,13 +2456,31 @@ __device__ __forceinline__ void fit_line(const BurstDev& b, int line,
 
 __global__ __launch_bounds__(kWave) void k_fit(BurstDev b, double* coef) {
   const int line = (blockIdx.x * kWave + threadIdx.x) / kFitLanes;
-  if (line < b.nlines) fit_line(b, line, coef);
+  if (line < b.nlines) fit_line(b, b.orb_t, b.orb_x, b.orb_v, line, coef);
+}
+
+// The fit of a burst whose orbit travels with the launch: no table on the
+// device, no upload, and nothing on the host to wait for.
+struct FitArg {
+  BurstDev b;
+  double* coef;
+  double orb[7 * kFitArgVec];   // [t(n) | x(3n) | v(3n)]
+};
+__global__ __launch_bounds__(kWave) void k_fit_arg(FitArg a) {
+  // The table is indexed in the kernel's argument segment itself.
+  typedef const char __attribute__((address_space(4)))* arg_t;
+  const double* orb = (const double*)((arg_t)__builtin_amdgcn_kernarg_segment_ptr() +
+                                      __builtin_offsetof(FitArg, orb));
+  const int line = (blockIdx.x * kWave + threadIdx.x) / kFitLanes;
+  if (line < a.b.nlines)
+    fit_line(a.b, orb, orb + a.b.nsv, orb + 4 * a.b.nsv, line, a.coef);
 }
 
 __global__ __launch_bounds__(kWave) void k_batch_fit(const BurstDev* __restrict__ bursts) {
   const BurstDev& b = bursts[blockIdx.y];
   const int line = (blockIdx.x * kWave + threadIdx.x) / kFitLanes;
-  if (line < b.nlines) fit_line(b, line, const_cast<double*>(b.coef));
+  if (line < b.nlines)
+    fit_line(b, b.orb_t, b.orb_x, b.orb_v, line, const_cast<double*>(b.coef));
 }
 
 // setxyz: ECEF of [firstpix, lastpix], zero elsewhere; fit nodes per line.
@@ -3052,6 +3071,18 @@ hipError_t launch_batch_fit(const BurstDev* d_bursts, int nbursts,
 hipError_t launch_fit_one(const BurstDev& b, double* coef, hipStream_t s) {
   hipLaunchKernelGGL(k_fit, dim3(blocks_for((size_t)b.nlines * kFitLanes, kWave)), dim3(kWave), 0,
                      s, b, coef);
+  return hipGetLastError();
+}
+
+hipError_t launch_fit_arg(const BurstDev& b, const double* orbit, double* coef, hipStream_t s) {
+  if (b.nsv > kFitArgVec) return hipErrorInvalidValue;
+  FitArg a;
+  a.b = b;
+  a.coef = coef;
+  std::copy(orbit, orbit + 7 * (size_t)b.nsv, a.orb);
+  std::fill(a.orb + 7 * (size_t)b.nsv, a.orb + 7 * kFitArgVec, 0.0);
+  hipLaunchKernelGGL(k_fit_arg, dim3(blocks_for((size_t)b.nlines * kFitLanes, kWave)),
+                     dim3(kWave), 0, s, a);
   return hipGetLastError();
 }
 

@@ -97,61 +97,67 @@ TDBP_HD void dft16(float2* x) {
 constexpr int kOsLds = kOsN + 2 * (kOsN / 32);
 TDBP_HD constexpr int os_pad(int p) { return p + 2 * (p >> 5); }
 
-// Twiddle w^m, m < kOsN, from two short tables (1.5 KB, LDS on the device):
-// hi[i] = w^(64 i), i < 128, and lo[i] = w^i, i < 64; w^m = hi[m / 64]
-// lo[m mod 64] (one rounding more than a full table).
-constexpr int kTwHi = kOsN / 64;
-constexpr int kTwLo = 64;
+// Twiddles come from tables, every one of them rounded once from FP64: the
+// table of an L-point stage (16, L/16) holds w_L^(j k) at [k L/16 + j] (k < 16,
+// j < L/16), so the lanes of a wave read it in order.  The first stage's table
+// (L = N, 8 N bytes) stays in global memory, where the caches keep it; those of
+// the stages after it (N/16 values, for 8192 points 512 + 32) go to LDS.
+// Fifteen twiddles built as products of four lookups took 60 of a stage's 270
+// vector instructions, and their roundings were the pair's largest error.
+TDBP_HD constexpr int os_mid_values(int n) { return n == kOsN ? n / 16 + n / 256 : n / 16; }
+TDBP_HD constexpr int os_table_values(int n) { return n + os_mid_values(n); }
 struct OsTwiddle {
-  const float2* hi;
-  const float2* lo;
-  TDBP_HD float2 operator()(int m) const { return c_mul(hi[m >> 6], lo[m & 63]); }
+  const float2* first;
+  const float2* mid;   // 8192 points: the stage (16, 2) at mid + 512
 };
-
-// w^(k STEP), k STEP < kOsN: hi alone for a multiple of 64 (lo[0] = 1).
-template <int STEP>
-TDBP_HD float2 os_tw(const OsTwiddle& tw, int k) {
-  if constexpr (STEP % 64 == 0) return tw.hi[k * (STEP / 64)];
-  else return tw(k * STEP);
-}
-
-// t[r] = w^(U j r), r < 16: powers 1, 2, 4, 8 from the tables, the other
-// eleven as products (at most three more roundings).
-template <int U>
-TDBP_HD void os_twiddles16(const OsTwiddle& tw, int j, float2* t) {
-  t[0] = make_float2(1.f, 0.f);
-  t[1] = os_tw<U>(tw, j);
-  t[2] = os_tw<2 * U>(tw, j);
-  t[4] = os_tw<4 * U>(tw, j);
-  t[8] = os_tw<8 * U>(tw, j);
-  t[3] = c_mul(t[1], t[2]);
-  t[5] = c_mul(t[1], t[4]);
-  t[6] = c_mul(t[2], t[4]);
-  t[7] = c_mul(t[3], t[4]);
-#pragma unroll
-  for (int r = 9; r < 16; ++r) t[r] = c_mul(t[r - 8], t[8]);
-}
-
-// A radix-16 stage of butterfly j (twiddle w^(U j r)) whose values sit at
-// lds[a0 + STEP r + STEP2 floor(r/2)]: read, [DIT: twiddle], DFT, [DIF:
-// twiddle], write back in place.
-template <int U, int STEP, bool DIT, int STEP2 = 0>
-TDBP_HD void os_stage16(float2* lds, int a0, int j, const OsTwiddle& tw, float2* v) {
-  float2 t[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) v[r] = lds[a0 + STEP * r + STEP2 * (r >> 1)];
-  os_twiddles16<U>(tw, j, t);
-  if constexpr (DIT) {
-#pragma unroll
-    for (int r = 1; r < 16; ++r) v[r] = c_mul(v[r], t[r]);
+// Entry i of a length's tables (first, then mid) is w_N^m, m the return value.
+TDBP_HD int os_table_power(int n, int i) {
+  int step = 1, L = n;   // w_L = w_N^step
+  while (i >= L) {
+    i -= L;
+    L /= 16;
+    step *= 16;
   }
+  return step * ((i / (L / 16)) * (i % (L / 16)));
+}
+
+// v[k] times the twiddles of butterfly j of an L-point stage: all fifteen from
+// the table (FULL), or six and the other nine as products of two of them.  FULL
+// is the more exact (1.6e-7 against 1.8e-7 over a 1024-point round trip, 2.2e-7
+// with four lookups) and about 5 % slower: its loads cost the caches and LDS
+// more than the products cost the vector units.
+template <int L, bool FULL = false>
+TDBP_HD void os_apply(const float2* tab, int j, float2* v) {
+  if constexpr (FULL) {
+#pragma unroll
+    for (int k = 1; k < 16; ++k) v[k] = c_mul(v[k], tab[k * (L / 16) + j]);
+    return;
+  }
+  float2 lo[4], hi[4];
+#pragma unroll
+  for (int r = 1; r < 4; ++r) {
+    lo[r] = tab[r * (L / 16) + j];
+    hi[r] = tab[4 * r * (L / 16) + j];
+  }
+#pragma unroll
+  for (int k = 1; k < 16; ++k) {
+    const int q = k >> 2, r = k & 3;
+    v[k] = c_mul(v[k], q == 0 ? lo[r] : r == 0 ? hi[q] : c_mul(hi[q], lo[r]));
+  }
+}
+
+// A radix-16 stage of butterfly j (twiddles of an L-point stage) whose values
+// sit at lds[a0 + STEP r]: read, [DIT: twiddle], DFT, [DIF: twiddle], write back
+// in place.
+template <int L, int STEP, bool DIT, bool FULL>
+TDBP_HD void os_stage16(float2* lds, int a0, int j, const float2* tab, float2* v) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r] = lds[a0 + STEP * r];
+  if constexpr (DIT) os_apply<L, FULL>(tab, j, v);
   dft16(v);
-  if constexpr (!DIT) {
+  if constexpr (!DIT) os_apply<L, FULL>(tab, j, v);
 #pragma unroll
-    for (int k = 1; k < 16; ++k) v[k] = c_mul(v[k], t[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < 16; ++k) lds[a0 + STEP * k + STEP2 * (k >> 1)] = v[k];
+  for (int k = 0; k < 16; ++k) lds[a0 + STEP * k] = v[k];
 }
 
 // The stages of thread t.  Stage (16, 512): butterfly t, values t + 512 r,
@@ -159,21 +165,21 @@ TDBP_HD void os_stage16(float2* lds, int a0, int j, const OsTwiddle& tw, float2*
 // Stage (16, 32): butterfly j = t mod 32 of sub-block t / 32.  Stage (16, 2):
 // butterfly t mod 2 of sub-block t / 2.  Stage (2, 1): the eight pairs at
 // positions 2 (t + 512 h), held in registers as v[2h], v[2h + 1].
+template <bool FULL = false>
 TDBP_HD void os_dif_first(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  float2 w[16];
-  os_twiddles16<1>(tw, t, w);
   dft16(v);
-#pragma unroll
-  for (int k = 1; k < 16; ++k) v[k] = c_mul(v[k], w[k]);
+  os_apply<kOsN, FULL>(tw.first, t, v);
   float2* q = lds + os_pad(t);
 #pragma unroll
   for (int k = 0; k < 16; ++k) q[544 * k] = v[k];
 }
+template <bool FULL = false>
 TDBP_HD void os_dif_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<16, 34, false>(lds, 544 * (t >> 5) + (t & 31), t & 31, tw, v);
+  os_stage16<512, 34, false, FULL>(lds, 544 * (t >> 5) + (t & 31), t & 31, tw.mid, v);
 }
+template <bool FULL = false>
 TDBP_HD void os_dif_mid2(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<256, 2, false>(lds, 34 * (t >> 1) + (t & 1), t & 1, tw, v);
+  os_stage16<32, 2, false, FULL>(lds, 34 * (t >> 1) + (t & 1), t & 1, tw.mid + 512, v);
 }
 TDBP_HD void os_dif_last(const float2* lds, int t, float2* v) {
   const float2* q = lds + os_pad(2 * t);
@@ -192,20 +198,20 @@ TDBP_HD void os_dit_first(float2* lds, int t, const float2* v) {
     q[1088 * h + 1] = c_sub(v[2 * h], v[2 * h + 1]);
   }
 }
+template <bool FULL = false>
 TDBP_HD void os_dit_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<256, 2, true>(lds, 34 * (t >> 1) + (t & 1), t & 1, tw, v);
+  os_stage16<32, 2, true, FULL>(lds, 34 * (t >> 1) + (t & 1), t & 1, tw.mid + 512, v);
 }
+template <bool FULL = false>
 TDBP_HD void os_dit_mid2(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<16, 34, true>(lds, 544 * (t >> 5) + (t & 31), t & 31, tw, v);
+  os_stage16<512, 34, true, FULL>(lds, 544 * (t >> 5) + (t & 31), t & 31, tw.mid, v);
 }
+template <bool FULL = false>
 TDBP_HD void os_dit_last(const float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  float2 w[16];
   const float2* q = lds + os_pad(t);
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = q[544 * r];
-  os_twiddles16<1>(tw, t, w);
-#pragma unroll
-  for (int r = 1; r < 16; ++r) v[r] = c_mul(v[r], w[r]);
+  os_apply<kOsN, FULL>(tw.first, t, v);
   dft16(v);
 }
 
@@ -214,16 +220,16 @@ TDBP_HD void os_dit_last(const float2* lds, int t, const OsTwiddle& tw, float2* 
 // os_dif_host: data in natural order -> data[p] = X[drev(p)].
 // os_dit_host: data[p] = Y[drev(p)] -> data in natural order, the forward
 // transform of Y.
+template <int N>
 struct OsHostTables {
-  float2 hi[kTwHi], lo[kTwLo];
-  explicit OsHostTables(const float2* table) {
-    for (int i = 0; i < kTwHi; ++i) hi[i] = table[64 * i];
-    for (int i = 0; i < kTwLo; ++i) lo[i] = table[i];
+  float2 v[os_table_values(N)];
+  explicit OsHostTables(const float2* table) {   // w^m of 8192 points
+    for (int i = 0; i < os_table_values(N); ++i) v[i] = table[kOsN / N * os_table_power(N, i)];
   }
-  OsTwiddle tw() const { return OsTwiddle{hi, lo}; }
+  OsTwiddle tw() const { return OsTwiddle{v, v + N}; }
 };
 inline void os_dif_host(float2* data, const float2* table) {
-  const OsHostTables tb(table);
+  const OsHostTables<kOsN> tb(table);
   const OsTwiddle tw = tb.tw();
   float2* lds = new float2[kOsLds];
   float2 v[16];
@@ -240,7 +246,7 @@ inline void os_dif_host(float2* data, const float2* table) {
   delete[] lds;
 }
 inline void os_dit_host(float2* data, const float2* table) {
-  const OsHostTables tb(table);
+  const OsHostTables<kOsN> tb(table);
   const OsTwiddle tw = tb.tw();
   float2* lds = new float2[kOsLds];
   float2 v[16];
@@ -257,132 +263,197 @@ inline void os_dit_host(float2* data, const float2* table) {
   delete[] lds;
 }
 
-// ---------------------------------------------------------------- 4096
-// The 4096-point pair of the interferograms' upsampling (int/crossmul.f90),
-// the same scheme with stages (16, 256), (16, 16), (16, 1) and kUpThreads =
-// 256 threads: position p = 256 d0 + 16 d1 + d2 holds bin d0 + 16 d1 + 256
-// d2 after the DIF; thread t holds values t + 256 m in natural order and
-// positions 16 t + m in the DIF order.  Twiddles w_4096^e = w^(2e) come from
-// the 8192-point tables.  Layout: position p at up_pad(p) = p + floor(p/32)
-// (offsets 264 k, 16 r + floor(r/2) and r within a butterfly); stages (16,
-// 256) and (16, 1) touch each bank pair once per half-wave, stage (16, 16)
+// ------------------------------------------------- 1024, 2048, 4096
+// The N-point pairs of the interferograms' upsampling (int/crossmul.f90), the
+// same scheme with N/16 threads and stages (16, N/16), (16, R), (R, 1), R =
+// N/256 = 4, 8 or 16: position p = (N/16) d0 + R d1 + d2 holds bin d0 + 16 d1
+// + 256 d2 after the DIF; thread t holds values t + (N/16) m in natural order
+// and positions 16 t + m in the DIF order (16/R whole sub-blocks of the last
+// stage).  Layout: position p at up_pad(p) = p + floor(p/32), so the values of a
+// butterfly sit (N/16)(33/32) k, R r + floor(R r/32) and r apart; stages
+// (16, N/16) and (R, 1) touch each bank pair once per half-wave, stage (16, R)
 // twice (no additive padding clears all three, a host simulation shows).
 constexpr int kUpN = 4096;
-constexpr int kUpThreads = kUpN / 16;
-constexpr int kUpLds = kUpN + kUpN / 32;
+// Lengths with every twiddle from the table: those where the interferograms'
+// errors would else exceed a library transform's (2048 points, looks 4 x 2:
+// 1.1e-7 against 1.0e-7).
+TDBP_HD constexpr bool up_full(int n) { return n != kUpN; }
+TDBP_HD constexpr int up_threads(int n) { return n / 16; }
+TDBP_HD constexpr int up_lds(int n) { return n == kOsN ? kOsLds : n + n / 32; }
 TDBP_HD constexpr int up_pad(int p) { return p + (p >> 5); }
 
-TDBP_HD void up_dif_first(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  float2 w[16];
-  os_twiddles16<2>(tw, t, w);
-  dft16(v);
+// In-register forward DFT of 8 points, natural order in and out (n = 2 n1 +
+// n2, k = k1 + 4 k2).
+TDBP_HD void dft8(float2* x) {
+  float2 a0 = x[0], a1 = x[2], a2 = x[4], a3 = x[6];
+  float2 b0 = x[1], b1 = x[3], b2 = x[5], b3 = x[7];
+  dft4(a0, a1, a2, a3);
+  dft4(b0, b1, b2, b3);
+  b1 = c_w8(b1);
+  b2 = c_mni(b2);
+  b3 = c_w8_3(b3);
+  x[0] = c_add(a0, b0);
+  x[1] = c_add(a1, b1);
+  x[2] = c_add(a2, b2);
+  x[3] = c_add(a3, b3);
+  x[4] = c_sub(a0, b0);
+  x[5] = c_sub(a1, b1);
+  x[6] = c_sub(a2, b2);
+  x[7] = c_sub(a3, b3);
+}
+
+// The R-point DFTs of the 16/R sub-blocks in v.
+template <int R>
+TDBP_HD void up_dft_last(float2* v) {
+  if constexpr (R == 16) {
+    dft16(v);
+  } else {
 #pragma unroll
-  for (int k = 1; k < 16; ++k) v[k] = c_mul(v[k], w[k]);
+    for (int q = 0; q < 16; q += R) {
+      if constexpr (R == 8) dft8(v + q);
+      else dft4(v[q], v[q + 1], v[q + 2], v[q + 3]);
+    }
+  }
+}
+
+template <int N>
+TDBP_HD void up_dif_first(float2* lds, int t, const OsTwiddle& tw, float2* v) {
+  dft16(v);
+  os_apply<N, up_full(N)>(tw.first, t, v);
   float2* q = lds + up_pad(t);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) q[264 * k] = v[k];
+  for (int k = 0; k < 16; ++k) q[up_pad(N / 16) * k] = v[k];
 }
-TDBP_HD void up_dif_mid(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<32, 16, false, 1>(lds, 264 * (t >> 4) + (t & 15), t & 15, tw, v);
+// Stage (16, R) of butterfly t mod R of sub-block t / R.
+template <int N, bool DIT>
+TDBP_HD void up_mid(float2* lds, int t, const OsTwiddle& tw, float2* v) {
+  constexpr int R = N / 256;
+  const int j = t & (R - 1);
+  float2* q = lds + up_pad(N / 16) * (t / R) + j;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r] = q[up_pad(R * r)];
+  if constexpr (DIT) os_apply<N / 16, up_full(N)>(tw.mid, j, v);
+  dft16(v);
+  if constexpr (!DIT) os_apply<N / 16, up_full(N)>(tw.mid, j, v);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) q[up_pad(R * k)] = v[k];
 }
+template <int N>
 TDBP_HD void up_dif_last(const float2* lds, int t, float2* v) {
   const float2* q = lds + up_pad(16 * t);
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = q[r];
-  dft16(v);
+  up_dft_last<N / 256>(v);
 }
+template <int N>
 TDBP_HD void up_dit_first(float2* lds, int t, float2* v) {
-  dft16(v);
+  up_dft_last<N / 256>(v);
   float2* q = lds + up_pad(16 * t);
 #pragma unroll
   for (int k = 0; k < 16; ++k) q[k] = v[k];
 }
-TDBP_HD void up_dit_mid(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<32, 16, true, 1>(lds, 264 * (t >> 4) + (t & 15), t & 15, tw, v);
-}
+template <int N>
 TDBP_HD void up_dit_last(const float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  float2 w[16];
   const float2* q = lds + up_pad(t);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) v[r] = q[264 * r];
-  os_twiddles16<2>(tw, t, w);
-#pragma unroll
-  for (int r = 1; r < 16; ++r) v[r] = c_mul(v[r], w[r]);
+  for (int r = 0; r < 16; ++r) v[r] = q[up_pad(N / 16) * r];
+  os_apply<N, up_full(N)>(tw.first, t, v);
   dft16(v);
 }
 
-// Host 4096-point transforms, as os_dif_host / os_dit_host.
+// Host transforms of these lengths, as os_dif_host / os_dit_host.
+template <int N = kUpN>
 inline void up_dif_host(float2* data, const float2* table) {
-  const OsHostTables tb(table);
+  const OsHostTables<N> tb(table);
   const OsTwiddle tw = tb.tw();
-  float2* lds = new float2[kUpLds];
+  constexpr int kT = up_threads(N);
+  float2* lds = new float2[up_lds(N)];
   float2 v[16];
-  for (int t = 0; t < kUpThreads; ++t) {
-    for (int r = 0; r < 16; ++r) v[r] = data[t + kUpThreads * r];
-    up_dif_first(lds, t, tw, v);
+  for (int t = 0; t < kT; ++t) {
+    for (int r = 0; r < 16; ++r) v[r] = data[t + kT * r];
+    up_dif_first<N>(lds, t, tw, v);
   }
-  for (int t = 0; t < kUpThreads; ++t) up_dif_mid(lds, t, tw, v);
-  for (int t = 0; t < kUpThreads; ++t) {
-    up_dif_last(lds, t, v);
+  for (int t = 0; t < kT; ++t) up_mid<N, false>(lds, t, tw, v);
+  for (int t = 0; t < kT; ++t) {
+    up_dif_last<N>(lds, t, v);
     for (int m = 0; m < 16; ++m) data[16 * t + m] = v[m];
   }
   delete[] lds;
 }
+template <int N = kUpN>
 inline void up_dit_host(float2* data, const float2* table) {
-  const OsHostTables tb(table);
+  const OsHostTables<N> tb(table);
   const OsTwiddle tw = tb.tw();
-  float2* lds = new float2[kUpLds];
+  constexpr int kT = up_threads(N);
+  float2* lds = new float2[up_lds(N)];
   float2 v[16];
-  for (int t = 0; t < kUpThreads; ++t) {
+  for (int t = 0; t < kT; ++t) {
     for (int m = 0; m < 16; ++m) v[m] = data[16 * t + m];
-    up_dit_first(lds, t, v);
+    up_dit_first<N>(lds, t, v);
   }
-  for (int t = 0; t < kUpThreads; ++t) up_dit_mid(lds, t, tw, v);
-  for (int t = 0; t < kUpThreads; ++t) {
-    up_dit_last(lds, t, tw, v);
-    for (int k = 0; k < 16; ++k) data[t + kUpThreads * k] = v[k];
+  for (int t = 0; t < kT; ++t) up_mid<N, true>(lds, t, tw, v);
+  for (int t = 0; t < kT; ++t) {
+    up_dit_last<N>(lds, t, tw, v);
+    for (int k = 0; k < 16; ++k) data[t + kT * k] = v[k];
   }
   delete[] lds;
 }
 
-// Copies the two twiddle tables from the full table w^m (`table`, m <
-// kOsN) into `twl` (kTwHi + kTwLo values, LDS); a barrier must follow before
-// any transform reads them.
+// The tables of N points on the device (os_table_values(N) values), and the ones
+// that go to LDS copied into `twl` (os_mid_values(N) values); a barrier must
+// follow before any transform reads them.
+template <int N>
 __device__ __forceinline__ OsTwiddle os_twiddles_lds(float2* twl, const float2* __restrict__ table) {
-  const int t = threadIdx.x;
-  if (t < kTwHi) twl[t] = table[64 * t];
-  else if (t < kTwHi + kTwLo) twl[t] = table[t - kTwHi];
-  return OsTwiddle{twl, twl + kTwHi};
+  for (int i = threadIdx.x; i < os_mid_values(N); i += blockDim.x) twl[i] = table[N + i];
+  return OsTwiddle{table, twl};
 }
 
-// Device DIF by kOsThreads threads: v[m] holds value threadIdx.x + kOsThreads
-// m of the block on entry and position 2 (threadIdx.x + kOsThreads (m / 2)) +
+// Entry i of the tables of n points.
+__device__ __forceinline__ float2 os_table_entry(int n, int i) {
+  const double pi = 3.141592653589793115997963468544185161590576171875;
+  double sn, cs;
+  sincos(-2.0 * pi * (double)os_table_power(n, i) / n, &sn, &cs);
+  return make_float2((float)cs, (float)sn);
+}
+
+// The index again, as a value the compiler cannot connect with the first: the
+// last stage's twiddles are the first's, and keeping them in 30 registers from
+// one to the other would spill what the stages between need.
+__device__ __forceinline__ int os_fresh(int t) {
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// Device DIF by kOsThreads threads, t their index: v[m] holds value t +
+// kOsThreads m of the block on entry and position 2 (t + kOsThreads (m / 2)) +
 // m mod 2 of the output on return.  The twiddle tables must be ordered
 // before the call.  On return every thread's remaining LDS positions are its
 // own (os_dit_regs may follow without a barrier).
-__device__ __forceinline__ void os_dif_regs(float2* lds, const OsTwiddle& tw, float2* v) {
-  const int t = threadIdx.x;
-  os_dif_first(lds, t, tw, v);
+template <bool FULL = false>
+__device__ __forceinline__ void os_dif_regs(float2* lds, int t, const OsTwiddle& tw,
+                                            float2* v) {
+  os_dif_first<FULL>(lds, t, tw, v);
   __syncthreads();
-  os_dif_mid1(lds, t, tw, v);
+  os_dif_mid1<FULL>(lds, t, tw, v);
   __syncthreads();
-  os_dif_mid2(lds, t, tw, v);
+  os_dif_mid2<FULL>(lds, t, tw, v);
   __syncthreads();
   os_dif_last(lds, t, v);
 }
 
-// Device DIT: v in the DIF output order on entry, value threadIdx.x +
-// kOsThreads m of the forward transform on return.  LDS positions other
+// Device DIT: v in the DIF output order on entry, value t + kOsThreads m of the forward transform on return.  LDS positions other
 // threads may still read must not be needed by the caller afterwards.
-__device__ __forceinline__ void os_dit_regs(float2* lds, const OsTwiddle& tw, float2* v) {
-  const int t = threadIdx.x;
+template <bool FULL = false>
+__device__ __forceinline__ void os_dit_regs(float2* lds, int t, const OsTwiddle& tw,
+                                            float2* v) {
   os_dit_first(lds, t, v);
+  t = os_fresh(t);
   __syncthreads();
-  os_dit_mid1(lds, t, tw, v);
+  os_dit_mid1<FULL>(lds, t, tw, v);
   __syncthreads();
-  os_dit_mid2(lds, t, tw, v);
+  os_dit_mid2<FULL>(lds, t, tw, v);
   __syncthreads();
-  os_dit_last(lds, t, tw, v);
+  os_dit_last<FULL>(lds, t, tw, v);
 }
 
 }  // namespace tdbp

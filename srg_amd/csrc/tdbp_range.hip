@@ -168,15 +168,10 @@ k_rc_store(const float2* __restrict__ raw, int nlines, int stride, int base,
 
 // ------------------------------------------------- fused overlap-save
 
-// The twiddle table of the 8192-point transform, w^m = e^{-2 pi i m/N} in FP64
-// rounded to FP32.
+// The twiddle tables of the 8192-point transform.
 __global__ void k_os_twiddles(float2* __restrict__ tw) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= kOsN) return;
-  const double pi = 3.141592653589793115997963468544185161590576171875;
-  double sn, cs;
-  sincos(-2.0 * pi * (double)m / kOsN, &sn, &cs);
-  tw[m] = make_float2((float)cs, (float)sn);
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < os_table_values(kOsN)) tw[i] = os_table_entry(kOsN, i);
 }
 
 // Forward transform of one 8192-point vector (the reference function's
@@ -186,13 +181,13 @@ __global__ void k_os_twiddles(float2* __restrict__ tw) {
 __global__ void __launch_bounds__(kOsThreads) k_os_spectrum(float2* __restrict__ v,
                                                              const float2* __restrict__ tw) {
   __shared__ float2 lds[kOsLds];
-  __shared__ float2 twl[kTwHi + kTwLo];
-  const OsTwiddle w = os_twiddles_lds(twl, tw);
+  __shared__ float2 twl[os_mid_values(kOsN)];
+  const OsTwiddle w = os_twiddles_lds<kOsN>(twl, tw);
   const int t = threadIdx.x;
   float2 x[16];
   for (int m = 0; m < 16; ++m) x[m] = v[t + m * kOsThreads];
   __syncthreads();   // the twiddle tables; every read of v is done
-  os_dif_regs(lds, w, x);
+  os_dif_regs(lds, t, w, x);
   for (int m = 0; m < 16; ++m) v[2 * (t + (m >> 1) * kOsThreads) + (m & 1)] = x[m];
 }
 
@@ -213,7 +208,7 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
         const float2* __restrict__ spec, const float2* __restrict__ tw,
         float2* __restrict__ out, int out_stride, int zero_header, unsigned* __restrict__ lmax) {
   __shared__ float2 lds[kOsLds];
-  __shared__ float2 twl[kTwHi + kTwLo];
+  __shared__ float2 twl[os_mid_values(kOsN)];
   // Work item q = (line, block), line-major, dealt so that XCD x (blocks x,
   // x + 8, ...) takes the x-th eighth of the items in order: the blocks of a
   // line, whose echo windows overlap by npts - 1 samples, share one L2.
@@ -225,7 +220,7 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
   const int b = q - l * nblk;
   const int M = kOsN - npts + 1;
   const int k0 = b * M;
-  const OsTwiddle w = os_twiddles_lds(twl, tw);
+  const OsTwiddle w = os_twiddles_lds<kOsN>(twl, tw);
   const float2* echo = raw + (size_t)l * stride + kHdr;
   // thread t holds values t + kOsThreads m, m < 16, of the block (natural
   // order), between the transforms positions 2 (t + kOsThreads (m / 2)) +
@@ -238,12 +233,12 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
     v[m] = k0 + n < nsamps ? echo[k0 + n] : make_float2(0.f, 0.f);
   }
   __syncthreads();   // the twiddle tables
-  os_dif_regs(lds, w, v);
+  os_dif_regs(lds, t, w, v);
 #pragma unroll
   for (int m = 0; m < 16; ++m)
     v[m] = c_mul(make_float2(v[m].x, -v[m].y),
                  spec[2 * (t + (m >> 1) * kOsThreads) + (m & 1)]);
-  os_dit_regs(lds, w, v);
+  os_dit_regs(lds, t, w, v);
   const int kend = min(M, nvalid - k0);
   float mx = 0.f;
   float2* o = out ? out + (size_t)l * out_stride : nullptr;
@@ -416,11 +411,11 @@ int compress_overlap_save(RcState* r, const float2* raw, int nlines, int stride,
     return set_error(TDBP_ERR_NOMEM, "range compression: reference spectrum");
   }
   if (!r->tw) {
-    if (hipMalloc((void**)&r->tw, sizeof(float2) * kOsN) != hipSuccess) {
+    if (hipMalloc((void**)&r->tw, sizeof(float2) * os_table_values(kOsN)) != hipSuccess) {
       r->tw = nullptr;
       return set_error(TDBP_ERR_NOMEM, "range compression: twiddles");
     }
-    hipLaunchKernelGGL(k_os_twiddles, dim3(kOsN / 256), dim3(256), 0, s, r->tw);
+    hipLaunchKernelGGL(k_os_twiddles, dim3((os_table_values(kOsN) + 255) / 256), dim3(256), 0, s, r->tw);
     if ((st = hip_check(hipGetLastError(), "twiddle launch"))) return st;
   }
   if (!r->os_valid || !same_chirp(r->os_of, c)) {

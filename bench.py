@@ -885,7 +885,7 @@ def main():
     log(f"mixed {args.storage} vs FP64 kernel: phase {ph * 1e3:.4f} mrad, amp {amp:.2e}")
 
     # End to end from cf32 samples resident in HBM: per step every burst is
-    # packed to the storage type (k_pack + k_unify_scales into the buffers the
+    # packed to the storage type (k_pack_scale + k_pack into the buffers the
     # batch reads), then the batch runs.
     e2e = None
     if stor != T.CF32:
@@ -906,7 +906,7 @@ def main():
         e2e = {"value": round(pairs / e2e_ms / 1e6, 2), "ms_per_step": round(e2e_ms, 3),
                "speedup_vs_plain_fp64": round(plain_ms / e2e_ms, 3),
                "includes": f"pack of the {len(dev)} cf32 bursts to {args.storage} "
-                           f"(k_pack + k_unify_scales) + the batched kernel; cf32 inputs "
+                           f"(k_pack_scale + k_pack) + the batched kernel; cf32 inputs "
                            f"resident in HBM"}
         log(f"end to end (pack + batch): {e2e_ms:.2f} ms ({e2e['value']} GP/s)")
     else:

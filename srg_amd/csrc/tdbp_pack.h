@@ -77,4 +77,90 @@ __device__ __forceinline__ void word_components(uint32_t w, int dtype, float* re
   }
 }
 
+// A pulse's n samples by one workgroup: the largest |component| (NaN passed
+// over, as fmaxf does), and the words: each sample at the pulse's own scale
+// (inv = 1/own), then, where k_unify_scales would move the pulse to another
+// scale, multiplied by f and rounded again as it does (rescale).  Two samples a
+// lane and load, four loads in flight: HBM bounds both.  Rows start anywhere a
+// sample (8 bytes in, 4 out) may, hence the alignment of the types.
+constexpr int kPackBlock = 1024;
+typedef float PackF4 __attribute__((ext_vector_type(4), aligned(8)));
+typedef uint32_t PackU2 __attribute__((ext_vector_type(2), aligned(4)));
+
+__device__ __forceinline__ float pack_max(float m, float a, float b) {
+  return fmaxf(m, fmaxf(fabsf(a), fabsf(b)));
+}
+
+// The workgroup's value for every thread; `part` holds one float per wave.
+__device__ __forceinline__ float block_max(float m, float* part) {
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = part[0];
+  for (int w = 1; w < kPackBlock / 64; ++w) m = fmaxf(m, part[w]);
+  return m;
+}
+
+__device__ __forceinline__ float row_max(const float2* __restrict__ y, int n, float* part) {
+  const PackF4* y2 = (const PackF4*)y;
+  const int n2 = n >> 1;
+  float m = 0.f;
+  int i = threadIdx.x;
+  for (; i + 3 * kPackBlock < n2; i += 4 * kPackBlock) {
+    PackF4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = y2[i + k * kPackBlock];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m = pack_max(pack_max(m, v[k].x, v[k].y), v[k].z, v[k].w);
+  }
+  for (; i < n2; i += kPackBlock) {
+    const PackF4 v = y2[i];
+    m = pack_max(pack_max(m, v.x, v.y), v.z, v.w);
+  }
+  if ((n & 1) && threadIdx.x == 0) m = pack_max(m, y[n - 1].x, y[n - 1].y);
+  return block_max(m, part);
+}
+
+template <int DT>
+__device__ __forceinline__ uint32_t pack_sample(float re, float im, float inv, bool rescale,
+                                                float f) {
+  uint32_t w = pack_word(re * inv, im * inv, DT);
+  if (rescale) {
+    word_components(w, DT, &re, &im);
+    w = pack_word(re * f, im * f, DT);
+  }
+  return w;
+}
+
+template <int DT>
+__device__ __forceinline__ void pack_row(const float2* __restrict__ y, int n,
+                                         uint32_t* __restrict__ o, float inv, bool rescale,
+                                         float f) {
+  const PackF4* y2 = (const PackF4*)y;
+  PackU2* o2 = (PackU2*)o;
+  const int n2 = n >> 1;
+  auto pair = [&](const PackF4& v) {
+    return PackU2{pack_sample<DT>(v.x, v.y, inv, rescale, f),
+                  pack_sample<DT>(v.z, v.w, inv, rescale, f)};
+  };
+  int i = threadIdx.x;
+  for (; i + 3 * kPackBlock < n2; i += 4 * kPackBlock) {
+    PackF4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = y2[i + k * kPackBlock];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o2[i + k * kPackBlock] = pair(v[k]);
+  }
+  for (; i < n2; i += kPackBlock) o2[i] = pair(y2[i]);
+  if ((n & 1) && threadIdx.x == 0)
+    o[n - 1] = pack_sample<DT>(y[n - 1].x, y[n - 1].y, inv, rescale, f);
+}
+
+// The scale k_unify_scales leaves a pulse of scale s in a call whose largest
+// is M.
+__device__ __forceinline__ float unified_scale(float s, float M, int dtype) {
+  const float lowest = dtype == TDBP_CI16 ? M * (1.0f / (1 << kI16Unify)) : M * (1.0f / 65536.0f);
+  return M == 0.f ? 1.f : (s == M || (s > 0.f && s < lowest)) ? s : M;
+}
+
 }  // namespace tdbp

@@ -259,35 +259,22 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
 }
 
 // The packed words of cf32 rows y (kHdr + nvalid samples per row, stride
-// y_stride): header words zero, then each sample as k_pack would make it at
-// the line's own scale own[l], then, where k_unify_scales would rescale the
-// line to scale[l], rescaled as it does (one rounding after the other).
-constexpr int kPackBlock = 256;
+// y_stride), one workgroup per line: header words zero, then the samples from
+// the line's own scale own[l] to scale[l] (pack_row).  1500 x 21018 samples in
+// 64 us (5.9 TB/s); 64 small workgroups a line, 8 bytes a lane and load, took
+// 105 us.
+template <int DT>
 __global__ void __launch_bounds__(kPackBlock)
 k_os_pack_rows(const float2* __restrict__ y, int y_stride, int nvalid,
                uint32_t* __restrict__ packed, const float* __restrict__ own,
-               const float* __restrict__ scale, int dtype) {
-  const int l = blockIdx.y;
-  const int S = kHdr + nvalid;
+               const float* __restrict__ scale) {
+  const int l = blockIdx.x;
   const float so = own[l], sf = scale[l];
-  const float inv = pulse_inv(so);
   const bool rescale = so > 0.f && so != sf;
-  const float f = rescale ? so / sf : 1.f;
-  const float2* yl = y + (size_t)l * y_stride;
-  uint32_t* o = packed + (size_t)l * S;
-  for (int k = blockIdx.x * kPackBlock + threadIdx.x; k < S; k += gridDim.x * kPackBlock) {
-    uint32_t w = 0u;
-    if (k >= kHdr) {
-      const float2 v = yl[k];
-      w = pack_word(v.x * inv, v.y * inv, dtype);
-      if (rescale) {
-        float re, im;
-        word_components(w, dtype, &re, &im);
-        w = pack_word(re * f, im * f, dtype);
-      }
-    }
-    o[k] = w;
-  }
+  uint32_t* o = packed + (size_t)l * (kHdr + nvalid);
+  if (threadIdx.x < kHdr) o[threadIdx.x] = 0u;
+  pack_row<DT>(y + (size_t)l * y_stride + kHdr, nvalid, o + kHdr, pulse_inv(so), rescale,
+               rescale ? so / sf : 1.f);
 }
 
 // Per line: its own scale (the pack kernel's, from the largest |component|)
@@ -311,11 +298,8 @@ k_os_scales(unsigned* __restrict__ lmax, int L, int dtype, float* __restrict__ o
   __syncthreads();
   float M = part[0];
   for (int w = 1; w < kScaleBlock / 64; ++w) M = fmaxf(M, part[w]);
-  const float lowest = dtype == TDBP_CI16 ? M * (1.0f / (1 << kI16Unify)) : M * (1.0f / 65536.0f);
-  for (int l = threadIdx.x; l < L; l += kScaleBlock) {
-    const float s = own[l];
-    scale[l] = M == 0.f ? 1.f : (s == M || (s > 0.f && s < lowest)) ? s : M;
-  }
+  for (int l = threadIdx.x; l < L; l += kScaleBlock)
+    scale[l] = unified_scale(own[l], M, dtype);
 }
 
 __global__ void k_zero_words(unsigned* __restrict__ p, int n) {
@@ -398,10 +382,8 @@ int transform_length(int nsamps) {
 // The fused overlap-save path of tdbp_range_compress (npts <= kOsN / 2).
 // cf32 only: one launch.  Packed: the first launch writes the cf32 rows (if
 // asked) and the per-line maxima, k_os_scales turns them into the scales
-// k_pack and k_unify_scales would give, and a second launch recomputes the
-// lines and writes their words -- the words of tdbp_pack_samples on the cf32
-// rows, with HBM reading the echoes twice instead of writing and reading
-// cf32 rows and rewriting the rescaled words.
+// tdbp_pack_samples would give, and a second launch packs the rows to its
+// words.
 int compress_overlap_save(RcState* r, const float2* raw, int nlines, int stride,
                           const tdbp_chirp& c, float2* out, int out_stride, int flags,
                           void* packed, float* scale, int dtype, hipStream_t s) {
@@ -477,9 +459,11 @@ int compress_overlap_save(RcState* r, const float2* raw, int nlines, int stride,
   hipLaunchKernelGGL(k_os_scales, dim3(1), dim3(kScaleBlock), 0, s, r->lmax, nlines, dtype,
                      r->own, scale);
   if ((st = hip_check(hipGetLastError(), "scale launch"))) return st;
-  const int gx = std::min((kHdr + c.nvalid + kPackBlock - 1) / kPackBlock, 64);
-  hipLaunchKernelGGL(k_os_pack_rows, dim3((unsigned)gx, (unsigned)nlines), dim3(kPackBlock), 0,
-                     s, rows, rows_stride, c.nvalid, (uint32_t*)packed, r->own, scale, dtype);
+  const auto k = dtype == TDBP_CF16   ? k_os_pack_rows<TDBP_CF16>
+                 : dtype == TDBP_CI16 ? k_os_pack_rows<TDBP_CI16>
+                                      : k_os_pack_rows<TDBP_CBF16>;
+  hipLaunchKernelGGL(k, dim3((unsigned)nlines), dim3(kPackBlock), 0, s, rows, rows_stride,
+                     c.nvalid, (uint32_t*)packed, r->own, scale);
   return hip_check(hipGetLastError(), "pack launch");
 }
 

@@ -22,8 +22,8 @@
 //
 // For nnn = 1024 to 8192 (widths 513 ... 8192, the images of these bursts) one
 // kernel does everything: a workgroup of two halves takes an output line, each
-// half upsamples the rows of one image in LDS (the in-place DIF of
-// tdbp_osfft.h, the ramp in its output order, the DIT back), and products,
+// half upsamples the rows of one image in LDS (the in-place pair
+// of tdbp_osfft.h with the ramp between, in digit-reversed order), and products,
 // looks and masks are formed there, with no upsampled rows in HBM
 // (k_xmul_rows at looks 1 x 1, crossmul's default; k_xmul_looks).  Output
 // lines too few for that to fill the chip take one workgroup per row instead
@@ -97,14 +97,10 @@ __global__ void k_up_tables(int n, float2* __restrict__ tab) {
     return;
   }
   const int k = i - os_table_values(n), m = k / (n / 16), t = k - m * (n / 16);
-  int b;
-  if (n == kOsN) {
-    const int p = 2 * (t + (m >> 1) * kOsThreads) + (m & 1);
-    b = (p >> 9) + 16 * ((p >> 5) & 15) + 256 * ((p >> 1) & 15) + 4096 * (p & 1);
-  } else {
-    const int p = 16 * t + m, r = n / 256;
-    b = p / (n / 16) + 16 * ((p / r) & 15) + 256 * (p & (r - 1));
-  }
+  const int p = 16 * t + m, r = n / 256;
+  const int b = n == kOsN
+                    ? (p >> 9) + 16 * ((p >> 5) & 15) + 256 * ((p >> 1) & 15) + 4096 * (p & 1)
+                    : p / (n / 16) + 16 * ((p / r) & 15) + 256 * (p & (r - 1));
   const int ks = b < n / 2 ? b : b - n;
   float s1, c1;
   sincospif((float)ks / (float)n, &s1, &c1);
@@ -137,29 +133,36 @@ template <int N>
 __device__ __forceinline__ void up_transform(const OsTwiddle& w, const float2* __restrict__ ramp,
                                              float2* lds, int t, float2* u) {
   __syncthreads();   // the twiddle tables; the previous row's last LDS reads
+  float2 c[16], T[8];
+  const auto ramps = [&] {
+#pragma unroll
+    for (int m = 0; m < 16; ++m) c[m] = ramp[m * up_threads(N) + t];
+  };
   if constexpr (N == kOsN) {
-    os_dif_regs<up_full(N)>(lds, t, w, u);
+    os_dif_regs(lds, t, w, u, ramps);
   } else {
-    up_dif_first<N>(lds, t, w, u);
+    up_dif_first<N>(lds, t, u);
+    os_tw_last1<N>(w, t, T);   // a stage ahead, as in os_dif_regs
     __syncthreads();
     up_mid<N, false>(lds, t, w, u);
-    __syncthreads();
-    up_dif_last<N>(lds, t, u);
+    ramps();
+    wave_sync();   // as in os_dif_regs: R threads' values
+    up_dif_last<N>(lds, t, T, u);
   }
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
-    const float2 a = u[m], c = ramp[m * up_threads(N) + t];
-    u[m] = make_float2(a.x * c.x - a.y * c.y, -(a.x * c.y + a.y * c.x));   // conj(a c)
+    const float2 a = u[m];
+    u[m] = make_float2(a.x * c[m].x - a.y * c[m].y, -(a.x * c[m].y + a.y * c[m].x));   // conj(a c)
   }
   if constexpr (N == kOsN) {
-    os_dit_regs<up_full(N)>(lds, t, w, u);
+    os_dit_regs(lds, t, w, u);
   } else {
     up_dit_first<N>(lds, t, u);
-    t = os_fresh(t);
-    __syncthreads();
+    os_tw_last2<N>(w, t, T);
+    wave_sync();
     up_mid<N, true>(lds, t, w, u);
     __syncthreads();
-    up_dit_last<N>(lds, t, w, u);
+    up_dit_last<N>(lds, t, T, u);
   }
 #pragma unroll
   for (int k = 0; k < 16; ++k) u[k].y = -u[k].y;
@@ -172,7 +175,7 @@ __global__ void __launch_bounds__(up_threads(N)) __attribute__((amdgpu_waves_per
 k_up_fused(const float2* __restrict__ img, int na, int row0, float scale,
            const float2* __restrict__ tab, float2* __restrict__ up) {
   __shared__ float2 lds[up_lds(N)];
-  __shared__ float2 twl[os_mid_values(N)];
+  __shared__ float2 twl[os_lds_values(N)];
   const OsTwiddle w = os_twiddles_lds<N>(twl, tab);
   const int t = threadIdx.x, i = blockIdx.x;
   float2 v[16];
@@ -252,10 +255,11 @@ __global__ void k_xmul(const float2* __restrict__ up1, const float2* __restrict_
 // values and odd samples of the columns it takes and hands the other half's
 // over through LDS; then per column the sum over the sample pair of
 // up1 conj(up2), the amplitudes and the mask, as k_xmul computes them for one
-// row and one column -- each image read once, no upsampled batch in HBM.  VALU
-// issue bounds it (the transforms' butterflies and twiddles), close above HBM:
-// 13500 x 4000 0.50 ms, 3.5 TB/s; 3000 x 1800 57 us and 3000 x 4400 278 us
-// (366 and 840 us through rocFFT).
+// row and one column -- each image read once, no upsampled batch in HBM.  Vector
+// issue and LDS (the transforms' butterflies and exchanges) bound it, close above
+// HBM: 13500 x 4000 0.47 ms, 3.7 TB/s (0.52 ms with twiddle products apart from
+// the butterflies and a barrier between all stages); 3000 x 1800 55 us and 3000 x
+// 4400 235 us (366 and 840 us through rocFFT).
 template <int N>
 __global__ void __launch_bounds__(2 * up_threads(N)) __attribute__((amdgpu_waves_per_eu(4)))
 k_xmul_rows(const float2* __restrict__ img1, const float2* __restrict__ img2, int na,
@@ -263,7 +267,7 @@ k_xmul_rows(const float2* __restrict__ img1, const float2* __restrict__ img2, in
             float2* __restrict__ amp) {
   constexpr int kT = up_threads(N);
   __shared__ float2 lds[2][up_lds(N)];
-  __shared__ float2 twl[os_mid_values(N)];
+  __shared__ float2 twl[os_lds_values(N)];
   const OsTwiddle w = os_twiddles_lds<N>(twl, tab);
   const int T = threadIdx.x, h = T / kT, t = T % kT;   // h wave-uniform
   const int r = blockIdx.x;
@@ -323,9 +327,9 @@ k_xmul_rows(const float2* __restrict__ img1, const float2* __restrict__ img2, in
 // sums then lie in LDS by column, and thread after thread takes an output
 // column: its looksac sums, and the even samples and the mask from the image
 // rows themselves (read for the second time, mostly from the caches).  The
-// transforms bound it as they do k_xmul_rows: 5403 x 1789 at 4 x 2 0.11 ms, where
+// transforms bound it as they do k_xmul_rows: 5403 x 1789 at 4 x 2 0.105 ms, where
 // rocFFT batches of 512 rows, five launches and four passes over HBM each, took
-// 0.69 ms; 11000 x 4000 at 4 x 2 0.48 ms against 1.27 ms with the upsampled rows
+// 0.69 ms; 11000 x 4000 at 4 x 2 0.46 ms against 1.27 ms with the upsampled rows
 // in HBM.
 template <int N>
 __global__ void __launch_bounds__(2 * up_threads(N)) __attribute__((amdgpu_waves_per_eu(4)))
@@ -334,7 +338,7 @@ k_xmul_looks(const float2* __restrict__ img1, const float2* __restrict__ img2, i
              float2* __restrict__ amp) {
   constexpr int kT = up_threads(N);
   __shared__ __align__(16) float2 lds[2][up_lds(N)];
-  __shared__ float2 twl[os_mid_values(N)];
+  __shared__ float2 twl[os_lds_values(N)];
   static_assert(sizeof lds >= sizeof(float4) * N, "the columns' sums fit the transforms' LDS");
   const OsTwiddle w = os_twiddles_lds<N>(twl, tab);
   const int T = threadIdx.x, h = T / kT;   // h wave-uniform

@@ -2,19 +2,28 @@
 // compression (overlap-save blocks of one echo line, tdbp_range.hip), shared
 // by the device kernels and a host check.
 //
-// In place, mixed radix 16 x 16 x 16 x 2.  The forward transform of a block
-// runs decimation in frequency (DIF): stage (R, s) with L = R s takes, in
-// every L-point sub-block at base b and for j < s, the values b + j + s r (r
-// < R), an R-point DFT, times w^((N/L) j k) (w = e^{-2 pi i/N}), back to b +
-// j + s k.  Stages (16, 512), (16, 32), (16, 2), (2, 1) leave X[drev(p)] at
-// position p, drev(p) = d0 + 16 d1 + 256 d2 + 4096 d3 for p = 512 d0 + 32 d1
-// + 2 d2 + d3.  The second transform runs decimation in time (DIT) on that
-// order: the same stages in reverse, each twiddling its inputs by
-// w^((N/L) j r) before the DFT, from values in digit-reversed order to the
-// forward transform in natural order.  A product of two DIF outputs position
-// by position is the product of the spectra, so a convolution needs no
-// reordering at all.  Forward sign e^{-2 pi i nk/N}; the unnormalised
+// In place, mixed radix 16 x 16 x 16 x 2.  Stage (R, s) takes, in every
+// sub-block of R s values at base b and for j < s, the values b + j + s r (r <
+// R) times t^r, an R-point DFT, back to b + j + s k.
+// The first transform of a block (natural order in) runs stages (16, 512),
+// (16, 32), (16, 2), (2, 1).  It splits the polynomial of the values, modulo
+// x^N - 1 at first, into its remainders: a sub-block whose digits so far are d0,
+// d1 .. stands for the bins K = d0 + 16 d1 + .. modulo 16^stage, and t = w^(s K)
+// (w = e^{-2 pi i/N}), the same for all its butterflies, 1 in the first stage.
+// Position p = 512 d0 + 32 d1 + 2 d2 + d3 ends with bin drev(p) = d0 + 16 d1 +
+// 256 d2 + 4096 d3.  (This order out of natural order in is that of decimation
+// in frequency, whose twiddles follow the butterflies; here they precede them.)
+// The second transform runs decimation in time (DIT) on that order: the same
+// stages in reverse with t = w^(N/(R s) j), from values in digit-reversed order
+// to the forward transform in natural order.  A product of two outputs of the
+// first, position by position, is the product of the spectra, so a convolution
+// needs no reordering at all.  Forward sign e^{-2 pi i nk/N}; the unnormalised
 // inverse of y is conj(FFT(conj(y))).
+// Twiddles before the butterflies go into them: a + u b is two FMAs a component
+// and a - u b = 2 a - (a + u b) a third, so a radix-16 stage is 32 butterflies of
+// six FMAs, 192 instructions, where the DFT and then (or first) fifteen twiddle
+// products, nine of them formed as products, took 272; the first stage of either
+// transform has none.  The kernels are bound by vector issue (93 % busy).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -28,8 +37,8 @@ namespace tdbp {
 constexpr int kOsN = 8192;          // transform length
 // Threads of the device transforms: one radix-16 butterfly per thread and
 // stage; thread t holds values t + kOsThreads m (m < 16) of the block in
-// natural order, or positions 2 (t + kOsThreads h) + e (m = 2 h + e) in the
-// DIF output order.  Two ~70 KB workgroups fill a CU's LDS: 4 waves per SIMD.
+// natural order, or positions 16 t + m in digit-reversed order.  Two ~70 KB
+// workgroups fill a CU's LDS: 4 waves per SIMD.
 // (1024 threads, radix 8: 0.45 ms per IW burst against 0.40 ms at 512 --
 // spills at 64 VGPRs, and every barrier waits for 16 waves.)
 constexpr int kOsThreads = kOsN / 16;
@@ -90,129 +99,190 @@ TDBP_HD void dft16(float2* x) {
 // padding per 32.  Every access of the transforms touches each pair of the
 // 64 LDS banks once per half-wave (the 16-byte reads and writes of stage (2,
 // 1) twice, their minimum): stage (16, 512) 32 consecutive positions,
-// (16, 32) 32 consecutive, (16, 2) pairs 32 apart, (2, 1) 16-byte pairs.  The
-// values of one butterfly sit a compile-time distance apart (544, 34 and 2
-// values; the pairs of (2, 1) 1088 apart across a thread's eight
-// butterflies), so every LDS address is a base plus an immediate.
+// (16, 32) 32 consecutive, (16, 2) pairs 32 apart, (2, 1) 16-byte pairs 16
+// positions apart.  The values of one butterfly sit a compile-time distance
+// apart (544, 34, 2 and 1 values), so every LDS address is a base plus an
+// immediate.
 constexpr int kOsLds = kOsN + 2 * (kOsN / 32);
 TDBP_HD constexpr int os_pad(int p) { return p + 2 * (p >> 5); }
 
-// Twiddles come from tables, every one of them rounded once from FP64: the
-// table of an L-point stage (16, L/16) holds w_L^(j k) at [k L/16 + j] (k < 16,
-// j < L/16), so the lanes of a wave read it in order.  The first stage's table
-// (L = N, 8 N bytes) stays in global memory, where the caches keep it; those of
-// the stages after it (N/16 values, for 8192 points 512 + 32) go to LDS.
-// Fifteen twiddles built as products of four lookups took 60 of a stage's 270
-// vector instructions, and their roundings were the pair's largest error.
-TDBP_HD constexpr int os_mid_values(int n) { return n == kOsN ? n / 16 + n / 256 : n / 16; }
-TDBP_HD constexpr int os_table_values(int n) { return n + os_mid_values(n); }
+// a + u b and a - u b, in place; MI: u times -i in the place of u.
+template <bool MI>
+TDBP_HD void bfly(float2& a, float2& b, float2 u) {
+  const float2 p = MI ? make_float2(fmaf(u.y, b.x, fmaf(u.x, b.y, a.x)),
+                                    fmaf(u.y, b.y, fmaf(-u.x, b.x, a.y)))
+                      : make_float2(fmaf(-u.y, b.y, fmaf(u.x, b.x, a.x)),
+                                    fmaf(u.y, b.x, fmaf(u.x, b.y, a.y)));
+  b = make_float2(fmaf(2.f, a.x, -p.x), fmaf(2.f, a.y, -p.y));
+  a = p;
+}
+
+// In-register forward DFT of R values x_r t^r (R = 2, 4, 8, 16), natural order in
+// and out, from R/2 twiddles T: the powers t^(R/2), .., t^2, t, the last three
+// with their multiples by w8 (t^2) and w16^k, k < 4 (t) -- w16^(k + 4) = -i w16^k
+// and the like need none.  Level by level, the DFTs of 2, 4, .. values.
+template <int R>
+TDBP_HD void dft_tw(float2* x, const float2* T) {
+  if constexpr (R == 2) {
+    bfly<false>(x[0], x[1], T[0]);
+  } else {
+    // DFTs of the even and of the odd values, at t^2; then both together at t.
+    float2 e[R / 2], o[R / 2];
+#pragma unroll
+    for (int r = 0; r < R / 2; ++r) {
+      e[r] = x[2 * r];
+      o[r] = x[2 * r + 1];
+    }
+    dft_tw<R / 2>(e, T);
+    dft_tw<R / 2>(o, T);
+    const float2* u = T + R / 4;
+#pragma unroll
+    for (int k = 0; k < R / 2; ++k) {
+      if (k < R / 4) bfly<false>(e[k], o[k], u[k]);
+      else bfly<true>(e[k], o[k], u[k - R / 4]);
+      x[k] = e[k];
+      x[k + R / 2] = o[k];
+    }
+  }
+}
+// T[i] of dft_tw<R> for t = w_N^e is w_N^m, m the return value: R/2 values, the
+// last R/4 (1 for R = 2) for t itself, those before them for t^2, ..
+TDBP_HD int dft_tw_power(int n, int e, int R, int i) {
+  while (R > 2 && i < R / 4) {
+    e *= 2;
+    R /= 2;
+  }
+  const int k = R > 2 ? i - R / 4 : 0;
+  return (e + k * (n / R)) % n;
+}
+
+// The twiddles of a stage as [i][index], i < 8, so that the lanes of a wave read
+// them in order, every one rounded once from FP64.  Per length N: in global
+// memory (the caches keep them) the last stages of the first transform [8][N/16]
+// (by thread) and of the second [8][N/16] (by j), for 8192 points the third of
+// the first [8][256] (by sub-block); in LDS the second stage of the first [8][16]
+// (by sub-block), stage (16, N/256) of the second (by j), for 8192 points its
+// stage (16, 2) (by j).
+TDBP_HD constexpr int os_at_last2(int n) { return n / 2; }
+TDBP_HD constexpr int os_at_third(int n) { return n; }
+TDBP_HD constexpr int os_at_lds(int n) { return n == kOsN ? n + 2048 : n; }
+constexpr int kOsMid2 = 128;   // in the LDS part: the second transform's stages
+TDBP_HD constexpr int os_at_two(int n) { return kOsMid2 + n / 32; }
+TDBP_HD constexpr int os_lds_values(int n) { return os_at_two(n) + (n == kOsN ? 16 : 0); }
+TDBP_HD constexpr int os_table_values(int n) { return os_at_lds(n) + os_lds_values(n); }
 struct OsTwiddle {
-  const float2* first;
-  const float2* mid;   // 8192 points: the stage (16, 2) at mid + 512
+  const float2* g;   // the length's whole table
+  const float2* s;   // its LDS part
 };
-// Entry i of a length's tables (first, then mid) is w_N^m, m the return value.
+// Bins (modulo 256, 4096) of the sub-blocks after two and three stages.
+TDBP_HD int os_bin2(int b) { return (b >> 4) + 16 * (b & 15); }
+TDBP_HD int os_bin3(int b) { return (b >> 8) + 16 * ((b >> 4) & 15) + 256 * (b & 15); }
+// Entry i of a length's tables is w_n^m, m the return value.
 TDBP_HD int os_table_power(int n, int i) {
-  int step = 1, L = n;   // w_L = w_N^step
-  while (i >= L) {
-    i -= L;
-    L /= 16;
-    step *= 16;
+  const int q = n / 16, r = n / 256;   // threads, radix of the last stage
+  if (i < n / 2) {   // the first transform's last stage
+    const int k = i / q, t = i % q;
+    if (n == kOsN) return os_bin3(8 * t + k) % n;   // radix 2
+    const int h = r / 2;                            // twiddles of one butterfly
+    return dft_tw_power(n, os_bin2((16 / r) * t + k / h), r, k % h);
   }
-  return step * ((i / (L / 16)) * (i % (L / 16)));
+  i -= n / 2;
+  if (i < n / 2) return dft_tw_power(n, i % q, 16, i / q);
+  i -= n / 2;
+  if (n == kOsN) {
+    if (i < 2048) return dft_tw_power(n, 2 * os_bin2(i % 256), 16, i / 256);
+    i -= 2048;
+  }
+  if (i < kOsMid2) return dft_tw_power(n, r * (i % 16), 16, i / 16);
+  i -= kOsMid2;
+  if (i < 8 * r) return dft_tw_power(n, 16 * (i % r), 16, i / r);
+  i -= 8 * r;
+  return dft_tw_power(n, 256 * (i % 2), 16, i / 2);
 }
 
-// v[k] times the twiddles of butterfly j of an L-point stage: all fifteen from
-// the table (FULL), or six and the other nine as products of two of them.  FULL
-// is the more exact (1.6e-7 against 1.8e-7 over a 1024-point round trip, 2.2e-7
-// with four lookups) and about 5 % slower: its loads cost the caches and LDS
-// more than the products cost the vector units.
-template <int L, bool FULL = false>
-TDBP_HD void os_apply(const float2* tab, int j, float2* v) {
-  if constexpr (FULL) {
+// The eight twiddles tab[i N + j].
+template <int N>
+TDBP_HD void os_load_tw(const float2* tab, int j, float2* T) {
 #pragma unroll
-    for (int k = 1; k < 16; ++k) v[k] = c_mul(v[k], tab[k * (L / 16) + j]);
-    return;
-  }
-  float2 lo[4], hi[4];
-#pragma unroll
-  for (int r = 1; r < 4; ++r) {
-    lo[r] = tab[r * (L / 16) + j];
-    hi[r] = tab[4 * r * (L / 16) + j];
-  }
-#pragma unroll
-  for (int k = 1; k < 16; ++k) {
-    const int q = k >> 2, r = k & 3;
-    v[k] = c_mul(v[k], q == 0 ? lo[r] : r == 0 ? hi[q] : c_mul(hi[q], lo[r]));
-  }
+  for (int i = 0; i < 8; ++i) T[i] = tab[i * N + j];
 }
 
-// A radix-16 stage of butterfly j (twiddles of an L-point stage) whose values
-// sit at lds[a0 + STEP r]: read, [DIT: twiddle], DFT, [DIF: twiddle], write back
-// in place.
-template <int L, int STEP, bool DIT, bool FULL>
-TDBP_HD void os_stage16(float2* lds, int a0, int j, const float2* tab, float2* v) {
+// A radix-16 stage whose values sit at lds[a0 + STEP r]: read, DFT with the
+// twiddles T, write back in place.
+template <int STEP>
+TDBP_HD void os_stage16(float2* lds, int a0, const float2* T, float2* v) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = lds[a0 + STEP * r];
-  if constexpr (DIT) os_apply<L, FULL>(tab, j, v);
-  dft16(v);
-  if constexpr (!DIT) os_apply<L, FULL>(tab, j, v);
+  dft_tw<16>(v, T);
 #pragma unroll
   for (int k = 0; k < 16; ++k) lds[a0 + STEP * k] = v[k];
 }
 
+// The twiddles from global memory of thread t: the first transform's third and
+// last stage, the second's last.
+TDBP_HD void os_tw_third(const OsTwiddle& tw, int t, float2* T) {
+  os_load_tw<256>(tw.g + os_at_third(kOsN), t >> 1, T);
+}
+template <int N>
+TDBP_HD void os_tw_last1(const OsTwiddle& tw, int t, float2* T) {
+  os_load_tw<N / 16>(tw.g, t, T);
+}
+template <int N>
+TDBP_HD void os_tw_last2(const OsTwiddle& tw, int t, float2* T) {
+  os_load_tw<N / 16>(tw.g + os_at_last2(N), t, T);
+}
+
 // The stages of thread t.  Stage (16, 512): butterfly t, values t + 512 r,
-// which the thread holds in registers (DIF: from registers; DIT: into them).
-// Stage (16, 32): butterfly j = t mod 32 of sub-block t / 32.  Stage (16, 2):
-// butterfly t mod 2 of sub-block t / 2.  Stage (2, 1): the eight pairs at
-// positions 2 (t + 512 h), held in registers as v[2h], v[2h + 1].
-template <bool FULL = false>
-TDBP_HD void os_dif_first(float2* lds, int t, const OsTwiddle& tw, float2* v) {
+// which the thread holds in registers (first transform: from registers; second:
+// into them).  Stage (16, 32): butterfly j = t mod 32 of sub-block t / 32.
+// Stage (16, 2): butterfly t mod 2 of sub-block t / 2.  Stage (2, 1): the eight
+// pairs at positions 16 t + 2 h, held in registers as v[2h], v[2h + 1].  All but
+// the first of these stay within the 512 positions of 32 threads, so that only
+// stage (16, 512) needs the workgroup's barrier on its other side.
+TDBP_HD void os_dif_first(float2* lds, int t, float2* v) {
   dft16(v);
-  os_apply<kOsN, FULL>(tw.first, t, v);
   float2* q = lds + os_pad(t);
 #pragma unroll
   for (int k = 0; k < 16; ++k) q[544 * k] = v[k];
 }
-template <bool FULL = false>
 TDBP_HD void os_dif_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<512, 34, false, FULL>(lds, 544 * (t >> 5) + (t & 31), t & 31, tw.mid, v);
+  float2 T[8];
+  os_load_tw<16>(tw.s, t >> 5, T);
+  os_stage16<34>(lds, 544 * (t >> 5) + (t & 31), T, v);
 }
-template <bool FULL = false>
-TDBP_HD void os_dif_mid2(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<32, 2, false, FULL>(lds, 34 * (t >> 1) + (t & 1), t & 1, tw.mid + 512, v);
+TDBP_HD void os_dif_mid2(float2* lds, int t, const float2* T, float2* v) {
+  os_stage16<2>(lds, 34 * (t >> 1) + (t & 1), T, v);
 }
-TDBP_HD void os_dif_last(const float2* lds, int t, float2* v) {
-  const float2* q = lds + os_pad(2 * t);
+TDBP_HD void os_dif_last(const float2* lds, int t, const float2* T, float2* v) {
+  const float2* q = lds + os_pad(16 * t);
 #pragma unroll
-  for (int h = 0; h < 8; ++h) {
-    const float2 a = q[1088 * h], b = q[1088 * h + 1];
-    v[2 * h] = c_add(a, b);
-    v[2 * h + 1] = c_sub(a, b);
-  }
+  for (int m = 0; m < 16; ++m) v[m] = q[m];
+#pragma unroll
+  for (int h = 0; h < 8; ++h) bfly<false>(v[2 * h], v[2 * h + 1], T[h]);
 }
 TDBP_HD void os_dit_first(float2* lds, int t, const float2* v) {
-  float2* q = lds + os_pad(2 * t);
+  float2* q = lds + os_pad(16 * t);
 #pragma unroll
   for (int h = 0; h < 8; ++h) {
-    q[1088 * h] = c_add(v[2 * h], v[2 * h + 1]);
-    q[1088 * h + 1] = c_sub(v[2 * h], v[2 * h + 1]);
+    q[2 * h] = c_add(v[2 * h], v[2 * h + 1]);
+    q[2 * h + 1] = c_sub(v[2 * h], v[2 * h + 1]);
   }
 }
-template <bool FULL = false>
 TDBP_HD void os_dit_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<32, 2, true, FULL>(lds, 34 * (t >> 1) + (t & 1), t & 1, tw.mid + 512, v);
+  float2 T[8];
+  os_load_tw<2>(tw.s + os_at_two(kOsN), t & 1, T);
+  os_stage16<2>(lds, 34 * (t >> 1) + (t & 1), T, v);
 }
-template <bool FULL = false>
 TDBP_HD void os_dit_mid2(float2* lds, int t, const OsTwiddle& tw, float2* v) {
-  os_stage16<512, 34, true, FULL>(lds, 544 * (t >> 5) + (t & 31), t & 31, tw.mid, v);
+  float2 T[8];
+  os_load_tw<32>(tw.s + kOsMid2, t & 31, T);
+  os_stage16<34>(lds, 544 * (t >> 5) + (t & 31), T, v);
 }
-template <bool FULL = false>
-TDBP_HD void os_dit_last(const float2* lds, int t, const OsTwiddle& tw, float2* v) {
+TDBP_HD void os_dit_last(const float2* lds, int t, const float2* T, float2* v) {
   const float2* q = lds + os_pad(t);
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = q[544 * r];
-  os_apply<kOsN, FULL>(tw.first, t, v);
-  dft16(v);
+  dft_tw<16>(v, T);
 }
 
 // Host transforms (the check of the device code): the same stages, layout
@@ -226,7 +296,7 @@ struct OsHostTables {
   explicit OsHostTables(const float2* table) {   // w^m of 8192 points
     for (int i = 0; i < os_table_values(N); ++i) v[i] = table[kOsN / N * os_table_power(N, i)];
   }
-  OsTwiddle tw() const { return OsTwiddle{v, v + N}; }
+  OsTwiddle tw() const { return OsTwiddle{v, v + os_at_lds(N)}; }
 };
 inline void os_dif_host(float2* data, const float2* table) {
   const OsHostTables<kOsN> tb(table);
@@ -235,13 +305,18 @@ inline void os_dif_host(float2* data, const float2* table) {
   float2 v[16];
   for (int t = 0; t < kOsThreads; ++t) {
     for (int r = 0; r < 16; ++r) v[r] = data[t + kOsThreads * r];
-    os_dif_first(lds, t, tw, v);
+    os_dif_first(lds, t, v);
   }
   for (int t = 0; t < kOsThreads; ++t) os_dif_mid1(lds, t, tw, v);
-  for (int t = 0; t < kOsThreads; ++t) os_dif_mid2(lds, t, tw, v);
+  float2 T[8];
   for (int t = 0; t < kOsThreads; ++t) {
-    os_dif_last(lds, t, v);
-    for (int m = 0; m < 16; ++m) data[2 * (t + kOsThreads * (m >> 1)) + (m & 1)] = v[m];
+    os_tw_third(tw, t, T);
+    os_dif_mid2(lds, t, T, v);
+  }
+  for (int t = 0; t < kOsThreads; ++t) {
+    os_tw_last1<kOsN>(tw, t, T);
+    os_dif_last(lds, t, T, v);
+    for (int m = 0; m < 16; ++m) data[16 * t + m] = v[m];
   }
   delete[] lds;
 }
@@ -251,13 +326,15 @@ inline void os_dit_host(float2* data, const float2* table) {
   float2* lds = new float2[kOsLds];
   float2 v[16];
   for (int t = 0; t < kOsThreads; ++t) {
-    for (int m = 0; m < 16; ++m) v[m] = data[2 * (t + kOsThreads * (m >> 1)) + (m & 1)];
+    for (int m = 0; m < 16; ++m) v[m] = data[16 * t + m];
     os_dit_first(lds, t, v);
   }
   for (int t = 0; t < kOsThreads; ++t) os_dit_mid1(lds, t, tw, v);
   for (int t = 0; t < kOsThreads; ++t) os_dit_mid2(lds, t, tw, v);
+  float2 T[8];
   for (int t = 0; t < kOsThreads; ++t) {
-    os_dit_last(lds, t, tw, v);
+    os_tw_last2<kOsN>(tw, t, T);
+    os_dit_last(lds, t, T, v);
     for (int k = 0; k < 16; ++k) data[t + kOsThreads * k] = v[k];
   }
   delete[] lds;
@@ -274,91 +351,85 @@ inline void os_dit_host(float2* data, const float2* table) {
 // (16, N/16) and (R, 1) touch each bank pair once per half-wave, stage (16, R)
 // twice (no additive padding clears all three, a host simulation shows).
 constexpr int kUpN = 4096;
-// Lengths with every twiddle from the table: those where the interferograms'
-// errors would else exceed a library transform's (2048 points, looks 4 x 2:
-// 1.1e-7 against 1.0e-7).
-TDBP_HD constexpr bool up_full(int n) { return n != kUpN; }
 TDBP_HD constexpr int up_threads(int n) { return n / 16; }
 TDBP_HD constexpr int up_lds(int n) { return n == kOsN ? kOsLds : n + n / 32; }
 TDBP_HD constexpr int up_pad(int p) { return p + (p >> 5); }
 
-// In-register forward DFT of 8 points, natural order in and out (n = 2 n1 +
-// n2, k = k1 + 4 k2).
-TDBP_HD void dft8(float2* x) {
-  float2 a0 = x[0], a1 = x[2], a2 = x[4], a3 = x[6];
-  float2 b0 = x[1], b1 = x[3], b2 = x[5], b3 = x[7];
-  dft4(a0, a1, a2, a3);
-  dft4(b0, b1, b2, b3);
-  b1 = c_w8(b1);
-  b2 = c_mni(b2);
-  b3 = c_w8_3(b3);
-  x[0] = c_add(a0, b0);
-  x[1] = c_add(a1, b1);
-  x[2] = c_add(a2, b2);
-  x[3] = c_add(a3, b3);
-  x[4] = c_sub(a0, b0);
-  x[5] = c_sub(a1, b1);
-  x[6] = c_sub(a2, b2);
-  x[7] = c_sub(a3, b3);
-}
-
-// The R-point DFTs of the 16/R sub-blocks in v.
+// The plain R-point DFTs of the 16/R sub-blocks in v.
 template <int R>
-TDBP_HD void up_dft_last(float2* v) {
+TDBP_HD void up_dft_plain(float2* v) {
   if constexpr (R == 16) {
     dft16(v);
-  } else {
+  } else if constexpr (R == 4) {
 #pragma unroll
-    for (int q = 0; q < 16; q += R) {
-      if constexpr (R == 8) dft8(v + q);
-      else dft4(v[q], v[q + 1], v[q + 2], v[q + 3]);
+    for (int q = 0; q < 16; q += 4) dft4(v[q], v[q + 1], v[q + 2], v[q + 3]);
+  } else {   // 8 points: n = 2 n1 + n2, k = k1 + 4 k2
+#pragma unroll
+    for (int q = 0; q < 16; q += 8) {
+      float2* x = v + q;
+      float2 a[4], b[4];
+      for (int k = 0; k < 4; ++k) {
+        a[k] = x[2 * k];
+        b[k] = x[2 * k + 1];
+      }
+      dft4(a[0], a[1], a[2], a[3]);
+      dft4(b[0], b[1], b[2], b[3]);
+      b[1] = c_w8(b[1]);
+      b[2] = c_mni(b[2]);
+      b[3] = c_w8_3(b[3]);
+      for (int k = 0; k < 4; ++k) {
+        x[k] = c_add(a[k], b[k]);
+        x[k + 4] = c_sub(a[k], b[k]);
+      }
     }
   }
 }
 
 template <int N>
-TDBP_HD void up_dif_first(float2* lds, int t, const OsTwiddle& tw, float2* v) {
+TDBP_HD void up_dif_first(float2* lds, int t, float2* v) {
   dft16(v);
-  os_apply<N, up_full(N)>(tw.first, t, v);
   float2* q = lds + up_pad(t);
 #pragma unroll
   for (int k = 0; k < 16; ++k) q[up_pad(N / 16) * k] = v[k];
 }
-// Stage (16, R) of butterfly t mod R of sub-block t / R.
+// Stage (16, R) of butterfly t mod R of sub-block t / R, of the second transform
+// (DIT) or the first.
 template <int N, bool DIT>
 TDBP_HD void up_mid(float2* lds, int t, const OsTwiddle& tw, float2* v) {
   constexpr int R = N / 256;
-  const int j = t & (R - 1);
-  float2* q = lds + up_pad(N / 16) * (t / R) + j;
+  const int j = t & (R - 1), b = t / R;
+  float2* q = lds + up_pad(N / 16) * b + j;
+  float2 T[8];
+  if constexpr (DIT) os_load_tw<R>(tw.s + kOsMid2, j, T);
+  else os_load_tw<16>(tw.s, b, T);
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = q[up_pad(R * r)];
-  if constexpr (DIT) os_apply<N / 16, up_full(N)>(tw.mid, j, v);
-  dft16(v);
-  if constexpr (!DIT) os_apply<N / 16, up_full(N)>(tw.mid, j, v);
+  dft_tw<16>(v, T);
 #pragma unroll
   for (int k = 0; k < 16; ++k) q[up_pad(R * k)] = v[k];
 }
 template <int N>
-TDBP_HD void up_dif_last(const float2* lds, int t, float2* v) {
+TDBP_HD void up_dif_last(const float2* lds, int t, const float2* T, float2* v) {
+  constexpr int R = N / 256;
   const float2* q = lds + up_pad(16 * t);
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = q[r];
-  up_dft_last<N / 256>(v);
+#pragma unroll
+  for (int k = 0; k < 16 / R; ++k) dft_tw<R>(v + R * k, T + R / 2 * k);
 }
 template <int N>
 TDBP_HD void up_dit_first(float2* lds, int t, float2* v) {
-  up_dft_last<N / 256>(v);
+  up_dft_plain<N / 256>(v);
   float2* q = lds + up_pad(16 * t);
 #pragma unroll
   for (int k = 0; k < 16; ++k) q[k] = v[k];
 }
 template <int N>
-TDBP_HD void up_dit_last(const float2* lds, int t, const OsTwiddle& tw, float2* v) {
+TDBP_HD void up_dit_last(const float2* lds, int t, const float2* T, float2* v) {
   const float2* q = lds + up_pad(t);
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = q[up_pad(N / 16) * r];
-  os_apply<N, up_full(N)>(tw.first, t, v);
-  dft16(v);
+  dft_tw<16>(v, T);
 }
 
 // Host transforms of these lengths, as os_dif_host / os_dit_host.
@@ -371,11 +442,13 @@ inline void up_dif_host(float2* data, const float2* table) {
   float2 v[16];
   for (int t = 0; t < kT; ++t) {
     for (int r = 0; r < 16; ++r) v[r] = data[t + kT * r];
-    up_dif_first<N>(lds, t, tw, v);
+    up_dif_first<N>(lds, t, v);
   }
   for (int t = 0; t < kT; ++t) up_mid<N, false>(lds, t, tw, v);
   for (int t = 0; t < kT; ++t) {
-    up_dif_last<N>(lds, t, v);
+    float2 T[8];
+    os_tw_last1<N>(tw, t, T);
+    up_dif_last<N>(lds, t, T, v);
     for (int m = 0; m < 16; ++m) data[16 * t + m] = v[m];
   }
   delete[] lds;
@@ -393,18 +466,21 @@ inline void up_dit_host(float2* data, const float2* table) {
   }
   for (int t = 0; t < kT; ++t) up_mid<N, true>(lds, t, tw, v);
   for (int t = 0; t < kT; ++t) {
-    up_dit_last<N>(lds, t, tw, v);
+    float2 T[8];
+    os_tw_last2<N>(tw, t, T);
+    up_dit_last<N>(lds, t, T, v);
     for (int k = 0; k < 16; ++k) data[t + kT * k] = v[k];
   }
   delete[] lds;
 }
 
 // The tables of N points on the device (os_table_values(N) values), and the ones
-// that go to LDS copied into `twl` (os_mid_values(N) values); a barrier must
+// that go to LDS copied into `twl` (os_lds_values(N) values); a barrier must
 // follow before any transform reads them.
 template <int N>
 __device__ __forceinline__ OsTwiddle os_twiddles_lds(float2* twl, const float2* __restrict__ table) {
-  for (int i = threadIdx.x; i < os_mid_values(N); i += blockDim.x) twl[i] = table[N + i];
+  for (int i = threadIdx.x; i < os_lds_values(N); i += blockDim.x)
+    twl[i] = table[os_at_lds(N) + i];
   return OsTwiddle{table, twl};
 }
 
@@ -416,44 +492,58 @@ __device__ __forceinline__ float2 os_table_entry(int n, int i) {
   return make_float2((float)cs, (float)sn);
 }
 
-// The index again, as a value the compiler cannot connect with the first: the
-// last stage's twiddles are the first's, and keeping them in 30 registers from
-// one to the other would spill what the stages between need.
+// Orders the LDS accesses of a wave's lanes (which the hardware executes in
+// order): between stages whose values stay within a wave.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Device, first transform by kOsThreads threads, t their index (whole waves from
+// a multiple of 64 on): v[m] holds value t + kOsThreads m of the block on entry
+// and position 16 t + m of the output on return.  The LDS twiddles must be
+// ordered before the call.  Twiddles from global memory are loaded a stage ahead;
+// so is what `ahead` loads for the caller, before the last stage.  On return
+// every thread's remaining LDS positions are its wave's own (os_dit_regs may
+// follow without a barrier).
+template <class F>
+__device__ __forceinline__ void os_dif_regs(float2* lds, int t, const OsTwiddle& tw, float2* v,
+                                            F&& ahead) {
+  float2 T[8], U[8];
+  os_dif_first(lds, t, v);
+  os_tw_third(tw, t, T);
+  __syncthreads();
+  os_dif_mid1(lds, t, tw, v);
+  os_tw_last1<kOsN>(tw, t, U);
+  wave_sync();
+  os_dif_mid2(lds, t, T, v);
+  ahead();
+  wave_sync();
+  os_dif_last(lds, t, U, v);
+}
+
+// Device, second transform (DIT): v in the first's output order on entry, value
+// t + kOsThreads m of the forward transform on return.  LDS positions other
+// threads may still read must not be needed by the caller afterwards.
+__device__ __forceinline__ void os_dit_regs(float2* lds, int t, const OsTwiddle& tw,
+                                            float2* v) {
+  float2 T[8];
+  os_dit_first(lds, t, v);
+  wave_sync();
+  os_dit_mid1(lds, t, tw, v);
+  os_tw_last2<kOsN>(tw, t, T);
+  wave_sync();
+  os_dit_mid2(lds, t, tw, v);
+  __syncthreads();
+  os_dit_last(lds, t, T, v);
+}
+
+// An index as a value the compiler cannot connect with the one it was made from:
+// what is computed from it is not kept from one use to another.
 __device__ __forceinline__ int os_fresh(int t) {
   asm volatile("" : "+v"(t));
   return t;
-}
-
-// Device DIF by kOsThreads threads, t their index: v[m] holds value t +
-// kOsThreads m of the block on entry and position 2 (t + kOsThreads (m / 2)) +
-// m mod 2 of the output on return.  The twiddle tables must be ordered
-// before the call.  On return every thread's remaining LDS positions are its
-// own (os_dit_regs may follow without a barrier).
-template <bool FULL = false>
-__device__ __forceinline__ void os_dif_regs(float2* lds, int t, const OsTwiddle& tw,
-                                            float2* v) {
-  os_dif_first<FULL>(lds, t, tw, v);
-  __syncthreads();
-  os_dif_mid1<FULL>(lds, t, tw, v);
-  __syncthreads();
-  os_dif_mid2<FULL>(lds, t, tw, v);
-  __syncthreads();
-  os_dif_last(lds, t, v);
-}
-
-// Device DIT: v in the DIF output order on entry, value t + kOsThreads m of the forward transform on return.  LDS positions other
-// threads may still read must not be needed by the caller afterwards.
-template <bool FULL = false>
-__device__ __forceinline__ void os_dit_regs(float2* lds, int t, const OsTwiddle& tw,
-                                            float2* v) {
-  os_dit_first(lds, t, v);
-  t = os_fresh(t);
-  __syncthreads();
-  os_dit_mid1<FULL>(lds, t, tw, v);
-  __syncthreads();
-  os_dit_mid2<FULL>(lds, t, tw, v);
-  __syncthreads();
-  os_dit_last<FULL>(lds, t, tw, v);
 }
 
 }  // namespace tdbp

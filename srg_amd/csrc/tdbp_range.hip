@@ -175,20 +175,20 @@ __global__ void k_os_twiddles(float2* __restrict__ tw) {
 }
 
 // Forward transform of one 8192-point vector (the reference function's
-// spectrum), one workgroup, in place: natural order in, the DIF output order
-// out (position p holds bin drev(p)), which is the order k_rc_os multiplies
-// its own DIF outputs in.
+// spectrum), one workgroup, in place: natural order in, digit-reversed order
+// out, position 16 t + m (bin drev(16 t + m)) at [m kOsThreads + t], as the
+// threads of k_rc_os multiply their own first transform's outputs with it.
 __global__ void __launch_bounds__(kOsThreads) k_os_spectrum(float2* __restrict__ v,
                                                              const float2* __restrict__ tw) {
   __shared__ float2 lds[kOsLds];
-  __shared__ float2 twl[os_mid_values(kOsN)];
+  __shared__ float2 twl[os_lds_values(kOsN)];
   const OsTwiddle w = os_twiddles_lds<kOsN>(twl, tw);
   const int t = threadIdx.x;
   float2 x[16];
   for (int m = 0; m < 16; ++m) x[m] = v[t + m * kOsThreads];
   __syncthreads();   // the twiddle tables; every read of v is done
-  os_dif_regs(lds, t, w, x);
-  for (int m = 0; m < 16; ++m) v[2 * (t + (m >> 1) * kOsThreads) + (m & 1)] = x[m];
+  os_dif_regs(lds, t, w, x, [] {});
+  for (int m = 0; m < 16; ++m) v[m * kOsThreads + t] = x[m];
 }
 
 // Block b of line l: outputs k0 + k, k < M = 8192 - npts + 1, k0 = b M, of
@@ -201,14 +201,17 @@ __global__ void __launch_bounds__(kOsThreads) k_os_spectrum(float2* __restrict__
 // header samples) and, when lmax is given, the largest |component| of the
 // block's outputs into lmax[l] (FP32 bits; max as fmaxf takes it, so NaN is
 // passed over as the pack kernel does).
-// Two workgroups per CU (LDS 2 x 71 KB): 4 waves per SIMD.
+// Two workgroups per CU (LDS 2 x 73 KB): 4 waves per SIMD.  Vector issue (1530
+// instructions a wave, 76 % busy) and LDS (about as busy) bound it together: an
+// IW burst's 1500 lines in 0.21 ms, as with 1950 vector instructions (93 % busy)
+// before the twiddles went into the butterflies.
 __global__ void __launch_bounds__(kOsThreads)
 __attribute__((amdgpu_waves_per_eu(4)))
 k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int npts, int nvalid,
         const float2* __restrict__ spec, const float2* __restrict__ tw,
         float2* __restrict__ out, int out_stride, int zero_header, unsigned* __restrict__ lmax) {
   __shared__ float2 lds[kOsLds];
-  __shared__ float2 twl[os_mid_values(kOsN)];
+  __shared__ float2 twl[os_lds_values(kOsN)];
   // Work item q = (line, block), line-major, dealt so that XCD x (blocks x,
   // x + 8, ...) takes the x-th eighth of the items in order: the blocks of a
   // line, whose echo windows overlap by npts - 1 samples, share one L2.
@@ -223,8 +226,7 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
   const OsTwiddle w = os_twiddles_lds<kOsN>(twl, tw);
   const float2* echo = raw + (size_t)l * stride + kHdr;
   // thread t holds values t + kOsThreads m, m < 16, of the block (natural
-  // order), between the transforms positions 2 (t + kOsThreads (m / 2)) +
-  // m mod 2 (the DIF output order)
+  // order), between the transforms positions 16 t + m (digit-reversed order)
   const int t = threadIdx.x;
   float2 v[16];
 #pragma unroll
@@ -233,11 +235,13 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
     v[m] = k0 + n < nsamps ? echo[k0 + n] : make_float2(0.f, 0.f);
   }
   __syncthreads();   // the twiddle tables
-  os_dif_regs(lds, t, w, v);
+  float2 sp[16];
+  os_dif_regs(lds, t, w, v, [&] {
 #pragma unroll
-  for (int m = 0; m < 16; ++m)
-    v[m] = c_mul(make_float2(v[m].x, -v[m].y),
-                 spec[2 * (t + (m >> 1) * kOsThreads) + (m & 1)]);
+    for (int m = 0; m < 16; ++m) sp[m] = spec[m * kOsThreads + t];
+  });
+#pragma unroll
+  for (int m = 0; m < 16; ++m) v[m] = c_mul(make_float2(v[m].x, -v[m].y), sp[m]);
   os_dit_regs(lds, t, w, v);
   const int kend = min(M, nvalid - k0);
   float mx = 0.f;

@@ -134,9 +134,10 @@ __device__ __forceinline__ void up_transform(const OsTwiddle& w, const float2* _
                                              float2* lds, int t, float2* u) {
   __syncthreads();   // the twiddle tables; the previous row's last LDS reads
   float2 c[16], T[8];
+  const int t2 = N == kOsN ? os_mid_thread(t) : t;   // holds positions 16 t2 + m between
   const auto ramps = [&] {
 #pragma unroll
-    for (int m = 0; m < 16; ++m) c[m] = ramp[m * up_threads(N) + t];
+    for (int m = 0; m < 16; ++m) c[m] = ramp[m * up_threads(N) + t2];
   };
   if constexpr (N == kOsN) {
     os_dif_regs(lds, t, w, u, ramps);

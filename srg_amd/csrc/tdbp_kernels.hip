@@ -2869,7 +2869,7 @@ inline unsigned blocks_for(size_t n, int bs) {
 // ms without it; FP64 on 800 x 800 (3.4 rounds) 0.56 with, 0.64 without.  Split
 // tiles never take it: most of them hold no work, and an empty one costs an
 // atomic of 0.2 us on its counter (1200 x 2638 samples onto 737 x 409 pixels,
-// 4810 tiles: 0.31 -> 0.13 ms).
+// 4810 tiles: 0.31 -> 0.12 ms).
 template <void (*K)(BurstDev)>
 hipError_t persistent_launch(const BurstDev& b, hipStream_t s) {
   if (!b.counters) return hipErrorInvalidValue;

@@ -95,16 +95,13 @@ TDBP_HD void dft16(float2* x) {
   for (int k = 0; k < 16; ++k) x[k] = y[k];
 }
 
-// LDS layout: position p at os_pad(p) = p + 2 floor(p / 32), two values of
-// padding per 32.  Every access of the transforms touches each pair of the
-// 64 LDS banks once per half-wave (the 16-byte reads and writes of stage (2,
-// 1) twice, their minimum): stage (16, 512) 32 consecutive positions,
-// (16, 32) 32 consecutive, (16, 2) pairs 32 apart, (2, 1) 16-byte pairs 16
-// positions apart.  The values of one butterfly sit a compile-time distance
-// apart (544, 34, 2 and 1 values), so every LDS address is a base plus an
-// immediate.
-constexpr int kOsLds = kOsN + 2 * (kOsN / 32);
-TDBP_HD constexpr int os_pad(int p) { return p + 2 * (p >> 5); }
+// LDS layout: position p at os_pad(p) = p + floor(p / 32).  Every access of the
+// transforms then touches each pair of the 64 LDS banks once per half-wave: stages
+// (16, 512) and (16, 32) 32 consecutive positions, (16, 2) 32 positions 32 apart.
+// The values of one butterfly sit a compile-time distance apart (528, 33 and 2
+// values), so every LDS address is a base plus an immediate.
+constexpr int kOsLds = kOsN + kOsN / 32;
+TDBP_HD constexpr int os_pad(int p) { return p + (p >> 5); }
 
 // a + u b and a - u b, in place; MI: u times -i in the place of u.
 template <bool MI>
@@ -207,15 +204,23 @@ TDBP_HD void os_load_tw(const float2* tab, int j, float2* T) {
   for (int i = 0; i < 8; ++i) T[i] = tab[i * N + j];
 }
 
-// A radix-16 stage whose values sit at lds[a0 + STEP r]: read, DFT with the
-// twiddles T, write back in place.
+// The values of a radix-16 stage, at lds[a0 + STEP r].
 template <int STEP>
-TDBP_HD void os_stage16(float2* lds, int a0, const float2* T, float2* v) {
+TDBP_HD void os_read16(const float2* lds, int a0, float2* v) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = lds[a0 + STEP * r];
-  dft_tw<16>(v, T);
+}
+template <int STEP>
+TDBP_HD void os_write16(float2* lds, int a0, const float2* v) {
 #pragma unroll
   for (int k = 0; k < 16; ++k) lds[a0 + STEP * k] = v[k];
+}
+// The stage: read, DFT with the twiddles T, write back in place.
+template <int STEP>
+TDBP_HD void os_stage16(float2* lds, int a0, const float2* T, float2* v) {
+  os_read16<STEP>(lds, a0, v);
+  dft_tw<16>(v, T);
+  os_write16<STEP>(lds, a0, v);
 }
 
 // The twiddles from global memory of thread t: the first transform's third and
@@ -237,51 +242,57 @@ TDBP_HD void os_tw_last2(const OsTwiddle& tw, int t, float2* T) {
 // into them).  Stage (16, 32): butterfly j = t mod 32 of sub-block t / 32.
 // Stage (16, 2): butterfly t mod 2 of sub-block t / 2.  Stage (2, 1): the eight
 // pairs at positions 16 t + 2 h, held in registers as v[2h], v[2h + 1].  All but
-// the first of these stay within the 512 positions of 32 threads, so that only
+// the first of these stay within the 1024 positions of a wave (stages (16, 2) and
+// (2, 1) with their threads in another order there, os_mid_thread), so that only
 // stage (16, 512) needs the workgroup's barrier on its other side.
 TDBP_HD void os_dif_first(float2* lds, int t, float2* v) {
   dft16(v);
   float2* q = lds + os_pad(t);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) q[544 * k] = v[k];
+  for (int k = 0; k < 16; ++k) q[528 * k] = v[k];
 }
 TDBP_HD void os_dif_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
   float2 T[8];
   os_load_tw<16>(tw.s, t >> 5, T);
-  os_stage16<34>(lds, 544 * (t >> 5) + (t & 31), T, v);
+  os_stage16<33>(lds, 528 * (t >> 5) + (t & 31), T, v);
 }
 TDBP_HD void os_dif_mid2(float2* lds, int t, const float2* T, float2* v) {
-  os_stage16<2>(lds, 34 * (t >> 1) + (t & 1), T, v);
+  os_stage16<2>(lds, 33 * (t >> 1) + (t & 1), T, v);
 }
-TDBP_HD void os_dif_last(const float2* lds, int t, const float2* T, float2* v) {
-  const float2* q = lds + os_pad(16 * t);
-#pragma unroll
-  for (int m = 0; m < 16; ++m) v[m] = q[m];
+TDBP_HD void os_dif_pairs(const float2* T, float2* v) {
 #pragma unroll
   for (int h = 0; h < 8; ++h) bfly<false>(v[2 * h], v[2 * h + 1], T[h]);
 }
-TDBP_HD void os_dit_first(float2* lds, int t, const float2* v) {
-  float2* q = lds + os_pad(16 * t);
+TDBP_HD void os_dif_last(const float2* lds, int t, const float2* T, float2* v) {
+  os_read16<1>(lds, os_pad(16 * t), v);
+  os_dif_pairs(T, v);
+}
+TDBP_HD void os_dit_pairs(float2* v) {
 #pragma unroll
   for (int h = 0; h < 8; ++h) {
-    q[2 * h] = c_add(v[2 * h], v[2 * h + 1]);
-    q[2 * h + 1] = c_sub(v[2 * h], v[2 * h + 1]);
+    const float2 a = v[2 * h], b = v[2 * h + 1];
+    v[2 * h] = c_add(a, b);
+    v[2 * h + 1] = c_sub(a, b);
   }
+}
+TDBP_HD void os_dit_first(float2* lds, int t, float2* v) {
+  os_dit_pairs(v);
+  os_write16<1>(lds, os_pad(16 * t), v);
 }
 TDBP_HD void os_dit_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
   float2 T[8];
   os_load_tw<2>(tw.s + os_at_two(kOsN), t & 1, T);
-  os_stage16<2>(lds, 34 * (t >> 1) + (t & 1), T, v);
+  os_stage16<2>(lds, 33 * (t >> 1) + (t & 1), T, v);
 }
 TDBP_HD void os_dit_mid2(float2* lds, int t, const OsTwiddle& tw, float2* v) {
   float2 T[8];
   os_load_tw<32>(tw.s + kOsMid2, t & 31, T);
-  os_stage16<34>(lds, 544 * (t >> 5) + (t & 31), T, v);
+  os_stage16<33>(lds, 528 * (t >> 5) + (t & 31), T, v);
 }
 TDBP_HD void os_dit_last(const float2* lds, int t, const float2* T, float2* v) {
   const float2* q = lds + os_pad(t);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) v[r] = q[544 * r];
+  for (int r = 0; r < 16; ++r) v[r] = q[528 * r];
   dft_tw<16>(v, T);
 }
 
@@ -500,27 +511,70 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The thread of stages (16, 2) and (2, 1) that thread t is on the device: lanes r
+// and r + 32 of a wave are a pair 2 q, 2 q + 1.
+__device__ __forceinline__ int os_mid_thread(int t) {
+  return (t & ~63) | ((t & 31) << 1) | ((t >> 5) & 1);
+}
+// Between those stages the values change hands within the pairs, position 32 q +
+// j + 2 k of thread 2 q + j as v[k] against 32 q + 16 j + m as v[m]: the second
+// half of the lower lane's values against the first half of the upper's, which
+// v_permlane32_swap does for two registers at once, in the place of an LDS write
+// and read (a third of the transforms' LDS cycles).
+__device__ __forceinline__ void pair_swap(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                  false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void pairs_gather(float2* v) {
+  float2 w[16];
+#pragma unroll
+  for (int h = 0; h < 8; ++h) {
+    w[2 * h] = v[h];
+    w[2 * h + 1] = v[h + 8];
+    pair_swap(w[2 * h].x, w[2 * h + 1].x);
+    pair_swap(w[2 * h].y, w[2 * h + 1].y);
+  }
+#pragma unroll
+  for (int m = 0; m < 16; ++m) v[m] = w[m];
+}
+__device__ __forceinline__ void pairs_scatter(float2* v) {
+  float2 w[16];
+#pragma unroll
+  for (int h = 0; h < 8; ++h) {
+    w[h] = v[2 * h];
+    w[h + 8] = v[2 * h + 1];
+    pair_swap(w[h].x, w[h + 8].x);
+    pair_swap(w[h].y, w[h + 8].y);
+  }
+#pragma unroll
+  for (int m = 0; m < 16; ++m) v[m] = w[m];
+}
+
 // Device, first transform by kOsThreads threads, t their index (whole waves from
 // a multiple of 64 on): v[m] holds value t + kOsThreads m of the block on entry
-// and position 16 t + m of the output on return.  The LDS twiddles must be
-// ordered before the call.  Twiddles from global memory are loaded a stage ahead;
-// so is what `ahead` loads for the caller, before the last stage.  On return
-// every thread's remaining LDS positions are its wave's own (os_dit_regs may
-// follow without a barrier).
+// and position 16 os_mid_thread(t) + m of the output on return.  The LDS twiddles
+// must be ordered before the call.  Twiddles from global memory are loaded a stage
+// ahead; so is what `ahead` loads for the caller, before the last stage.  On return
+// every LDS position is free for the wave that os_dit_regs writes it from (which
+// may follow without a barrier).
 template <class F>
 __device__ __forceinline__ void os_dif_regs(float2* lds, int t, const OsTwiddle& tw, float2* v,
                                             F&& ahead) {
+  const int t2 = os_mid_thread(t);
   float2 T[8], U[8];
   os_dif_first(lds, t, v);
-  os_tw_third(tw, t, T);
+  os_tw_third(tw, t2, T);
   __syncthreads();
   os_dif_mid1(lds, t, tw, v);
-  os_tw_last1<kOsN>(tw, t, U);
+  os_tw_last1<kOsN>(tw, t2, U);
   wave_sync();
-  os_dif_mid2(lds, t, T, v);
+  os_read16<2>(lds, 33 * (t2 >> 1) + (t2 & 1), v);
+  dft_tw<16>(v, T);
   ahead();
-  wave_sync();
-  os_dif_last(lds, t, U, v);
+  pairs_gather(v);
+  os_dif_pairs(U, v);
 }
 
 // Device, second transform (DIT): v in the first's output order on entry, value
@@ -528,10 +582,14 @@ __device__ __forceinline__ void os_dif_regs(float2* lds, int t, const OsTwiddle&
 // threads may still read must not be needed by the caller afterwards.
 __device__ __forceinline__ void os_dit_regs(float2* lds, int t, const OsTwiddle& tw,
                                             float2* v) {
+  const int t2 = os_mid_thread(t);
   float2 T[8];
-  os_dit_first(lds, t, v);
+  os_dit_pairs(v);
+  pairs_scatter(v);
+  os_load_tw<2>(tw.s + os_at_two(kOsN), t2 & 1, T);
+  dft_tw<16>(v, T);
   wave_sync();
-  os_dit_mid1(lds, t, tw, v);
+  os_write16<2>(lds, 33 * (t2 >> 1) + (t2 & 1), v);
   os_tw_last2<kOsN>(tw, t, T);
   wave_sync();
   os_dit_mid2(lds, t, tw, v);

@@ -177,7 +177,7 @@ __global__ void k_os_twiddles(float2* __restrict__ tw) {
 // Forward transform of one 8192-point vector (the reference function's
 // spectrum), one workgroup, in place: natural order in, digit-reversed order
 // out, position 16 t + m (bin drev(16 t + m)) at [m kOsThreads + t], as the
-// threads of k_rc_os multiply their own first transform's outputs with it.
+// threads of k_rc_os (os_mid_thread) multiply their own outputs with it.
 __global__ void __launch_bounds__(kOsThreads) k_os_spectrum(float2* __restrict__ v,
                                                              const float2* __restrict__ tw) {
   __shared__ float2 lds[kOsLds];
@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(kOsThreads) k_os_spectrum(float2* __restrict__
   for (int m = 0; m < 16; ++m) x[m] = v[t + m * kOsThreads];
   __syncthreads();   // the twiddle tables; every read of v is done
   os_dif_regs(lds, t, w, x, [] {});
-  for (int m = 0; m < 16; ++m) v[m * kOsThreads + t] = x[m];
+  for (int m = 0; m < 16; ++m) v[m * kOsThreads + os_mid_thread(t)] = x[m];
 }
 
 // Block b of line l: outputs k0 + k, k < M = 8192 - npts + 1, k0 = b M, of
@@ -226,7 +226,7 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
   const OsTwiddle w = os_twiddles_lds<kOsN>(twl, tw);
   const float2* echo = raw + (size_t)l * stride + kHdr;
   // thread t holds values t + kOsThreads m, m < 16, of the block (natural
-  // order), between the transforms positions 16 t + m (digit-reversed order)
+  // order), between the transforms positions 16 t2 + m (digit-reversed order)
   const int t = threadIdx.x;
   float2 v[16];
 #pragma unroll
@@ -236,9 +236,10 @@ k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int 
   }
   __syncthreads();   // the twiddle tables
   float2 sp[16];
+  const int t2 = os_mid_thread(t);
   os_dif_regs(lds, t, w, v, [&] {
 #pragma unroll
-    for (int m = 0; m < 16; ++m) sp[m] = spec[m * kOsThreads + t];
+    for (int m = 0; m < 16; ++m) sp[m] = spec[m * kOsThreads + t2];
   });
 #pragma unroll
   for (int m = 0; m < 16; ++m) v[m] = c_mul(make_float2(v[m].x, -v[m].y), sp[m]);

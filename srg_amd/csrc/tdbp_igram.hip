@@ -488,19 +488,31 @@ bool fused_length(size_t nnn) {
   return nnn >= (size_t)kUpMin && nnn <= (size_t)kUpMax && !(e && std::strcmp(e, "1") == 0);
 }
 
-// The fused kernels' tables, made on first use on the device.
-int tables(IgState& s, hipStream_t st) {
+// The fused kernels' tables, made on first use on the device, on a stream of
+// their own that the call waits for: calls on any stream may read them from
+// then on, also where the first one's stream is being captured.
+int tables(IgState& s) {
   if (s.tables) return TDBP_OK;
-  if (hipMalloc((void**)&s.tables, sizeof(float2) * kUpTables) != hipSuccess) {
-    s.tables = nullptr;
+  float2* t = nullptr;
+  hipStream_t st = nullptr;
+  if (hipMalloc((void**)&t, sizeof(float2) * kUpTables) != hipSuccess)
     return set_error(TDBP_ERR_NOMEM, "interferogram tables");
-  }
-  for (int n = kUpMin; n <= kUpMax; n *= 2) {
+  int e = hip_check(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "upsample tables");
+  for (int n = kUpMin; n <= kUpMax && !e; n *= 2) {
     hipLaunchKernelGGL(k_up_tables, dim3((up_table_values(n) + 255) / 256), dim3(256), 0, st, n,
-                       s.tables + up_table_at(n));
-    const int e = hip_check(hipGetLastError(), "upsample tables");
-    if (e) return e;
+                       t + up_table_at(n));
+    e = hip_check(hipGetLastError(), "upsample tables");
   }
+  if (st) {
+    const int e2 = hip_check(hipStreamSynchronize(st), "upsample tables");
+    if (!e) e = e2;
+    (void)hipStreamDestroy(st);
+  }
+  if (e) {
+    (void)hipFree(t);
+    return e;
+  }
+  s.tables = t;
   return TDBP_OK;
 }
 
@@ -568,7 +580,7 @@ int tdbp_crossmul(const void* d_img1, const void* d_img2, int na, int nvalid, fl
   FusedKernels k = {};
   const float2* tab = nullptr;
   if (fused) {
-    if ((st = tables(s, str))) return st;
+    if ((st = tables(s))) return st;
     k = fused_kernels(nnn);
     tab = s.tables + up_table_at((int)nnn);
     const dim3 grid((unsigned)nout), block((unsigned)(nnn / 8));

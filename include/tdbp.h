@@ -523,7 +523,9 @@ int tdbp_range_compress(const void *d_raw, int nlines, int raw_stride,
  * unscaled input sum is <= 1e-6 in either image (crossmul.f90:110-122, the
  * reference default).  Upsampling: zero-pad to nnn = next power of two >= na,
  * forward FFT, spectrum halves to both ends of 2 nnn, inverse FFT, / nnn / 2
- * (:127-148).  looksdn <= 512. */
+ * (:127-148).  looksdn <= 512.  Calls may overlap on several streams and
+ * threads; replays of a captured call must not overlap other calls on its
+ * device (they share one batch of upsampled rows). */
 int tdbp_crossmul(const void *d_img1, const void *d_img2, int na, int nvalid, float scale,
                   int looksac, int looksdn, int mask, void *d_igram, void *d_amp,
                   void *stream);

@@ -126,6 +126,11 @@ int cu_count() {
   return n > 0 ? n : 256;
 }
 
+bool stream_captures(hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return s && (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
+}
+
 // ------------------------------------------------------------ geometry
 
 int validate_geom(const tdbp_geom* g) {
@@ -282,10 +287,7 @@ int default_variant(int precision) {
 // while the stream is captured: the fit of a captured call stays refused, by
 // the wait below, as replays would keep the orbit of the capture.
 static bool orbit_in_args(const tdbp_geom* g, hipStream_t s) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (s && (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone))
-    return false;
-  return g->numstatevec <= kFitArgVec;
+  return g->numstatevec <= kFitArgVec && !stream_captures(s);
 }
 
 // The fit on a stream.  Orbits of up to kFitArgVec vectors go with the launch

@@ -15,6 +15,7 @@ int hip_check(hipError_t e, const char* what);
 int ensure_device(int device);
 int current_device_ready();
 int cu_count();
+bool stream_captures(hipStream_t s);   // whether a graph is being captured from it
 int validate_geom(const tdbp_geom* g);
 void fill_burst(const tdbp_geom* g, BurstDev* b);
 int set_tiles(BurstDev* b, int variant, bool own);

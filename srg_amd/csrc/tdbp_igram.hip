@@ -451,13 +451,19 @@ __global__ void k_makecc(const float2* __restrict__ ig, const float2* __restrict
 }
 
 // Per device: the transform buffers of one batch, grown as calls need them; a
-// call uses its own length nnn (rows nnn apart).
+// call uses its own length nnn (rows nnn apart).  Calls take turns with them:
+// each waits on its stream for the end of the last one's, whichever stream that
+// was on.  A call that is being captured can neither wait for nor record that:
+// its graph keeps the buffers it was captured with (never freed then), and its
+// replays are the caller's to keep apart from other calls.
 struct IgState {
   size_t values = 0;       // values each up buffer holds
   size_t buf_values = 0;
   float2* buf = nullptr;   // [kRows][nnn] spectra of a rocFFT batch
   float2* up1 = nullptr;   // [rows][nnn] odd samples of image 1
   float2* up2 = nullptr;
+  hipEvent_t used = nullptr;  // the end of the last call that used them
+  bool captured = false;      // some graph holds them
   float2* tables = nullptr;   // [kUpTables] of the fused kernels
 };
 std::mutex g_ig_mu;
@@ -468,12 +474,11 @@ int buffers(IgState& s, size_t values, size_t buf_values) {
   (void)hipDeviceSynchronize();
   values = std::max(values, s.values);
   buf_values = std::max(buf_values, s.buf_values);
-  if (s.buf) (void)hipFree(s.buf);
-  if (s.up1) (void)hipFree(s.up1);
-  if (s.up2) (void)hipFree(s.up2);
-  float2* tables = s.tables;   // do not depend on nnn
-  s = IgState();
-  s.tables = tables;
+  for (float2* p : {s.buf, s.up1, s.up2})
+    if (p && !s.captured) (void)hipFree(p);
+  s.buf = s.up1 = s.up2 = nullptr;
+  s.values = s.buf_values = 0;
+  s.captured = false;
   if ((buf_values && hipMalloc((void**)&s.buf, sizeof(float2) * buf_values) != hipSuccess) ||
       hipMalloc((void**)&s.up1, sizeof(float2) * values) != hipSuccess ||
       hipMalloc((void**)&s.up2, sizeof(float2) * values) != hipSuccess)
@@ -550,6 +555,39 @@ int upsample_rocfft(const float2* img, int na, int rows, int row0, int nvalid_ro
   return e;
 }
 
+// The two-pass form: batch after batch of output lines, rows upsampled into the
+// state's buffers, then products and looks out of them.
+int batches(IgState& s, const FusedKernels& k, const float2* tab, bool fused, size_t nnn,
+            const float2* i1, const float2* i2, int na, int nout, int lines_per_batch,
+            float scale, int looksac, int looksdn, int mask, float2* ig, float2* amp,
+            hipStream_t str) {
+  int st = TDBP_OK;
+  for (int ol0 = 0; ol0 < nout; ol0 += lines_per_batch) {
+    const int nol = nout - ol0 < lines_per_batch ? nout - ol0 : lines_per_batch;
+    const int row0 = ol0 * looksdn;
+    const int rows = nol * looksdn;
+    // An image with itself is upsampled once.
+    for (int i = 0; i < (i2 == i1 ? 1 : 2); ++i) {
+      const float2* img = i ? i2 : i1;
+      float2* up = i ? s.up2 : s.up1;
+      if (fused) {
+        hipLaunchKernelGGL(k.up, dim3((unsigned)rows), dim3((unsigned)(nnn / 16)), 0, str, img,
+                           na, row0, scale, tab, up);
+        st = hip_check(hipGetLastError(), "fused upsample");
+      } else {
+        st = upsample_rocfft(img, na, rows, row0, nout * looksdn, nnn, scale, s, up, str);
+      }
+      if (st) return st;
+    }
+    const int nw = na / looksac;
+    hipLaunchKernelGGL(k_xmul, dim3((unsigned)((nw + 127) / 128), nol), dim3(128), 0, str,
+                       s.up1, i2 == i1 ? s.up1 : s.up2, (int)nnn, i1, i2, na, scale, row0, nol,
+                       ol0, looksac, looksdn, mask, ig, amp);
+    if ((st = hip_check(hipGetLastError(), "crossmul launch"))) return st;
+  }
+  return TDBP_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -600,30 +638,18 @@ int tdbp_crossmul(const void* d_img1, const void* d_img2, int na, int nvalid, fl
   if ((st = buffers(s, (size_t)std::max(batch_rows, looksdn) * nnn,
                     fused ? 0 : (size_t)kRows * nnn)))
     return st;
-  for (int ol0 = 0; ol0 < nout; ol0 += lines_per_batch) {
-    const int nol = nout - ol0 < lines_per_batch ? nout - ol0 : lines_per_batch;
-    const int row0 = ol0 * looksdn;
-    const int rows = nol * looksdn;
-    // An image with itself is upsampled once.
-    for (int i = 0; i < (i2 == i1 ? 1 : 2); ++i) {
-      const float2* img = i ? i2 : i1;
-      float2* up = i ? s.up2 : s.up1;
-      if (fused) {
-        hipLaunchKernelGGL(k.up, dim3((unsigned)rows), dim3((unsigned)(nnn / 16)), 0, str, img,
-                           na, row0, scale, tab, up);
-        st = hip_check(hipGetLastError(), "fused upsample");
-      } else {
-        st = upsample_rocfft(img, na, rows, row0, used_rows, nnn, scale, s, up, str);
-      }
-      if (st) return st;
-    }
-    const int nw = na / looksac;
-    hipLaunchKernelGGL(k_xmul, dim3((unsigned)((nw + 127) / 128), nol), dim3(128), 0, str,
-                       s.up1, i2 == i1 ? s.up1 : s.up2, (int)nnn, i1, i2, na, scale, row0, nol,
-                       ol0, looksac, looksdn, mask ? 1 : 0, (float2*)d_igram, (float2*)d_amp);
-    if ((st = hip_check(hipGetLastError(), "crossmul launch"))) return st;
-  }
-  return TDBP_OK;
+  const bool capturing = stream_captures(str);
+  if (capturing) s.captured = true;
+  else if (!s.used)
+    st = hip_check(hipEventCreateWithFlags(&s.used, hipEventDisableTiming), "crossmul event");
+  else
+    st = hip_check(hipStreamWaitEvent(str, s.used, 0), "crossmul wait");
+  if (st) return st;
+  st = batches(s, k, tab, fused, nnn, i1, i2, na, nout, lines_per_batch, scale, looksac, looksdn,
+               mask ? 1 : 0, (float2*)d_igram, (float2*)d_amp, str);
+  // Also where a launch failed: the ones before it may be running.
+  const int st2 = capturing ? TDBP_OK : hip_check(hipEventRecord(s.used, str), "crossmul event");
+  return st ? st : st2;
 }
 
 int tdbp_makecc(const void* d_igram, const void* d_amp, int npix, int nlines, float* d_out,

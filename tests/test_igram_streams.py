@@ -33,3 +33,35 @@ F.fake_clear()
 T.crossmul(a, b, stream=s1)
 assert len(launches(log(), "k_up_tables")) == 4, log()
 """)
+
+
+# Few output lines (two passes over a shared batch), a width without a fused
+# kernel, and both after one another.
+def test_calls_take_turns_with_the_batch_buffers():
+    run(SETUP + """
+wide = [T.DeviceArray((9, 8200), np.complex64) for _ in range(2)]
+for stream, pair, looks in ((s1, (a, b), 8), (s2, (a, b), 8), (s1, wide, 2), (s2, (a, b), 8)):
+    T.crossmul(*pair, looksdn=looks, stream=stream)
+l = log()
+read = launches(l, "k_xmulEPK")
+write = launches(l, "k_up_fused") + launches(l, "k_up_load")
+assert len(read) == 4 and launches(l, "k_up_load"), l
+for r in read:
+    later = [w for w in write if w > r]
+    assert all(ordered(l, r, w) for w in later), l
+""")
+
+
+def test_buffers_of_a_graph_are_kept():
+    run(SETUP + """
+keep = [T.crossmul(a, b, looksdn=8, stream=s1)]
+cap = C.c_void_p(s1.ptr)
+F.hipStreamBeginCapture(cap, 0)
+keep.append(T.crossmul(a, b, looksdn=8, stream=s1))
+F.hipStreamEndCapture(cap, C.byref(C.c_void_p()))
+F.fake_clear()
+big = T.DeviceArray((24, 8192), np.complex64)
+keep.append(T.crossmul(big, big, looksdn=12, stream=s2))
+assert [c for c in log() if c[0] == "hipDeviceSynchronize"]   # they grew
+assert not [c for c in log() if c[0] == "hipFree"], log()
+""")

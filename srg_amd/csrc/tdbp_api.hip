@@ -13,6 +13,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "tdbp_api_internal.h"
@@ -389,10 +390,39 @@ int run_backproject(const tdbp_geom* g, const tdbp_samples* smp,
 // contiguous copy, through a pinned chunk on the host side.  A pitched
 // hipMemcpy2DAsync moves such rows one by one: 7.9 ms for 1200 lines; the
 // gather with a copy into pageable memory took 0.10 ms, through the pinned
-// chunk 0.05 ms.  The chunk (320 KB, one per process, taken in turns) is kept.
+// chunk 0.05 ms.
 constexpr int kHeaderChunk = 4096;   // lines
-static std::mutex g_header_mu;
-static uint8_t* g_header_pin = nullptr;
+
+// Pinned chunks (320 KB): a call holds one while it runs, so calls on different
+// streams do not wait for each other; up to four idle ones are kept.
+namespace {
+std::mutex g_header_mu;
+uint8_t* g_header_idle[4] = {};
+
+uint8_t* take_header_chunk() {
+  {
+    std::lock_guard<std::mutex> lk(g_header_mu);
+    for (uint8_t*& p : g_header_idle)
+      if (p) return std::exchange(p, nullptr);
+  }
+  uint8_t* p = nullptr;
+  const hipError_t e =
+      hipHostMalloc((void**)&p, (size_t)kHeaderChunk * 80, hipHostMallocPortable);
+  return hip_check(e, "header staging") ? nullptr : p;
+}
+
+void return_header_chunk(uint8_t* p) {
+  {
+    std::lock_guard<std::mutex> lk(g_header_mu);
+    for (uint8_t*& q : g_header_idle)
+      if (!q) {
+        q = p;
+        return;
+      }
+  }
+  (void)hipHostFree(p);
+}
+}  // namespace
 
 static int copy_headers(void* d_lines, int nlines, int stride, uint8_t* host, bool to_device,
                         void* stream) {
@@ -401,38 +431,31 @@ static int copy_headers(void* d_lines, int nlines, int stride, uint8_t* host, bo
   int st = current_device_ready();
   if (st) return st;
   hipStream_t s = (hipStream_t)stream;
-  std::lock_guard<std::mutex> lk(g_header_mu);
-  if (!g_header_pin &&
-      (st = hip_check(hipHostMalloc((void**)&g_header_pin, (size_t)kHeaderChunk * 80,
-                                    hipHostMallocPortable),
-                      "header staging"))) {
-    g_header_pin = nullptr;
-    return st;
-  }
+  uint8_t* pin = take_header_chunk();
+  if (!pin) return TDBP_ERR_HIP;
   void* d = nullptr;
-  if ((st = hip_check(hipMallocAsync(&d, (size_t)std::min(nlines, kHeaderChunk) * 80, s),
-                      "header scratch")))
-    return st;
+  st = hip_check(hipMallocAsync(&d, (size_t)std::min(nlines, kHeaderChunk) * 80, s),
+                 "header scratch");
   for (int l0 = 0; l0 < nlines && !st; l0 += kHeaderChunk) {
     const int n = std::min(kHeaderChunk, nlines - l0);
     const size_t bytes = (size_t)n * 80;
     char* lines = (char*)d_lines + (size_t)l0 * (size_t)stride * 8;
     if (to_device) {
-      std::memcpy(g_header_pin, host + (size_t)l0 * 80, bytes);
-      st = hip_check(hipMemcpyAsync(d, g_header_pin, bytes, hipMemcpyHostToDevice, s),
-                     "header upload");
+      std::memcpy(pin, host + (size_t)l0 * 80, bytes);
+      st = hip_check(hipMemcpyAsync(d, pin, bytes, hipMemcpyHostToDevice, s), "header upload");
       if (!st) st = hip_check(launch_headers(lines, n, stride, d, true, s), "header scatter");
     } else {
       st = hip_check(launch_headers(lines, n, stride, d, false, s), "header gather");
       if (!st)
-        st = hip_check(hipMemcpyAsync(g_header_pin, d, bytes, hipMemcpyDeviceToHost, s),
+        st = hip_check(hipMemcpyAsync(pin, d, bytes, hipMemcpyDeviceToHost, s),
                        "header download");
     }
     const int st2 = hip_check(hipStreamSynchronize(s), "header sync");
     if (!st) st = st2;
-    if (!st && !to_device) std::memcpy(host + (size_t)l0 * 80, g_header_pin, bytes);
+    if (!st && !to_device) std::memcpy(host + (size_t)l0 * 80, pin, bytes);
   }
-  (void)hipFreeAsync(d, s);
+  if (d) (void)hipFreeAsync(d, s);
+  return_header_chunk(pin);
   return st;
 }
 

@@ -390,7 +390,8 @@ int run_backproject(const tdbp_geom* g, const tdbp_samples* smp,
 // contiguous copy, through a pinned chunk on the host side.  A pitched
 // hipMemcpy2DAsync moves such rows one by one: 7.9 ms for 1200 lines; the
 // gather with a copy into pageable memory took 0.10 ms, through the pinned
-// chunk 0.05 ms.
+// chunk 0.05 ms.  Lines that are not the current device's own memory (a peer's,
+// managed or host memory) still go row by row: the kernel may not reach them.
 constexpr int kHeaderChunk = 4096;   // lines
 
 // Pinned chunks (320 KB): a call holds one while it runs, so calls on different
@@ -422,6 +423,15 @@ void return_header_chunk(uint8_t* p) {
   }
   (void)hipHostFree(p);
 }
+// Whether p is memory of the current device.
+bool on_current_device(const void* p) {
+  int dev = 0;
+  hipPointerAttribute_t a;
+  if (hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&a, p) == hipSuccess)
+    return a.type == hipMemoryTypeDevice && a.device == dev;
+  (void)hipGetLastError();   // an address the runtime does not know is no failed launch
+  return false;
+}
 }  // namespace
 
 static int copy_headers(void* d_lines, int nlines, int stride, uint8_t* host, bool to_device,
@@ -431,6 +441,14 @@ static int copy_headers(void* d_lines, int nlines, int stride, uint8_t* host, bo
   int st = current_device_ready();
   if (st) return st;
   hipStream_t s = (hipStream_t)stream;
+  if (!on_current_device(d_lines)) {
+    const size_t pitch = (size_t)stride * 8, n = (size_t)nlines;
+    st = to_device ? hip_check(hipMemcpy2DAsync(d_lines, pitch, host, 80, 80, n,
+                                                hipMemcpyHostToDevice, s), "header upload")
+                   : hip_check(hipMemcpy2DAsync(host, 80, d_lines, pitch, 80, n,
+                                                hipMemcpyDeviceToHost, s), "header download");
+    return st ? st : hip_check(hipStreamSynchronize(s), "header sync");
+  }
   uint8_t* pin = take_header_chunk();
   if (!pin) return TDBP_ERR_HIP;
   void* d = nullptr;

@@ -1,5 +1,6 @@
 """Line headers on a HIP runtime without a device: a call on one stream does not
-wait for what is queued on another's."""
+wait for what is queued on another's; lines of another device than the current
+one are copied by the runtime, not by a kernel of this one."""
 from fakehip import run
 
 
@@ -42,4 +43,19 @@ for t in threads:
     t.join(10)
 calls = [c[0] for c in log()]
 assert calls.count("hipHostMalloc") - calls.count("hipHostFree") <= 4
+""")
+
+
+def test_lines_of_another_device():
+    run("""
+T.init(0)
+raw = np.arange(5 * 160, dtype=np.uint8).reshape(5, 160)
+lines = T.DeviceArray((5, 20), np.complex64)
+lines.upload(raw.view(np.complex64))
+F.fake_owner(lines.ptr, 3)
+assert np.array_equal(T.headers_dtoh(lines), raw[:, :80])
+raw[:, :80] = 7
+T.headers_htod(lines, raw[:, :80])
+assert np.array_equal(lines.download().view(np.uint8).reshape(raw.shape), raw)
+assert not launches(log(), "k_headers")
 """)

@@ -321,7 +321,11 @@ int tdbp_autotune(const tdbp_geom *g, const tdbp_samples *s,
                   const double *d_satloc, const int16_t *d_dem, void *d_out,
                   int precision, int reps, float *ms, int *best);
 
-/* Kernel variant for TDBP_MIXED launches (autotuner output); -1 = auto. */
+/* Kernel variant for TDBP_MIXED launches (autotuner output); -1 = auto: the
+ * TDBP_VARIANT of the environment, else variant 5, or, for a burst of at most
+ * about one 256-pixel tile per CU, variant 5's wave tiles with a workgroup's
+ * waves sharing one tile's pulses.  A variant named here, in the environment or
+ * in a call runs as it is on every burst. */
 int tdbp_set_variant(int variant);
 int tdbp_variant_count(void);
 /* Describe variant v: rows x cols of the workgroup's pixel tile and pulses

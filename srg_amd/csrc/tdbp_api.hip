@@ -208,9 +208,10 @@ void fill_burst(const tdbp_geom* g, BurstDev* b) {
   b->dtype = TDBP_CF32;
 }
 
-// Tile grid of a burst for a variant; returns the variant to launch.  own: the
-// caller asked for this variant by index; else it is the default, and where
-// variant 1 or 5 would leave most of the chip idle that is kSplitVariant.
+// Tile grid of a burst for a variant; returns the variant to launch.  named: the
+// variant was asked for by index (in the call, by tdbp_set_variant or in the
+// environment); else it is the default, and where variant 1 or 5 would leave
+// most of the chip idle that is kSplitVariant.
 //
 // A wave that has a SIMD to itself issues an instruction about every 8 cycles,
 // whatever it waits for, so a burst of few tiles takes the time of one tile's
@@ -223,7 +224,7 @@ void fill_burst(const tdbp_geom* g, BurstDev* b) {
 // and 343 (298 and 340).  The rule sees the burst alone, so a batch computes
 // each of its bursts as a single launch does.
 constexpr double kSplitTiles = 256;
-int set_tiles(BurstDev* b, int variant, bool own) {
+int set_tiles(BurstDev* b, int variant, bool named) {
   // Lines with a valid aperture centre span L - A pulses of the track on the
   // ground.
   const auto norm = [](const double* x) {
@@ -233,7 +234,7 @@ int set_tiles(BurstDev* b, int variant, bool own) {
   const double lines = std::min<double>(
       b->nlines, (b->L - b->A) * step / std::max(std::fabs(b->deltalat) * 111320.0, 1e-3));
   const double tiles = std::max(lines, 0.0) * b->W / 256.0;
-  b->split = !own && (variant == 1 || variant == 5) && !b->cpu && tiles <= kSplitTiles;
+  b->split = !named && (variant == 1 || variant == 5) && !b->cpu && tiles <= kSplitTiles;
   if (b->split) variant = kSplitVariant;
   const Variant& v = kVariants[variant];
   b->tiles_r = (b->nlines + wg_rows(v) - 1) / wg_rows(v);
@@ -270,18 +271,23 @@ int check_samples(const tdbp_samples* s, int precision) {
   return TDBP_OK;
 }
 
-int default_variant(int precision) {
+int default_variant(int precision, bool* named) {
+  const auto from_env = [&](const char* name, int otherwise) {
+    const char* e = std::getenv(name);
+    const int v = e ? std::atoi(e) : -1;
+    *named = v >= 0 && v < kNumVariants;
+    return *named ? v : otherwise;
+  };
   if (precision == TDBP_PLAIN_FP64) {
     // Variant 1 (4 x 16 wave tiles side by side): 8.35-8.38 ms on one IW burst
     // against 8.37-9.30 for the others.
-    const char* e = std::getenv("TDBP_PLAIN_VARIANT");
-    const int v = e ? std::atoi(e) : 1;
-    return (v >= 0 && v < kNumVariants) ? v : 1;
+    return from_env("TDBP_PLAIN_VARIANT", 1);
   }
-  if (g_variant >= 0) return g_variant;
-  const char* e = std::getenv("TDBP_VARIANT");
-  const int v = e ? std::atoi(e) : 5;
-  return (v >= 0 && v < kNumVariants) ? v : 5;
+  if (g_variant >= 0) {
+    *named = true;
+    return g_variant;
+  }
+  return from_env("TDBP_VARIANT", 5);
 }
 
 // Whether the fit may carry the orbit in its arguments (launch_fit_arg).  Not
@@ -363,8 +369,9 @@ int run_backproject(const tdbp_geom* g, const tdbp_samples* smp,
   b.satloc = d_satloc;
   b.dem = d_dem;
   b.out = (float2*)d_out;
-  const bool asked = variant >= 0 && variant < kNumVariants;
-  variant = set_tiles(&b, asked ? variant : default_variant(precision), asked);
+  bool named = variant >= 0 && variant < kNumVariants;
+  if (!named) variant = default_variant(precision, &named);
+  variant = set_tiles(&b, variant, named);
   if ((st = counters_for(s, &b.counters))) return st;
   double* own = nullptr;
   if (!d_coef) {
@@ -779,7 +786,9 @@ int tdbp_backproject_noalloc(const tdbp_geom* g, const tdbp_samples* smp,
   b.satloc = d_satloc;
   b.dem = d_dem;
   b.out = (float2*)d_out;
-  const int variant = set_tiles(&b, default_variant(precision), false);
+  bool named = false;
+  int variant = default_variant(precision, &named);
+  variant = set_tiles(&b, variant, named);
   const int n = g->numstatevec;
   double* coef = sc + kScratchOrbit;
   if (orbit_in_args(g, s)) {

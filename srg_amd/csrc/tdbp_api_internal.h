@@ -18,11 +18,12 @@ int cu_count();
 bool stream_captures(hipStream_t s);   // whether a graph is being captured from it
 int validate_geom(const tdbp_geom* g);
 void fill_burst(const tdbp_geom* g, BurstDev* b);
-int set_tiles(BurstDev* b, int variant, bool own);
+int set_tiles(BurstDev* b, int variant, bool named);
 std::vector<double> pack_orbit(const tdbp_geom* g);
 void point_orbit(BurstDev* b, const double* d_orbit, int n);
 int check_samples(const tdbp_samples* s, int precision);
-int default_variant(int precision);
+// named: set by tdbp_set_variant or in the environment, not the built-in choice.
+int default_variant(int precision, bool* named);
 int fit_on_stream(BurstDev& b, const tdbp_geom* g, double* d_coef,
                   hipStream_t s);
 int run_backproject(const tdbp_geom* g, const tdbp_samples* smp,

@@ -37,7 +37,7 @@ struct BatchQueue {
 struct tdbp_batch {
   int precision = TDBP_MIXED;
   int variant = -1;
-  bool own_variant = false;   // the variant was asked for (or tuned), not the default
+  bool named = false;   // the variant was asked for by index (or tuned)
   int dtype = -1;
   std::vector<BurstDev> bursts;
   std::vector<MergeTarget> merges;  // per burst, applied in burst order
@@ -136,13 +136,13 @@ int build_tables(tdbp_batch* b) {
   if ((st = hip_check(hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking),
                       "batch stream")))
     return st;
-  if (b->variant < 0) b->variant = default_variant(b->precision);
+  if (b->variant < 0) b->variant = default_variant(b->precision, &b->named);
   if (b->variant == 8)   // the MFMA kernel needs 32-bit sample offsets in every burst
     for (auto& bd : b->bursts)
       if (!mfma_fits(bd)) b->variant = 5;
   b->max_lines = 0;
   for (auto& bd : b->bursts) {
-    set_tiles(&bd, b->variant, b->own_variant);
+    set_tiles(&bd, b->variant, b->named);
     b->max_lines = std::max(b->max_lines, bd.nlines);
   }
   const size_t nb = b->bursts.size();
@@ -250,7 +250,7 @@ tdbp_batch* tdbp_batch_create(int precision, int variant) {
   tdbp_batch* b = new tdbp_batch;
   b->precision = precision;
   b->variant = variant;
-  b->own_variant = variant >= 0;
+  b->named = variant >= 0;
   return b;
 }
 
@@ -359,7 +359,7 @@ int tdbp_batch_autotune(tdbp_batch* b, int reps, float* ms, int* best) {
     }
     unbuild(b);
     b->variant = v;
-    b->own_variant = true;
+    b->named = true;
     if ((st = build(b))) break;
     if ((st = tdbp_batch_run(b, b->cap))) break;   // warm-up
     (void)hipEventRecord(e0, b->cap);

@@ -634,7 +634,7 @@ def stack_bench(args, synth, T):
                        budget=budget, repeats=args.warmup + args.steps, autotune_reps=2)
     tuned = {"variant": run.tuned[0]} if run.tuned else {}
     if run.tuned:
-        log(f"batch autotune: variant {run.tuned[0]} {T.variant_info(run.tuned[0])}; "
+        log(f"batch autotune: variant {run.tuned[0]}; "
             f"ms per variant {[round(x, 1) for x in run.tuned[1]]}")
     pairs = sum(run.pairs)
     per_batch = [float(np.mean(ms[args.warmup:])) for ms in run.run_ms]
@@ -851,7 +851,7 @@ def main():
     if args.variant < 0:
         best, tune_ms = batch.autotune(reps=2)
         T.lib().tdbp_set_variant(best)   # the other-storage batches below use it too
-        log(f"batch autotune: variant {best} {T.variant_info(best)}; "
+        log(f"batch autotune: variant {best} {T.variant_info(batch.variant)}; "
             f"ms per variant {[round(x, 2) for x in tune_ms]}")
     batch.run(stream)
     stream.sync()

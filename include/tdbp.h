@@ -314,7 +314,8 @@ int tdbp_backproject_variant(const tdbp_geom *g, const tdbp_samples *s,
 
 /* Autotuner: time every VALU kernel variant on this burst (reps launches
  * each, after one warm-up), return the fastest in *best and, for TDBP_MIXED,
- * make it the default of later launches.  ms (optional, [count]) gets the
+ * make it the default of later launches (the default stays automatic where it
+ * already is that variant on this burst).  ms (optional, [count]) gets the
  * mean milliseconds per launch of each variant (0 for the MFMA variant 8,
  * which runs only when asked for by index).  Overwrites d_out. */
 int tdbp_autotune(const tdbp_geom *g, const tdbp_samples *s,
@@ -323,8 +324,8 @@ int tdbp_autotune(const tdbp_geom *g, const tdbp_samples *s,
 
 /* Kernel variant for TDBP_MIXED launches (autotuner output); -1 = auto: the
  * TDBP_VARIANT of the environment, else variant 5, or, for a burst of at most
- * about one 256-pixel tile per CU, variant 5's wave tiles with a workgroup's
- * waves sharing one tile's pulses.  A variant named here, in the environment or
+ * about one 256-pixel tile per CU, variant 11: variant 5's wave tiles with a
+ * workgroup's four waves sharing one tile's pulses.  A variant named here, in the environment or
  * in a call runs as it is on every burst. */
 int tdbp_set_variant(int variant);
 int tdbp_variant_count(void);
@@ -360,12 +361,14 @@ int tdbp_batch_set_merge(tdbp_batch *b, int burst, void *d_grid, int grid_lines,
 int tdbp_batch_run(tdbp_batch *b, void *stream);
 /* Variant the batch runs (resolved at the first run). */
 int tdbp_batch_variant(const tdbp_batch *b);
-/* Time every VALU variant (0-7, 9, 10) on this batch's own bursts -- reps graph
+/* Time every VALU variant (0-7, 9-11) on this batch's own bursts -- reps graph
  * launches each after a warm-up -- and keep the fastest for this batch only
  * (the process-wide default is unchanged; pass *best to tdbp_set_variant to
  * make it the default of later TDBP_MIXED launches).  ms (optional,
  * [tdbp_variant_count()]) gets the mean milliseconds per launch of each
- * variant (0 for the MFMA variant 8).  Overwrites the outputs and re-applies
+ * variant (0 for the MFMA variant 8).  On a batch in which the automatic
+ * choice gives some bursts variant 11 and others another, it is timed as well,
+ * and *best is -1 where it is the fastest.  Overwrites the outputs and re-applies
  * the merges (an overwrite, so the grid ends as after one run).  No
  * counterpart in the reference: the batched path is new. */
 int tdbp_batch_autotune(tdbp_batch *b, int reps, float *ms, int *best);

@@ -211,7 +211,8 @@ void fill_burst(const tdbp_geom* g, BurstDev* b) {
 // Tile grid of a burst for a variant; returns the variant to launch.  named: the
 // variant was asked for by index (in the call, by tdbp_set_variant or in the
 // environment); else it is the default, and where variant 1 or 5 would leave
-// most of the chip idle that is kSplitVariant.
+// most of the chip idle that is kSplitVariant.  The CPU twin's arithmetic has no
+// split form: kSplitVariant is variant 5 there.
 //
 // A wave that has a SIMD to itself issues an instruction about every 8 cycles,
 // whatever it waits for, so a burst of few tiles takes the time of one tile's
@@ -234,8 +235,9 @@ int set_tiles(BurstDev* b, int variant, bool named) {
   const double lines = std::min<double>(
       b->nlines, (b->L - b->A) * step / std::max(std::fabs(b->deltalat) * 111320.0, 1e-3));
   const double tiles = std::max(lines, 0.0) * b->W / 256.0;
-  b->split = !named && (variant == 1 || variant == 5) && !b->cpu && tiles <= kSplitTiles;
-  if (b->split) variant = kSplitVariant;
+  if (!named && (variant == 1 || variant == 5) && tiles <= kSplitTiles) variant = kSplitVariant;
+  if (variant == kSplitVariant && b->cpu) variant = 5;
+  b->split = variant == kSplitVariant;
   const Variant& v = kVariants[variant];
   b->tiles_r = (b->nlines + wg_rows(v) - 1) / wg_rows(v);
   b->tiles_c = (b->W + wg_cols(v) - 1) / wg_cols(v);
@@ -271,7 +273,7 @@ int check_samples(const tdbp_samples* s, int precision) {
   return TDBP_OK;
 }
 
-int default_variant(int precision, bool* named) {
+int automatic_variant(int precision, bool* named) {
   const auto from_env = [&](const char* name, int otherwise) {
     const char* e = std::getenv(name);
     const int v = e ? std::atoi(e) : -1;
@@ -283,11 +285,15 @@ int default_variant(int precision, bool* named) {
     // against 8.37-9.30 for the others.
     return from_env("TDBP_PLAIN_VARIANT", 1);
   }
-  if (g_variant >= 0) {
+  return from_env("TDBP_VARIANT", 5);
+}
+
+int default_variant(int precision, bool* named) {
+  if (precision == TDBP_MIXED && g_variant >= 0) {
     *named = true;
     return g_variant;
   }
-  return from_env("TDBP_VARIANT", 5);
+  return automatic_variant(precision, named);
 }
 
 // Whether the fit may carry the orbit in its arguments (launch_fit_arg).  Not

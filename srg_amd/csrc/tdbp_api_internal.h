@@ -22,7 +22,9 @@ int set_tiles(BurstDev* b, int variant, bool named);
 std::vector<double> pack_orbit(const tdbp_geom* g);
 void point_orbit(BurstDev* b, const double* d_orbit, int n);
 int check_samples(const tdbp_samples* s, int precision);
-// named: set by tdbp_set_variant or in the environment, not the built-in choice.
+// The variant of a launch that names none, and the same without regard to
+// tdbp_set_variant.  named: set by that or in the environment, not built in.
+int automatic_variant(int precision, bool* named);
 int default_variant(int precision, bool* named);
 int fit_on_stream(BurstDev& b, const tdbp_geom* g, double* d_coef,
                   hipStream_t s);

@@ -176,7 +176,9 @@ int build_tables(tdbp_batch* b) {
   b->pairs = 0;
   for (int64_t v : hp) b->pairs += v;
 
-  // Work queues, one set per tile kind.
+  // Work queues, one set per tile kind (kSplitVariant's whole bursts: the CPU
+  // twin's, on variant 5's tiles).
+  const int whole = b->variant == kSplitVariant ? 5 : b->variant;
   for (int split = 0; split < 2; ++split) {
     std::vector<std::vector<int2>> q(8);
     int g = 0;
@@ -198,7 +200,7 @@ int build_tables(tdbp_batch* b) {
     qbase[8] = (int)items.size();
     if (items.empty()) continue;
     BatchQueue d;
-    d.variant = split ? kSplitVariant : b->variant;
+    d.variant = split ? kSplitVariant : whole;
     if ((st = talloc(b, (void**)&d.items, items.size() * sizeof(int2))) ||
         (st = talloc(b, (void**)&d.qbase, 9 * sizeof(int))) ||
         (st = talloc(b, (void**)&d.counters, 8 * sizeof(int))))
@@ -336,7 +338,9 @@ void tdbp_batch_destroy(tdbp_batch* b) {
   delete b;
 }
 
-// Time every VALU variant on the batch's own bursts and keep the fastest.
+// Time every VALU variant on the batch's own bursts and keep the fastest.  Where
+// the automatic choice splits some of the bursts' tiles and not others, no
+// variant by itself is that choice: it is timed too, as the last candidate.
 int tdbp_batch_autotune(tdbp_batch* b, int reps, float* ms, int* best) {
   if (!b) return set_error(TDBP_ERR_ARG, "null batch");
   if (b->bursts.empty()) return set_error(TDBP_ERR_ARG, "empty batch");
@@ -349,17 +353,25 @@ int tdbp_batch_autotune(tdbp_batch* b, int reps, float* ms, int* best) {
     if (e0) (void)hipEventDestroy(e0);
     return st;
   }
+  bool named = false;
+  const int automatic = automatic_variant(b->precision, &named);
+  size_t split = 0;
+  for (BurstDev bd : b->bursts) {
+    set_tiles(&bd, automatic, named);
+    split += bd.split;
+  }
+  const bool both = !named && split > 0 && split < b->bursts.size();
   int bestv = -1;
   float bestms = 3.4e38f;
-  for (int v = 0; v < kNumVariants && !st; ++v) {
+  for (int v = 0; v < kNumVariants + (both ? 1 : 0) && !st; ++v) {
     // The MFMA variant (8) runs only when asked for by index.
-    if (kVariants[v].mfma) {
+    if (v < kNumVariants && kVariants[v].mfma) {
       if (ms) ms[v] = 0.f;
       continue;
     }
     unbuild(b);
-    b->variant = v;
-    b->named = true;
+    b->named = v < kNumVariants;
+    b->variant = b->named ? v : automatic;
     if ((st = build(b))) break;
     if ((st = tdbp_batch_run(b, b->cap))) break;   // warm-up
     (void)hipEventRecord(e0, b->cap);
@@ -369,24 +381,26 @@ int tdbp_batch_autotune(tdbp_batch* b, int reps, float* ms, int* best) {
     float t = 0.f;
     if (!st) (void)hipEventElapsedTime(&t, e0, e1);
     t /= reps;
-    if (ms) ms[v] = t;
+    if (ms && b->named) ms[v] = t;
     if (!st && t < bestms) {
       bestms = t;
-      bestv = v;
+      bestv = b->named ? v : -1;
     }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   unbuild(b);
   if (st) return st;
-  b->variant = bestv;
+  b->named = bestv >= 0;
+  b->variant = b->named ? bestv : automatic;
   if ((st = build(b))) return st;
   if (best) *best = bestv;
   return TDBP_OK;
 }
 
 // Time every variant on one burst and keep the fastest for later TDBP_MIXED
-// launches.  ms (optional) gets the mean time of each variant.
+// launches; where that is what the automatic choice runs on this burst, the
+// choice stays automatic, so that it suits later bursts of other sizes.  ms (optional) gets the mean time of each variant.
 int tdbp_autotune(const tdbp_geom* g, const tdbp_samples* s,
                   const double* d_satloc, const int16_t* d_dem, void* d_out,
                   int precision, int reps, float* ms, int* best) {
@@ -448,7 +462,13 @@ int tdbp_autotune(const tdbp_geom* g, const tdbp_samples* s,
   (void)hipStreamDestroy(str);
   if (st) return st;
   if (best) *best = bestv;
-  if (precision == TDBP_MIXED) tdbp_set_variant(bestv);
+  if (precision == TDBP_MIXED) {
+    BurstDev b;
+    fill_burst(g, &b);
+    bool named = false;
+    const int automatic = automatic_variant(precision, &named);
+    tdbp_set_variant(set_tiles(&b, automatic, named) == bestv ? -1 : bestv);
+  }
   return TDBP_OK;
 }
 

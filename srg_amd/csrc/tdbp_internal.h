@@ -57,11 +57,10 @@ struct Variant {
   int lds;           // 1: the pulse windows of the samples staged in LDS
                      //    (kLdsPulses pulses of kLdsWindow samples at a time)
 };
-constexpr int kNumVariants = 11;
+constexpr int kNumVariants = 12;
 // The tile that launches by default take instead of variants 1 and 5 (4-row
-// wave tiles) for a burst with too few pixels to fill the chip (set_tiles);
-// not a variant a caller can ask for.
-constexpr int kSplitVariant = kNumVariants;
+// wave tiles) for a burst with too few pixels to fill the chip (set_tiles).
+constexpr int kSplitVariant = 11;
 // LDS staging of the sample windows: pulses per sub-stage and samples per
 // pulse window (FP32 complex in LDS: 16 x 112 x 8 B = 14 KB per workgroup,
 // which with the 16 KB of pulse records leaves room for 5 workgroups in a
@@ -72,7 +71,7 @@ constexpr int kLdsWindow = 112;
 inline bool mfma_fits(const BurstDev& b) {
   return (size_t)b.L * (size_t)b.S * (b.dtype == TDBP_CF32 ? 8u : 4u) < (size_t)0xffffffffu;
 }
-extern const Variant kVariants[kNumVariants + 1];
+extern const Variant kVariants[kNumVariants];
 
 inline int wg_rows(const Variant& v) {
   return v.stack == kWavesStacked ? 4 * v.tile_rows : v.tile_rows;

@@ -40,7 +40,7 @@
 
 namespace tdbp {
 
-const Variant kVariants[kNumVariants + 1] = {
+const Variant kVariants[kNumVariants] = {
     {8, 0, 0, 0}, {4, 0, 0, 0}, {2, 0, 0, 0}, {1, 0, 0, 0}, {8, 1, 0, 0},
     {4, 1, 0, 0}, {2, 1, 0, 0}, {1, 1, 0, 0}, {4, 1, 1, 0},
     {4, 1, 0, 1}, {8, 1, 0, 1}, {4, kWavesSplit, 0, 0}};

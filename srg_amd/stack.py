@@ -191,7 +191,10 @@ def run_stack(bursts: Sequence[StackBurst], grids: Sequence[tdbp.DeviceArray],
             tdbp.sync()
             if on_resident is not None:
                 on_resident(idx, res)
-            batch = tdbp.Batch(precision, run.tuned[0] if run.tuned else variant)
+            pick = variant
+            if run.tuned and run.tuned[0] != 11:   # 11 is automatic, and for small bursts only
+                pick = run.tuned[0]
+            batch = tdbp.Batch(precision, pick)
             try:
                 for k, (i, r) in enumerate(zip(idx, res)):
                     g = bursts[i].geom

@@ -748,7 +748,8 @@ class Batch:
     def autotune(self, reps: int = 2):
         """Time every VALU variant on this batch (tdbp_batch_autotune) and keep
         the fastest for this batch (the process default is unchanged); returns
-        (best, ms per variant)."""
+        (best, ms per variant), best -1 where the automatic choice over bursts
+        of different sizes beats every variant."""
         n = lib().tdbp_variant_count()
         ms = (C.c_float * n)()
         best = C.c_int(-1)

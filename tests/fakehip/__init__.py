@@ -19,7 +19,7 @@ F = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
 F.fake_block.argtypes = [C.c_void_p, C.c_int]
 F.fake_waiting.argtypes = [C.c_void_p]
 F.fake_owner.argtypes = [C.c_void_p, C.c_int]
-F.fake_cost.argtypes = [C.c_char_p, C.c_double]
+F.fake_cost.argtypes = [C.c_char_p, C.c_double, C.c_double]
 import numpy as np
 from srg_amd import synth, tdbp as T
 

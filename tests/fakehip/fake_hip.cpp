@@ -24,7 +24,11 @@ std::map<void*, int> waiting;
 std::map<const void*, int> owner;             // pointers said to be another device's
 std::map<void*, std::vector<std::string>> capture, graphs;   // stream / graph -> launches
 std::map<void*, double> clock_of, stamp;      // simulated ms of a stream, of an event
-std::vector<std::pair<std::string, double>> costs;           // part of a kernel's name -> ms
+struct Cost {
+  std::string part;   // of a kernel's name
+  double alone, among;   // ms, in a graph that holds no other such kernel, or others
+};
+std::vector<Cost> costs;
 thread_local hipError_t last = hipSuccess;
 thread_local int device = 0;
 int devices = 1;
@@ -50,10 +54,10 @@ hipError_t note(const char* call, const std::string& text = "") {
   if (!text.empty()) calls.push_back(std::string(call) + " " + text);
   return hipSuccess;
 }
-double cost(const std::string& name) {
+const Cost* cost(const std::string& name) {
   for (auto& c : costs)
-    if (name.find(c.first) != std::string::npos) return c.second;
-  return 0.;
+    if (name.find(c.part) != std::string::npos) return &c;
+  return nullptr;
 }
 }  // namespace
 
@@ -89,9 +93,9 @@ void fake_owner(void* p, int dev) {
   std::lock_guard<std::mutex> lk(mu);
   owner[p] = dev;
 }
-void fake_cost(const char* part, double ms) {
+void fake_cost(const char* part, double alone, double among) {
   std::lock_guard<std::mutex> lk(mu);
-  costs.insert(costs.begin(), {part, ms});
+  costs.insert(costs.begin(), {part, alone, among});
 }
 
 // ---- kernels
@@ -126,7 +130,7 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_
       c->second.push_back(name);
       return hipSuccess;
     }
-    clock_of[s] += cost(name);
+    if (const Cost* k = cost(name)) clock_of[s] += k->alone;
   }
   return note("hipLaunchKernel", hex(s) + " " + name);
 }
@@ -281,8 +285,10 @@ hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*,
 }
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s) {
   std::lock_guard<std::mutex> lk(mu);
+  int timed = 0;
+  for (auto& name : graphs[e]) timed += cost(name) && cost(name)->alone > 0;
   for (auto& name : graphs[e]) {
-    clock_of[s] += cost(name);
+    if (const Cost* k = cost(name)) clock_of[s] += timed > 1 ? k->among : k->alone;
     calls.push_back("hipLaunchKernel " + hex(s) + " " + name);
   }
   return hipSuccess;

@@ -235,8 +235,11 @@ int set_tiles(BurstDev* b, int variant, bool named) {
   const double lines = std::min<double>(
       b->nlines, (b->L - b->A) * step / std::max(std::fabs(b->deltalat) * 111320.0, 1e-3));
   const double tiles = std::max(lines, 0.0) * b->W / 256.0;
-  if (!named && (variant == 1 || variant == 5) && tiles <= kSplitTiles) variant = kSplitVariant;
-  if (variant == kSplitVariant && b->cpu) variant = 5;
+  if (b->cpu) {
+    if (variant == kSplitVariant) variant = 5;
+  } else if (!named && (variant == 1 || variant == 5) && tiles <= kSplitTiles) {
+    variant = kSplitVariant;
+  }
   b->split = variant == kSplitVariant;
   const Variant& v = kVariants[variant];
   b->tiles_r = (b->nlines + wg_rows(v) - 1) / wg_rows(v);

@@ -1439,6 +1439,24 @@ __device__ __forceinline__ void plain_excess_tile(const BurstDev& b, int tile, P
     }
     __syncthreads();
   }
+  // An infinite sample leaves an infinity or NaN in the sum; the pairs' products
+  // would make NaN of every infinity, so such a lane's pulses are summed one by
+  // one instead.
+  const auto infinite = [](double v) { return !(fabs(v) <= 1.79769313486231571e308); };
+  const bool redo = live && wave_fit && (infinite(ar) || infinite(ai));
+  if (__any(redo ? 1 : 0)) {
+    if (redo) ar = ai = 0.;
+    for (int p0 = wlo; p0 < whi; p0 += kPlainStage) {
+      const int p1 = min(p0 + kPlainStage, whi);
+      int qa = max(p0, qlo), qb = min(p1, qhi);
+      if constexpr (STACK == kWavesSplit) split_stage(p0, p1, &qa, &qb);
+      for (int q = qa; q < qb; ++q) {
+        const double sx = sat[3 * q], sy = sat[3 * q + 1], sz = sat[3 * q + 2];
+        if (redo && (unsigned)(q - p.azs) < na)
+          plain_pair(base + (size_t)q * b.S, x, sx, sy, sz, b, ar, ai);
+      }
+    }
+  }
   if constexpr (STACK == kWavesSplit) {
     if (!split_join((double*)rec, &ar, &ai)) return;
   }

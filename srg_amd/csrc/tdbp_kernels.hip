@@ -2714,14 +2714,14 @@ k_pack(const float2* __restrict__ in, int S, int L, uint32_t* __restrict__ out,
        float* __restrict__ scale) {
   __shared__ float part[kPackBlock / kWave];
   const int p = blockIdx.x;
-  const float own = scale[p];
+  const float own = load_scale(scale + p);
   float m = 0.f;
-  for (int i = threadIdx.x; i < L; i += kPackBlock) m = fmaxf(m, scale[i]);
+  for (int i = threadIdx.x; i < L; i += kPackBlock) m = fmaxf(m, load_scale(scale + i));
   const float s = unified_scale(own, block_max(m, part), DT);   // barrier: scale[p] is read
   const bool rescale = own > 0.f && own != s;
   pack_row<DT>(in + (size_t)p * S, S, out + (size_t)p * S, pulse_inv(own), rescale,
                rescale ? own / s : 1.f);
-  if (threadIdx.x == 0) scale[p] = s;
+  if (threadIdx.x == 0) store_scale(scale + p, s);
 }
 
 // One block per pulse, after the packing range-compression store:
@@ -2737,16 +2737,16 @@ __global__ void k_unify_scales(uint32_t* __restrict__ packed, size_t rowwords, i
   __shared__ float part[kBlock / kWave];
   const int p = blockIdx.x;
   float m = 0.f;
-  for (int i = threadIdx.x; i < L; i += blockDim.x) m = fmaxf(m, scale[i]);
+  for (int i = threadIdx.x; i < L; i += blockDim.x) m = fmaxf(m, load_scale(scale + i));
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
   __syncthreads();
   float M = part[0];
   for (int w = 1; w < kBlock / kWave; ++w) M = fmaxf(M, part[w]);
-  const float s = scale[p];
+  const float s = load_scale(scale + p);
   __syncthreads();  // every thread has read scale[p] before it changes
   if (M == 0.f) {
-    if (threadIdx.x == 0) scale[p] = 1.f;
+    if (threadIdx.x == 0) store_scale(scale + p, 1.f);
     return;
   }
   const float lowest = dtype == TDBP_CI16 ? M * (1.0f / (1 << kI16Unify)) : M * (1.0f / 65536.0f);
@@ -2760,7 +2760,7 @@ __global__ void k_unify_scales(uint32_t* __restrict__ packed, size_t rowwords, i
       row[i] = pack_word(re * f, im * f, dtype);
     }
   }
-  if (threadIdx.x == 0) scale[p] = M;
+  if (threadIdx.x == 0) store_scale(scale + p, M);
 }
 
 // Counter-based normal pair (splitmix64 hash -> Box-Muller).

@@ -156,9 +156,21 @@ __device__ __forceinline__ void pack_row(const float2* __restrict__ y, int n,
     o[n - 1] = pack_sample<DT>(y[n - 1].x, y[n - 1].y, inv, rescale, f);
 }
 
+// Scales that other workgroups of the same launch may be rewriting (k_pack,
+// k_unify_scales): either value will do (unified_scale), a torn or cached-away
+// one would not.
+__device__ __forceinline__ float load_scale(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_scale(float* p, float s) {
+  __hip_atomic_store(p, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The scale k_unify_scales leaves a pulse of scale s in a call whose largest
-// is M.
-__device__ __forceinline__ float unified_scale(float s, float M, int dtype) {
+// is M.  With any of the call's scales already replaced by theirs the largest,
+// and so every other pulse's, comes out the same, but for a call of zeros alone:
+// there M may be 0 or 1, and the scale is 1 either way.
+__host__ __device__ inline float unified_scale(float s, float M, int dtype) {
   const float lowest = dtype == TDBP_CI16 ? M * (1.0f / (1 << kI16Unify)) : M * (1.0f / 65536.0f);
   return M == 0.f ? 1.f : (s == M || (s > 0.f && s < lowest)) ? s : M;
 }

@@ -256,16 +256,13 @@ TDBP_HD void os_dif_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
   os_load_tw<16>(tw.s, t >> 5, T);
   os_stage16<33>(lds, 528 * (t >> 5) + (t & 31), T, v);
 }
-TDBP_HD void os_dif_mid2(float2* lds, int t, const float2* T, float2* v) {
-  os_stage16<2>(lds, 33 * (t >> 1) + (t & 1), T, v);
+TDBP_HD void os_dif_mid2(const float2* lds, int t2, const float2* T, float2* v) {
+  os_read16<2>(lds, 33 * (t2 >> 1) + (t2 & 1), v);
+  dft_tw<16>(v, T);
 }
 TDBP_HD void os_dif_pairs(const float2* T, float2* v) {
 #pragma unroll
   for (int h = 0; h < 8; ++h) bfly<false>(v[2 * h], v[2 * h + 1], T[h]);
-}
-TDBP_HD void os_dif_last(const float2* lds, int t, const float2* T, float2* v) {
-  os_read16<1>(lds, os_pad(16 * t), v);
-  os_dif_pairs(T, v);
 }
 TDBP_HD void os_dit_pairs(float2* v) {
 #pragma unroll
@@ -275,14 +272,13 @@ TDBP_HD void os_dit_pairs(float2* v) {
     v[2 * h + 1] = c_sub(a, b);
   }
 }
-TDBP_HD void os_dit_first(float2* lds, int t, float2* v) {
-  os_dit_pairs(v);
-  os_write16<1>(lds, os_pad(16 * t), v);
-}
-TDBP_HD void os_dit_mid1(float2* lds, int t, const OsTwiddle& tw, float2* v) {
+TDBP_HD void os_dit_mid1(int t2, const OsTwiddle& tw, float2* v) {
   float2 T[8];
-  os_load_tw<2>(tw.s + os_at_two(kOsN), t & 1, T);
-  os_stage16<2>(lds, 33 * (t >> 1) + (t & 1), T, v);
+  os_load_tw<2>(tw.s + os_at_two(kOsN), t2 & 1, T);
+  dft_tw<16>(v, T);
+}
+TDBP_HD void os_dit_write(float2* lds, int t2, const float2* v) {
+  os_write16<2>(lds, 33 * (t2 >> 1) + (t2 & 1), v);
 }
 TDBP_HD void os_dit_mid2(float2* lds, int t, const OsTwiddle& tw, float2* v) {
   float2 T[8];
@@ -296,8 +292,43 @@ TDBP_HD void os_dit_last(const float2* lds, int t, const float2* T, float2* v) {
   dft_tw<16>(v, T);
 }
 
+// The thread of stages (16, 2) and (2, 1) that thread t is: lanes r and r + 32 of
+// a wave are a pair 2 q, 2 q + 1.
+TDBP_HD int os_mid_thread(int t) { return (t & ~63) | ((t & 31) << 1) | ((t >> 5) & 1); }
+// Between those stages the values change hands within the pairs, position 32 q +
+// j + 2 k of thread 2 q + j as v[k] against 32 q + 16 j + m as v[m]: the second
+// half of the lower lane's values against the first half of the upper's, which
+// v_permlane32_swap does for two registers at once, in the place of an LDS write
+// and read (a third of the transforms' LDS cycles).  swap(a, b): the upper
+// lane's a for the lower lane's b.
+template <class V, class S>
+TDBP_HD void pairs_gather(V* v, const S& swap) {
+  V w[16];
+#pragma unroll
+  for (int h = 0; h < 8; ++h) {
+    w[2 * h] = v[h];
+    w[2 * h + 1] = v[h + 8];
+    swap(w[2 * h], w[2 * h + 1]);
+  }
+#pragma unroll
+  for (int m = 0; m < 16; ++m) v[m] = w[m];
+}
+template <class V, class S>
+TDBP_HD void pairs_scatter(V* v, const S& swap) {
+  V w[16];
+#pragma unroll
+  for (int h = 0; h < 8; ++h) {
+    w[h] = v[2 * h];
+    w[h + 8] = v[2 * h + 1];
+    swap(w[h], w[h + 8]);
+  }
+#pragma unroll
+  for (int m = 0; m < 16; ++m) v[m] = w[m];
+}
+
 // Host transforms (the check of the device code): the same stages, layout
-// and registers, thread after thread, a stage loop in place of each barrier.
+// and per-thread registers, thread by thread, the pairs of stages (16, 2) and
+// (2, 1) exchanged as the device's lanes do.
 // os_dif_host: data in natural order -> data[p] = X[drev(p)].
 // os_dit_host: data[p] = Y[drev(p)] -> data in natural order, the forward
 // transform of Y.
@@ -309,45 +340,77 @@ struct OsHostTables {
   }
   OsTwiddle tw() const { return OsTwiddle{v, v + os_at_lds(N)}; }
 };
+struct OsLanes {   // a register of lanes r and r + 32
+  float2 lane[2];
+};
+struct OsHostSwap {
+  void operator()(OsLanes& a, OsLanes& b) const {
+    const float2 upper = a.lane[1];
+    a.lane[1] = b.lane[0];
+    b.lane[0] = upper;
+  }
+};
+template <class F>
+inline void os_host_pairs(float2 (*v)[16], F&& exchange) {   // v: all threads' registers
+  for (int t = 0; t < kOsThreads; ++t) {
+    if (t & 32) continue;
+    OsLanes w[16];
+    for (int m = 0; m < 16; ++m) w[m] = OsLanes{{v[t][m], v[t + 32][m]}};
+    exchange(w);
+    for (int m = 0; m < 16; ++m) {
+      v[t][m] = w[m].lane[0];
+      v[t + 32][m] = w[m].lane[1];
+    }
+  }
+}
 inline void os_dif_host(float2* data, const float2* table) {
   const OsHostTables<kOsN> tb(table);
   const OsTwiddle tw = tb.tw();
   float2* lds = new float2[kOsLds];
-  float2 v[16];
-  for (int t = 0; t < kOsThreads; ++t) {
-    for (int r = 0; r < 16; ++r) v[r] = data[t + kOsThreads * r];
-    os_dif_first(lds, t, v);
-  }
-  for (int t = 0; t < kOsThreads; ++t) os_dif_mid1(lds, t, tw, v);
+  float2(*v)[16] = new float2[kOsThreads][16];
   float2 T[8];
   for (int t = 0; t < kOsThreads; ++t) {
-    os_tw_third(tw, t, T);
-    os_dif_mid2(lds, t, T, v);
+    for (int r = 0; r < 16; ++r) v[t][r] = data[t + kOsThreads * r];
+    os_dif_first(lds, t, v[t]);
   }
+  for (int t = 0; t < kOsThreads; ++t) os_dif_mid1(lds, t, tw, v[t]);
   for (int t = 0; t < kOsThreads; ++t) {
-    os_tw_last1<kOsN>(tw, t, T);
-    os_dif_last(lds, t, T, v);
-    for (int m = 0; m < 16; ++m) data[16 * t + m] = v[m];
+    const int t2 = os_mid_thread(t);
+    os_tw_third(tw, t2, T);
+    os_dif_mid2(lds, t2, T, v[t]);
   }
+  os_host_pairs(v, [](OsLanes* w) { pairs_gather(w, OsHostSwap()); });
+  for (int t = 0; t < kOsThreads; ++t) {
+    const int t2 = os_mid_thread(t);
+    os_tw_last1<kOsN>(tw, t2, T);
+    os_dif_pairs(T, v[t]);
+    for (int m = 0; m < 16; ++m) data[16 * t2 + m] = v[t][m];
+  }
+  delete[] v;
   delete[] lds;
 }
 inline void os_dit_host(float2* data, const float2* table) {
   const OsHostTables<kOsN> tb(table);
   const OsTwiddle tw = tb.tw();
   float2* lds = new float2[kOsLds];
-  float2 v[16];
-  for (int t = 0; t < kOsThreads; ++t) {
-    for (int m = 0; m < 16; ++m) v[m] = data[16 * t + m];
-    os_dit_first(lds, t, v);
-  }
-  for (int t = 0; t < kOsThreads; ++t) os_dit_mid1(lds, t, tw, v);
-  for (int t = 0; t < kOsThreads; ++t) os_dit_mid2(lds, t, tw, v);
+  float2(*v)[16] = new float2[kOsThreads][16];
   float2 T[8];
   for (int t = 0; t < kOsThreads; ++t) {
-    os_tw_last2<kOsN>(tw, t, T);
-    os_dit_last(lds, t, T, v);
-    for (int k = 0; k < 16; ++k) data[t + kOsThreads * k] = v[k];
+    for (int m = 0; m < 16; ++m) v[t][m] = data[16 * os_mid_thread(t) + m];
+    os_dit_pairs(v[t]);
   }
+  os_host_pairs(v, [](OsLanes* w) { pairs_scatter(w, OsHostSwap()); });
+  for (int t = 0; t < kOsThreads; ++t) {
+    os_dit_mid1(os_mid_thread(t), tw, v[t]);
+    os_dit_write(lds, os_mid_thread(t), v[t]);
+  }
+  for (int t = 0; t < kOsThreads; ++t) os_dit_mid2(lds, t, tw, v[t]);
+  for (int t = 0; t < kOsThreads; ++t) {
+    os_tw_last2<kOsN>(tw, t, T);
+    os_dit_last(lds, t, T, v[t]);
+    for (int k = 0; k < 16; ++k) data[t + kOsThreads * k] = v[t][k];
+  }
+  delete[] v;
   delete[] lds;
 }
 
@@ -511,46 +574,19 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The thread of stages (16, 2) and (2, 1) that thread t is on the device: lanes r
-// and r + 32 of a wave are a pair 2 q, 2 q + 1.
-__device__ __forceinline__ int os_mid_thread(int t) {
-  return (t & ~63) | ((t & 31) << 1) | ((t >> 5) & 1);
-}
-// Between those stages the values change hands within the pairs, position 32 q +
-// j + 2 k of thread 2 q + j as v[k] against 32 q + 16 j + m as v[m]: the second
-// half of the lower lane's values against the first half of the upper's, which
-// v_permlane32_swap does for two registers at once, in the place of an LDS write
-// and read (a third of the transforms' LDS cycles).
-__device__ __forceinline__ void pair_swap(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
-                                                  false);
-  a = __uint_as_float(r[0]);
-  b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ void pairs_gather(float2* v) {
-  float2 w[16];
-#pragma unroll
-  for (int h = 0; h < 8; ++h) {
-    w[2 * h] = v[h];
-    w[2 * h + 1] = v[h + 8];
-    pair_swap(w[2 * h].x, w[2 * h + 1].x);
-    pair_swap(w[2 * h].y, w[2 * h + 1].y);
+// v_permlane32_swap of the two components.
+struct LaneSwap {
+  static __device__ __forceinline__ void one(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                    false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
   }
-#pragma unroll
-  for (int m = 0; m < 16; ++m) v[m] = w[m];
-}
-__device__ __forceinline__ void pairs_scatter(float2* v) {
-  float2 w[16];
-#pragma unroll
-  for (int h = 0; h < 8; ++h) {
-    w[h] = v[2 * h];
-    w[h + 8] = v[2 * h + 1];
-    pair_swap(w[h].x, w[h + 8].x);
-    pair_swap(w[h].y, w[h + 8].y);
+  __device__ __forceinline__ void operator()(float2& a, float2& b) const {
+    one(a.x, b.x);
+    one(a.y, b.y);
   }
-#pragma unroll
-  for (int m = 0; m < 16; ++m) v[m] = w[m];
-}
+};
 
 // Device, first transform by kOsThreads threads, t their index (whole waves from
 // a multiple of 64 on): v[m] holds value t + kOsThreads m of the block on entry
@@ -570,10 +606,9 @@ __device__ __forceinline__ void os_dif_regs(float2* lds, int t, const OsTwiddle&
   os_dif_mid1(lds, t, tw, v);
   os_tw_last1<kOsN>(tw, t2, U);
   wave_sync();
-  os_read16<2>(lds, 33 * (t2 >> 1) + (t2 & 1), v);
-  dft_tw<16>(v, T);
+  os_dif_mid2(lds, t2, T, v);
   ahead();
-  pairs_gather(v);
+  pairs_gather(v, LaneSwap());
   os_dif_pairs(U, v);
 }
 
@@ -585,11 +620,10 @@ __device__ __forceinline__ void os_dit_regs(float2* lds, int t, const OsTwiddle&
   const int t2 = os_mid_thread(t);
   float2 T[8];
   os_dit_pairs(v);
-  pairs_scatter(v);
-  os_load_tw<2>(tw.s + os_at_two(kOsN), t2 & 1, T);
-  dft_tw<16>(v, T);
+  pairs_scatter(v, LaneSwap());
+  os_dit_mid1(t2, tw, v);
   wave_sync();
-  os_write16<2>(lds, 33 * (t2 >> 1) + (t2 & 1), v);
+  os_dit_write(lds, t2, v);
   os_tw_last2<kOsN>(tw, t, T);
   wave_sync();
   os_dit_mid2(lds, t, tw, v);

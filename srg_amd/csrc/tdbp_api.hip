@@ -284,8 +284,10 @@ int automatic_variant(int precision, bool* named) {
     return *named ? v : otherwise;
   };
   if (precision == TDBP_PLAIN_FP64) {
-    // Variant 1 (4 x 16 wave tiles side by side): 8.35-8.38 ms on one IW burst
-    // against 8.37-9.30 for the others.
+    // Variant 1 (4 x 16 wave tiles side by side): 3.04 ms on one IW burst against
+    // 2.99 (variant 0), 3.00 (5), 3.06 (6), 3.08 (4), 3.24 (2), 3.43 (7) and 9.1
+    // (3): within 2 % but for the narrow tiles, so 1, the fastest of the pair by
+    // pair kernel, stays.
     return from_env("TDBP_PLAIN_VARIANT", 1);
   }
   return from_env("TDBP_VARIANT", 5);

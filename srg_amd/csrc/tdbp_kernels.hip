@@ -1005,7 +1005,7 @@ __device__ __forceinline__ void staged_stage(const BurstDev& b, const PolyPixel&
 // is a quadratic to 2e-11 m, so the index advances by differences and the
 // phase factor by a rotation (PlainBlock).  25 instructions per pair in a full
 // block, 33 over the launch with the blocks' and tiles' set-up, all in FP64
-// but the lerp, which is FP32 as in plain_pair.
+// but the lerp, which is FP32 as in plain_pair (in FP64 a burst took 5 % longer).
 //
 // What the form rests on is checked: per pixel the quartic at the window's
 // two ends (1e-10 m, the rounding of R itself in FP64 at 8.5e5 m) and the
@@ -1014,7 +1014,7 @@ __device__ __forceinline__ void staged_stage(const BurstDev& b, const PolyPixel&
 // position that does not fit the others) and the range gate with the bound on
 // e.  Waves or stages that miss a check take plain_pair pair by pair.
 //
-// One IW burst (1500 x 21000 samples, 4000 x 1500 pixels, 3.05e9 pairs): 3.15
+// One IW burst (1500 x 21000 samples, 4000 x 1500 pixels, 2.97e9 pairs): 3.15
 // ms against 7.0 ms pair by pair, the error either way that of the
 // FP32 lerp and the stored image (5.0e-8 at 64 pulses, 6.1e-8 at 720).  With z *= w, w *= v pulse after pulse instead of pairs about
 // the block's centre: 3.6 ms (37 instructions per pair); blocks of 64 pulses:
@@ -2218,7 +2218,7 @@ __device__ __forceinline__ void mfma_tile(const BurstDev& b, int tile, MShared& 
 
 // Occupancy target of the FP64 kernels: 3 waves per SIMD leave 168 VGPRs, which
 // hold a block's recurrences without spills; the loads run a pair ahead, and
-// the kernel keeps VALU busy 91 % of its cycles (one IW burst: 3.15 ms at 3,
+// the kernel keeps VALU busy 92 % of its cycles (one IW burst: 3.15 ms at 3,
 // 3.2 at 4 with spills outside the loops, 3.9 at 5).
 #define TDBP_PLAIN_OCC __attribute__((amdgpu_waves_per_eu(3)))
 

@@ -23,7 +23,7 @@
 // and a - u b = 2 a - (a + u b) a third, so a radix-16 stage is 32 butterflies of
 // six FMAs, 192 instructions, where the DFT and then (or first) fifteen twiddle
 // products, nine of them formed as products, took 272; the first stage of either
-// transform has none.  The kernels are bound by vector issue (93 % busy).
+// transform has none.  (k_rc_os: vector issue 79 % busy, 93 % with the products.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -39,8 +39,8 @@ constexpr int kOsN = 8192;          // transform length
 // stage; thread t holds values t + kOsThreads m (m < 16) of the block in
 // natural order, or positions 16 t + m in digit-reversed order.  Two ~70 KB
 // workgroups fill a CU's LDS: 4 waves per SIMD.
-// (1024 threads, radix 8: 0.45 ms per IW burst against 0.40 ms at 512 --
-// spills at 64 VGPRs, and every barrier waits for 16 waves.)
+// (1024 threads and radix 8, in an earlier form of the kernel, were slower by an
+// eighth: spills at 64 VGPRs, and every barrier waits for 16 waves.)
 constexpr int kOsThreads = kOsN / 16;
 
 TDBP_HD float2 c_add(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }

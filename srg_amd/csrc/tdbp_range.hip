@@ -201,10 +201,10 @@ __global__ void __launch_bounds__(kOsThreads) k_os_spectrum(float2* __restrict__
 // header samples) and, when lmax is given, the largest |component| of the
 // block's outputs into lmax[l] (FP32 bits; max as fmaxf takes it, so NaN is
 // passed over as the pack kernel does).
-// Two workgroups per CU (LDS 2 x 73 KB): 4 waves per SIMD.  Vector issue (1530
-// instructions a wave, 76 % busy) and LDS (about as busy) bound it together: an
-// IW burst's 1500 lines in 0.21 ms, as with 1950 vector instructions (93 % busy)
-// before the twiddles went into the butterflies.
+// Two workgroups per CU (LDS 2 x 71 KB): 4 waves per SIMD.  Vector issue is 79 %
+// busy (1535 instructions a wave) and LDS 51 % (105, no bank conflicts): an IW
+// burst's 1500 lines in 0.21 ms (0.22 with 1950 vector instructions, 93 % busy, before
+// the twiddles went into the butterflies).
 __global__ void __launch_bounds__(kOsThreads)
 __attribute__((amdgpu_waves_per_eu(4)))
 k_rc_os(const float2* __restrict__ raw, int nlines, int stride, int nsamps, int npts, int nvalid,
